@@ -4049,14 +4049,23 @@ static void launch_bwd(dim3 g, dim3 b, size_t lds, hipStream_t s, const float* A
 
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul);
 bool rep_disabled_by_env();
-int rep_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream);
-int rep_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga, float* gb,
-            int64_t batch, void* stream);
+int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
+            void* stream);
+int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
+            float* ga, float* gb, int64_t batch, void* stream);
 
 // The geometric product of real-matrix-type signatures goes through the matrix
-// representation unless CLF_GEOM_PATH=direct asks for the per-term kernels.
-static bool use_rep(int op, int n, uint32_t neg, uint32_t nul) {
+// representation unless CLF_GEOM_PATH=direct asks for the per-term kernels. At
+// n = 11, 12 a few rows stay on the small-batch per-term kernels, which spread
+// a row over more workgroups than the 32 x 32 kernels do (forward + backward,
+// us: n = 11, 1 row 5.4 + 8.4 against 5.5 + 9.0, 16 rows 5.4 + 9.1 against
+// 6.0 + 9.9, 64 rows 10.2 + 18.9 against 6.3 + 10.2; n = 12, 1 row 5.5 + 8.9
+// against 7.5 + 13.1, 16 rows 10.2 + 18.9 against 8.2 + 13.6; n = 10, 1 row
+// 4.9 + 7.6 against 4.2 + 6.2).
+static bool use_rep(int op, int n, uint32_t neg, uint32_t nul, int64_t batch) {
     if (rep_disabled_by_env()) return false;
+    bool lowneg;
+    if ((n == 11 || n == 12) && batch <= (n == 11 ? 16 : 4) && blocked_metric(op, n, neg, nul, lowneg)) return false;
     return rep_applicable(op, n, neg, nul);
 }
 
@@ -4069,7 +4078,7 @@ int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
     if (c == a || c == b) return set_error(CLF_ERR_ARG, "output must not alias an input");
     if ((((uintptr_t)a) | ((uintptr_t)b) | ((uintptr_t)c)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
-    if (use_rep(op, n, neg, nul)) return rep_fwd(n, neg, a, b, c, batch, stream);
+    if (use_rep(op, n, neg, nul, batch)) return rep_fwd(n, neg, nul, a, b, c, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     BlkParams P{};
     P.batch = batch;
@@ -4161,7 +4170,7 @@ int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
         return set_error(CLF_ERR_ARG, "gradient outputs must not alias inputs or each other");
     if ((((uintptr_t)a) | ((uintptr_t)b) | ((uintptr_t)gc) | ((uintptr_t)ga) | ((uintptr_t)gb)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
-    if (use_rep(op, n, neg, nul)) return rep_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
+    if (use_rep(op, n, neg, nul, batch)) return rep_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     BlkParams P{};
     P.batch = batch;

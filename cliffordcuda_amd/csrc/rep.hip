@@ -776,12 +776,20 @@ int split_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int
 int split_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
               float* gb, int64_t batch, void* stream);
 
+bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul);
+int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
+              void* stream);
+int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
+              float* ga, float* gb, int64_t batch, void* stream);
+
 // The matrix path serves the geometric product when the signature allows it
 // (real type, n = 4, 6, 8; every non-degenerate n = 7 signature; split type
-// n = 9, and n = 10 with e_9 null); returns false otherwise (the caller uses
-// the per-term kernels).
+// n = 9, and n = 10 with e_9 null; n = 10, 11, 12 with a real-type base of ten
+// generators); returns false otherwise (the caller uses the per-term kernels).
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul) {
-    if (n == 9 || n == 10) return split_applicable(op, n, neg, nul);
+    if (n == 9 || n == 10)
+        if (split_applicable(op, n, neg, nul)) return true;
+    if (n >= 10) return rep32_applicable(op, n, neg, nul);
     if (n == 7) return op == CLF_OP_GEOM && nul == 0u && rep7_applicable(neg);
     if (op != CLF_OP_GEOM || nul != 0u || n < 4 || n > 2 * kRepMaxLogM) return false;
     RepTable T;
@@ -810,7 +818,9 @@ static long long rep16_bwd_blocks(int64_t batch) {
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 
-int rep_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream) {
+int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
+            void* stream) {
+    if (n >= 10 && rep32_applicable(CLF_OP_GEOM, n, neg, nul)) return rep32_fwd(n, neg, nul, a, b, c, batch, stream);
     if (n == 9 || n == 10) return split_fwd(n, neg, a, b, c, batch, stream);
     if (n == 7) return rep7_fwd(neg, a, b, c, batch, stream);
     RepTable T;
@@ -846,8 +856,10 @@ int rep_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64
     return CLF_OK;
 }
 
-int rep_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga, float* gb,
-            int64_t batch, void* stream) {
+int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
+            float* ga, float* gb, int64_t batch, void* stream) {
+    if (n >= 10 && rep32_applicable(CLF_OP_GEOM, n, neg, nul))
+        return rep32_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
     if (n == 9 || n == 10) return split_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
     if (n == 7) return rep7_bwd(neg, a, b, gc, ldg, ga, gb, batch, stream);
     RepTable T;

@@ -1,0 +1,729 @@
+// Geometric product of the large algebras (n = 10, 11, 12) through 32 x 32 real
+// matrices on the matrix cores.
+//
+// Ten of the n generators ("base") form a signature with Cl = M_32(R)
+// (p - q = 0 or 2 mod 8); the other K = n - 10 generators ("ext", any square,
+// null too) extend it. With every blade written e_I e_S (I base, S ext) a row
+// is 2^K base rows x_S, and for (A_S e_S)(B_J e_J):
+//   C_R = sum_{S ^ J = R} sigma(S, J) A_S alpha^{|S|}(B_J),
+// alpha the grade involution of the base (e_S passes B_J's blades) and sigma
+// the ext signs. In the representation phi each term is one 32 x 32 x 32
+// product: 4^K products of 32768 multiply-adds a row instead of 4^n terms
+// (n = 10: 1/32 of them, n = 11: 1/32, n = 12: 1/32). Backward:
+//   gA_S = sum_J sigma(S, J) G_{S^J} alpha^{|S|}(B_J)^T,
+//   gB_J = sum_S sigma(S, J) alpha^{|S|}(A_S)^T alpha^{|S|}(G_{S^J}).
+// alpha is the conjugation by the base pseudoscalar, phi = +-P(ox, oz):
+//   alpha(B)[k][j] = (-1)^{popc(oz & (k ^ j))} B[k ^ ox][j ^ ox],
+// so an operand of alpha(B) is B's own read at another column with two signs.
+//
+// Layout. One wave takes one base row (n = 10: four rows per workgroup, n = 11
+// two, n = 12 one; the 2^K waves of a row share their blocks through LDS). Lane
+// (h, x) gathers the 16 blades of the labels (x, 16h + zl) (real Pauli products
+// P(x, z) as in rep.hip), runs the 32-point transform over z (16 points in
+// registers, the last stage across the lane halves by permlane swaps) and
+// writes P[r][p] = W[r][p] of the plain conversion or W'[r][p] = W[r][p ^ r] of
+// the transposed one. Operand k of MFMA lane i is then column i of row i ^ k:
+//   phi[i][k] = W'[i ^ k][i],  phi^T[i][k] = W[i ^ k][i],
+// one LDS address per lane, xor-ed with a step constant. Element (r, p) sits at
+//   word 32 rho(r) + (p ^ 4 (r & 7)),  rho(r) = r ^ ((r >> 3) & 1),
+// which is linear over xor and free of bank conflicts for the b128 row writes
+// (8 lanes, 8 groups), the b32 column reads (32 lanes, 32 banks), the b32 result
+// writes at [i ^ j][j] and the b128 row reads (16 lanes of a set, 16 groups).
+// Staged rows are chunk-swizzled (chunk group bit t flipped by the parity of
+// the chunk index under a host-chosen mask) so that the 32 gathers of a step
+// fall on 32 banks.
+//
+// Bound: 12 (forward) and 20 (backward) 2^n bytes a row over HBM against 4^K
+// 1024 matrix-core cycles a row forward and twice that backward: HBM at n = 10,
+// matrix issue beside it at n = 11, 12; a workgroup's own latency for a few
+// rows. Measured (us, forward + backward; per-term kernels before): n = 10,
+// 16384 rows 33 + 68 (6.1 and 4.9 TB/s; 352 + 679); n = 11, 4096 rows 26 + 47
+// (3.9 and 3.6 TB/s; 545 + 1180); n = 12, 1024 rows 22 + 40 (660 + 2580), 64
+// rows 8.5 + 14 (34 + 65).
+#include <map>
+#include <mutex>
+
+#include "rep_common.h"
+
+namespace clf {
+
+constexpr int kBig = 32;         // matrix side
+constexpr int kBigBase = 10;     // base generators
+constexpr int kBigMaxExt = 2;
+
+struct Rep32Table {
+    unsigned lane_pos[64];          // staged position (floats) of the blade of label (x, 16h), lane = 32h + x, ext blade 1
+    unsigned z_pos[16];             // xor for the low label bits zl
+    unsigned ext_pos[1 << kBigMaxExt];      // xor for ext blade S
+    unsigned sgn[1 << kBigMaxExt][64];      // bit zl: the coefficient enters with -1; bit 16 + zl: the transposed conversion's sign
+    unsigned chunk_mask[3];         // chunk group bit t is flipped by the parity of chunk & chunk_mask[t]
+    unsigned ox, oz;                // label of the base pseudoscalar
+    unsigned neg_pairs, zero_pairs; // ext signs: bit 4 S + J
+};
+
+// word of element (r, p), split into its xor-linear row part and p itself
+__host__ __device__ constexpr unsigned big_row(unsigned r) { return ((r ^ ((r >> 3) & 1u)) << 5) ^ ((r & 7u) << 2); }
+
+__device__ __forceinline__ float big_ld(const float* base, unsigned byte) {
+    return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) + byte);
+}
+
+__device__ __forceinline__ void big_st(float* base, unsigned byte, float v) {
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + byte) = v;
+}
+
+template <int K>
+__device__ __forceinline__ void big_sync() {
+    if constexpr (K == 0) wave_lds_sync();  // a row is one wave's own
+    else __syncthreads();
+}
+
+__device__ __forceinline__ unsigned big_chunk(unsigned q, const Rep32Table& T) {
+    unsigned s = 0;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) s |= (unsigned)(__popc(q & T.chunk_mask[t]) & 1) << t;
+    return q ^ s;
+}
+
+struct BigRow {
+    float4 v[4];
+};
+
+// the wave's 1024 floats of its row
+template <bool NT>
+__device__ __forceinline__ BigRow big_fetch(const float* __restrict__ src, int lane) {
+    BigRow r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float4* q = reinterpret_cast<const float4*>(src) + lane + 64 * j;
+        r.v[j] = NT ? load_stream(q) : *q;
+    }
+    return r;
+}
+
+__device__ __forceinline__ void big_stage(float* __restrict__ region, const BigRow& r, const unsigned (&cpos)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) reinterpret_cast<float4*>(region)[cpos[j]] = r.v[j];
+}
+
+template <bool NT>
+__device__ __forceinline__ void big_store(float* __restrict__ dst, const float* __restrict__ region,
+                                          const unsigned (&cpos)[4], int lane) {
+    float4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const float4*>(region)[cpos[j]];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float4* q = reinterpret_cast<float4*>(dst) + lane + 64 * j;
+        if (NT) store_stream(q, v[j]);
+        else *q = v[j];
+    }
+}
+
+// Keeps values derived from v (addresses, signs) from being held in registers
+// across the loop: they are recomputed where they are used.
+__device__ __forceinline__ unsigned big_fresh(unsigned v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// raw coefficients of the lane's 16 labels
+__device__ __forceinline__ void big_gather(const float* __restrict__ region, unsigned pos, const Rep32Table& T,
+                                           float (&t)[16]) {
+    pos = big_fresh(pos);
+#pragma unroll
+    for (int z = 0; z < 16; ++z) t[z] = region[pos ^ T.z_pos[z]];
+}
+
+// t with the conversion's signs (bits SHIFT .. SHIFT + 15 of m), transformed over z, written as the rows of P
+template <int SHIFT>
+__device__ __forceinline__ void big_convert(const float (&raw)[16], unsigned m, float* __restrict__ P, unsigned x,
+                                            unsigned h) {
+    float t[16];
+    m = big_fresh(m);
+#pragma unroll
+    for (int z = 0; z < 16; ++z)
+        t[z] = __uint_as_float(__float_as_uint(raw[z]) ^ ((m << (31 - SHIFT - z)) & 0x80000000u));
+    wht_inplace<16>(t);
+    // last stage: after the swaps t[j] and t[j + 8] hold z bit 4 = 0 and 1 of
+    // column 8h + j, on both halves
+    float w[2][8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        permlane_swap32(t[j], t[j + 8]);
+        w[0][j] = t[j] + t[j + 8];
+        w[1][j] = t[j] - t[j + 8];
+    }
+    float4* row = reinterpret_cast<float4*>(P + ((x ^ ((x >> 3) & 1u)) << 5));
+#pragma unroll
+    for (int c4 = 0; c4 < 2; ++c4)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            row[(4u * c4 + 2u * h + u) ^ (x & 7u)] =
+                make_float4(w[c4][4 * u], w[c4][4 * u + 1], w[c4][4 * u + 2], w[c4][4 * u + 3]);
+}
+
+// acc(i, j) = C[i][j] to P[i ^ j][j] (the plain conversion of C), the inverse
+// transform, and the lane's 16 signed coefficients
+__device__ __forceinline__ void big_unconvert(const floatx16& acc, float* __restrict__ P, unsigned m, unsigned lane,
+                                              float (&t)[16]) {
+    const unsigned x = lane & 31u, h = lane >> 5;
+    m = big_fresh(m);
+    const unsigned base = (big_row(x) ^ x ^ (h ? big_row(4u) : 0u)) << 2;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) big_st(P, base ^ (big_row(8u * (q >> 2) + (q & 3u)) << 2), acc[q]);
+    wave_lds_sync();
+    float w[2][8];
+    const float4* row = reinterpret_cast<const float4*>(P + ((x ^ ((x >> 3) & 1u)) << 5));
+#pragma unroll
+    for (int c4 = 0; c4 < 2; ++c4)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const float4 v = row[(4u * c4 + 2u * h + u) ^ (x & 7u)];
+            w[c4][4 * u] = v.x;
+            w[c4][4 * u + 1] = v.y;
+            w[c4][4 * u + 2] = v.z;
+            w[c4][4 * u + 3] = v.w;
+        }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        t[j] = w[0][j] + w[1][j];
+        t[j + 8] = w[0][j] - w[1][j];
+        permlane_swap32(t[j], t[j + 8]);
+    }
+    wht_inplace<16>(t);
+#pragma unroll
+    for (int z = 0; z < 16; ++z)
+        t[z] = __uint_as_float(__float_as_uint(t[z] * 0.03125f) ^ ((m << (31 - z)) & 0x80000000u));
+}
+
+__device__ __forceinline__ void big_scatter(float* __restrict__ region, unsigned pos, const Rep32Table& T,
+                                            const float (&t)[16]) {
+    pos = big_fresh(pos);
+#pragma unroll
+    for (int z = 0; z < 16; ++z) region[pos ^ T.z_pos[z]] = t[z];
+}
+
+// acc += A B, A[i][k] at byte abase ^ (row constant of k) of P, B[k][j] at
+// bbase likewise with the sign bsign ^ (parity of k & kmask)
+template <bool SIGNED>
+__device__ __forceinline__ void big_mac(floatx16& acc, const float* __restrict__ PA, unsigned abase, unsigned asign,
+                                        const float* __restrict__ PB, unsigned bbase, unsigned bsign,
+                                        unsigned kmask) {
+    float a[16], b[16];
+    abase = big_fresh(abase);
+    bbase = big_fresh(bbase);
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+        a[s] = big_ld(PA, abase ^ (big_row(s) << 2));
+        b[s] = big_ld(PB, bbase ^ (big_row(s) << 2));
+        if (SIGNED) {
+            a[s] = __uint_as_float(__float_as_uint(a[s]) ^ asign);
+            b[s] = __uint_as_float(__float_as_uint(b[s]) ^ bsign ^ ((unsigned)(__popc(kmask & s) & 1) << 31));
+        }
+    }
+    // two short chains per product, then plain sums: half the rounding of one
+    // running sum over all products' steps
+    floatx16 c0 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c1 = c0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        c0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s], b[s], c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[s + 8], b[s + 8], c1, 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) acc[q] += c0[q] + c1[q];
+}
+
+// What a lane needs of its place: its matrix index i (= j), half h, and the
+// byte bases of its operand columns, plain and of alpha.
+struct BigLane {
+    unsigned plain, alpha;  // byte of [i ^ 16h][i], of [i ^ 16h][i ^ ox]
+    unsigned sign_i;        // (-1)^{popc(oz & i)} as a sign bit
+    unsigned sign_ik;       // (-1)^{popc(oz & (i ^ 16h))}
+};
+
+__device__ __forceinline__ BigLane big_lane(unsigned lane, const Rep32Table& T) {
+    const unsigned i = lane & 31u, h = lane >> 5;
+    BigLane L;
+    L.plain = (big_row(i) ^ (h ? big_row(16u) : 0u) ^ i) << 2;
+    L.alpha = L.plain ^ (T.ox << 2);
+    L.sign_i = (unsigned)(__popc(T.oz & i) & 1) << 31;
+    L.sign_ik = (unsigned)(__popc(T.oz & (i ^ (h << 4))) & 1) << 31;
+    return L;
+}
+
+template <int K, bool NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep32_fwd_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, long long batch, Rep32Table T) {
+    constexpr unsigned NS = 1u << K;  // base rows per row
+    constexpr int kRows = 4 >> K;     // rows per workgroup
+    __shared__ __attribute__((aligned(4096))) float lds[2][4 * 1024];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const unsigned x = lane & 31u, h = lane >> 5;
+    const unsigned S = wave & (NS - 1u), first = wave - S;
+    float* ra = &lds[0][first * 1024];  // the row's region: staged a, then its P blocks
+    float* rb = &lds[1][first * 1024];
+    const unsigned pos = T.lane_pos[lane] ^ T.ext_pos[S];
+    const unsigned m = T.sgn[S][lane];
+    const BigLane L = big_lane(lane, T);
+    unsigned cpos[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cpos[j] = big_chunk(S * 256u + 64u * j + lane, T);
+
+    for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
+        long long row = row0 + (wave >> K);
+        const bool live = row < batch;  // rows past the end recompute the last row and are not stored
+        row = live ? row : batch - 1;
+        const long long off = (row << (kBigBase + K)) + S * 1024;
+        const BigRow va = big_fetch<NT>(A + off, lane), vb = big_fetch<NT>(B + off, lane);
+        big_stage(ra, va, cpos);
+        big_stage(rb, vb, cpos);
+        big_sync<K>();
+        float ta[16], tb[16];
+        big_gather(ra, pos, T, ta);
+        big_gather(rb, pos, T, tb);
+        big_sync<K>();
+        big_convert<16>(ta, m, ra + S * 1024, x, h);
+        big_convert<0>(tb, m, rb + S * 1024, x, h);
+        big_sync<K>();
+        floatx16 acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (unsigned I = 0; I < NS; ++I) {
+            const unsigned J = I ^ S, pair = 4u * I + J;
+            const bool odd = (__popc(I) & 1) != 0;
+            if (K == 0) {
+                big_mac<false>(acc, ra, L.plain, 0u, rb, L.plain, 0u, 0u);
+            } else if (!((T.zero_pairs >> pair) & 1u)) {
+                const unsigned flip = ((T.neg_pairs >> pair) & 1u) << 31;
+                big_mac<true>(acc, ra + I * 1024, L.plain, 0u, rb + J * 1024, odd ? L.alpha : L.plain,
+                              odd ? (L.sign_ik ^ flip) : flip, odd ? T.oz : 0u);
+            }
+        }
+        big_sync<K>();
+        big_unconvert(acc, ra + S * 1024, m, lane, ta);
+        big_scatter(rb, pos, T, ta);
+        big_sync<K>();
+        if (live) big_store<NT>(C + off, rb, cpos, lane);
+        big_sync<K>();
+    }
+}
+
+template <int K, bool NT, bool WA, bool WB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rep32_bwd_kernel(
+    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, long long ldg,
+    float* __restrict__ GA, float* __restrict__ GB, long long batch, Rep32Table T) {
+    constexpr unsigned NS = 1u << K;
+    constexpr int kRows = 4 >> K;
+    __shared__ __attribute__((aligned(4096))) float lds[3][4 * 1024];
+    const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const unsigned x = lane & 31u, h = lane >> 5;
+    const unsigned S = wave & (NS - 1u), first = wave - S;
+    float* r0 = &lds[0][first * 1024];  // staged gc, then P blocks of gc
+    float* r1 = &lds[1][first * 1024];  // staged b, then P blocks of b, of a, then gb in blade order
+    float* r2 = &lds[2][first * 1024];  // staged a, then ga in blade order
+    const unsigned pos = T.lane_pos[lane] ^ T.ext_pos[S];
+    const unsigned m = T.sgn[S][lane];
+    const BigLane L = big_lane(lane, T);
+    unsigned cpos[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cpos[j] = big_chunk(S * 256u + 64u * j + lane, T);
+    const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+
+    for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
+        long long row = row0 + (wave >> K);
+        const bool live = row < batch;
+        row = live ? row : batch - 1;
+        const long long off = (row << (kBigBase + K)) + S * 1024;
+        const BigRow vg = big_fetch<NT>(GC + ((row & row_mask(ldg)) << (kBigBase + K)) + S * 1024, lane);
+        BigRow va, vb;
+        if (WA) vb = big_fetch<NT>(B + off, lane);
+        if (WB) va = big_fetch<NT>(A + off, lane);
+        big_stage(r0, vg, cpos);
+        if (WA) big_stage(r1, vb, cpos);
+        if (WB) big_stage(r2, va, cpos);
+        big_sync<K>();
+        float tg[16], ta[16], tb[16];
+        big_gather(r0, pos, T, tg);
+        if (WA) big_gather(r1, pos, T, tb);
+        if (WB) big_gather(r2, pos, T, ta);
+        big_sync<K>();
+        if (WA) {
+            // gA_S = sum_J sigma(S, J) G_{S^J} alpha^{|S|}(B_J)^T
+            big_convert<16>(tg, m, r0 + S * 1024, x, h);
+            big_convert<16>(tb, m, r1 + S * 1024, x, h);
+            big_sync<K>();
+            const bool odd = (__popc(S) & 1) != 0;
+            floatx16 acc = zero;
+#pragma unroll 1
+            for (unsigned J = 0; J < NS; ++J) {
+                const unsigned pair = 4u * S + J;
+                if (K == 0) {
+                    big_mac<false>(acc, r0, L.plain, 0u, r1, L.plain, 0u, 0u);
+                } else if (!((T.zero_pairs >> pair) & 1u)) {
+                    const unsigned flip = ((T.neg_pairs >> pair) & 1u) << 31;
+                    big_mac<true>(acc, r0 + (S ^ J) * 1024, L.plain, 0u, r1 + J * 1024, odd ? L.alpha : L.plain,
+                                  odd ? (L.sign_ik ^ flip) : flip, odd ? T.oz : 0u);
+                }
+            }
+            // r2 is free (a was gathered before the last two syncs); the block
+            // is the wave's own until the scatter
+            big_unconvert(acc, r2 + S * 1024, m, lane, tb);
+            big_sync<K>();
+            big_scatter(r2, pos, T, tb);
+        }
+        if (WB) {
+            // gB_S = sum_I sigma(I, S) alpha^{|I|}(A_I)^T alpha^{|I|}(G_{I^S}); the two
+            // alphas' signs of k cancel
+            big_convert<0>(tg, m, r0 + S * 1024, x, h);
+            big_convert<0>(ta, m, r1 + S * 1024, x, h);
+        }
+        big_sync<K>();
+        if (WA && live) big_store<NT>(GA + off, r2, cpos, lane);
+        if (WB) {
+            floatx16 acc = zero;
+#pragma unroll 1
+            for (unsigned I = 0; I < NS; ++I) {
+                const unsigned pair = 4u * I + S;
+                const bool odd = (__popc(I) & 1) != 0;
+                if (K == 0) {
+                    big_mac<false>(acc, r1, L.plain, 0u, r0, L.plain, 0u, 0u);
+                } else if (!((T.zero_pairs >> pair) & 1u)) {
+                    const unsigned flip = ((T.neg_pairs >> pair) & 1u) << 31;
+                    big_mac<true>(acc, r1 + I * 1024, odd ? L.alpha : L.plain, odd ? L.sign_i : 0u,
+                                  r0 + (I ^ S) * 1024, odd ? L.alpha : L.plain, odd ? (L.sign_i ^ flip) : flip, 0u);
+                }
+            }
+            big_sync<K>();
+            big_unconvert(acc, r0 + S * 1024, m, lane, ta);
+            big_scatter(r1, pos, T, ta);
+            big_sync<K>();
+            if (live) big_store<NT>(GB + off, r1, cpos, lane);
+        }
+        big_sync<K>();
+    }
+}
+
+// ---- host side --------------------------------------------------------------
+
+namespace {
+
+// Ten base generators of the metric whose signature is a full real matrix
+// algebra: the ext generators are the first choice, highest generators first,
+// for which no null generator is left and p - q = 0 or 2 (mod 8).
+bool big_split(int n, uint32_t neg, uint32_t nul, unsigned& ext) {
+    const int k = n - kBigBase;
+    if (k < 0 || k > kBigMaxExt) return false;
+    const unsigned full = (1u << n) - 1u;
+    auto real_type = [&](unsigned e) {
+        const unsigned base = full & ~e;
+        if (base & nul) return false;
+        const int q = host_popc(base & neg);
+        const int d = ((kBigBase - 2 * q) % 8 + 8) % 8;
+        return d == 0 || d == 2;
+    };
+    if (k == 0) {
+        ext = 0;
+        return real_type(0u);
+    }
+    for (int a = n - 1; a >= 0; --a) {
+        if (k == 1) {
+            if (real_type(1u << a)) {
+                ext = 1u << a;
+                return true;
+            }
+            continue;
+        }
+        for (int b = a - 1; b >= 0; --b)
+            if (real_type((1u << a) | (1u << b))) {
+                ext = (1u << a) | (1u << b);
+                return true;
+            }
+    }
+    return false;
+}
+
+// Anticommuting real Pauli products on five qubits with the wanted squares
+// (the first q of them -1), by depth-first search in a fixed order.
+bool big_generators(int q, unsigned* gx, unsigned* gz) {
+    unsigned cand[kBigBase] = {0};
+    int g = 0;
+    while (g >= 0 && g < kBigBase) {
+        bool found = false;
+        for (unsigned c = cand[g] + 1; c < kBig * kBig; ++c) {
+            const unsigned cx = c / kBig, cz = c % kBig;
+            if ((host_popc(cx & cz) & 1) != (g < q ? 1 : 0)) continue;
+            bool ok = true;
+            for (int p = 0; p < g && ok; ++p) ok = ((host_popc(cz & gx[p]) + host_popc(gz[p] & cx)) & 1) == 1;
+            if (!ok) continue;
+            cand[g] = c;
+            gx[g] = cx;
+            gz[g] = cz;
+            found = true;
+            break;
+        }
+        if (found) {
+            ++g;
+            if (g < kBigBase) cand[g] = 0;
+        } else {
+            --g;
+        }
+    }
+    return g == kBigBase;
+}
+
+// Adds v to a basis kept in echelon form; false if it is in the span already.
+bool big_independent(unsigned (&basis)[5], int& rank, unsigned v) {
+    for (int i = 0; i < rank; ++i)
+        if ((v ^ basis[i]) < v) v ^= basis[i];
+    if (!v) return false;
+    basis[rank++] = v;
+    for (int i = rank - 1; i > 0 && basis[i] > basis[i - 1]; --i) std::swap(basis[i], basis[i - 1]);
+    return true;
+}
+
+bool big_table_build(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
+    unsigned ext = 0;
+    if (!big_split(n, neg, nul, ext)) return false;
+    const int k = n - kBigBase;
+    const unsigned full = (1u << n) - 1u, base = full & ~ext;
+    unsigned px[kBigBase], pz[kBigBase];
+    if (!big_generators(host_popc(base & neg), px, pz)) return false;
+
+    // The search's generators may be dealt to the metric's generators of the
+    // same square in any order: take the first deal (of a fixed sequence of
+    // shuffles) for which the blades of one label column fall on 32 banks.
+    // For fixed z the position's five low bits, as functions of x, are those of
+    // the blade: bits 0, 1 as they are, bits 2..4 plus any higher bits through
+    // the chunk masks.
+    unsigned gx[16] = {0}, gz[16] = {0}, blade_of[kBig * kBig] = {0};
+    unsigned long long seed = 1;
+    int best = -1;
+    unsigned bgx[16] = {0}, bgz[16] = {0}, bmask[3] = {0, 0, 0};
+    for (int attempt = 0; attempt < 64 && best < 5; ++attempt) {
+        int slot[kBigBase];
+        int np = 0, nn = 0;
+        const int q = host_popc(base & neg);
+        int perm[kBigBase];
+        for (int i = 0; i < kBigBase; ++i) perm[i] = i;
+        auto shuffle = [&](int lo, int hi) {
+            for (int i = hi - 1; i > lo; --i) {
+                seed = seed * 6364136223846793005ULL + 1442695040888963407ULL;
+                std::swap(perm[i], perm[lo + (int)((seed >> 33) % (unsigned)(i - lo + 1))]);
+            }
+        };
+        if (attempt) {
+            shuffle(0, q);
+            shuffle(q, kBigBase);
+        }
+        int idx = 0;
+        for (int g = 0; g < n; ++g) {
+            if (!((base >> g) & 1u)) continue;
+            slot[idx] = ((neg >> g) & 1u) ? perm[nn++] : perm[q + np++];
+            gx[g] = px[slot[idx]];
+            gz[g] = pz[slot[idx]];
+            ++idx;
+        }
+        // blade of every label; column z = 0 gives x -> blade
+        for (unsigned c = 0; c < (1u << kBigBase); ++c) {
+            unsigned I = 0, x = 0, z = 0, r = c;
+            for (int g = 0; g < n; ++g)
+                if ((base >> g) & 1u) {
+                    if (r & 1u) {
+                        I |= 1u << g;
+                        x ^= gx[g];
+                        z ^= gz[g];
+                    }
+                    r >>= 1;
+                }
+            blade_of[z * kBig + x] = I;
+        }
+        // a functional on the column: the 5-bit vector of its values at x = 1, 2, 4, 8, 16
+        auto functional = [&](unsigned mask) {
+            unsigned f = 0;
+            for (int b = 0; b < 5; ++b) f |= (unsigned)(host_popc(blade_of[1u << b] & mask) & 1) << b;
+            return f;
+        };
+        unsigned basis[5], mask[3] = {0, 0, 0};
+        int rank = 0;
+        big_independent(basis, rank, functional(1u));
+        big_independent(basis, rank, functional(2u));
+        for (int t = 0; t < 3; ++t)
+            for (unsigned hm = 0; hm < (1u << (n - 5)); ++hm)
+                if (big_independent(basis, rank, functional((4u << t) | (hm << 5)))) {
+                    mask[t] = hm << 3;  // chunk bits
+                    break;
+                }
+        if (rank > best) {
+            best = rank;
+            for (int g = 0; g < n; ++g) {
+                bgx[g] = gx[g];
+                bgz[g] = gz[g];
+            }
+            for (int t = 0; t < 3; ++t) bmask[t] = mask[t];
+        }
+    }
+    for (int t = 0; t < 3; ++t) T.chunk_mask[t] = bmask[t];
+
+    auto position = [&](unsigned I) {
+        unsigned q = I >> 2;
+        for (int t = 0; t < 3; ++t) q ^= (unsigned)(host_popc((I >> 2) & bmask[t]) & 1) << t;
+        return (q << 2) | (I & 3u);
+    };
+    auto deposit = [&](unsigned s) {  // ext blade s (its generators in ascending order) as index bits
+        unsigned I = 0;
+        for (int g = 0; g < n; ++g)
+            if ((ext >> g) & 1u) {
+                if (s & 1u) I |= 1u << g;
+                s >>= 1;
+            }
+        return I;
+    };
+    // label and sign of every base blade
+    unsigned sign_of[kBig * kBig];
+    for (unsigned c = 0; c < (1u << kBigBase); ++c) {
+        unsigned I = 0, x = 0, z = 0, r = c;
+        bool negsign = false;
+        for (int g = 0; g < n; ++g)
+            if ((base >> g) & 1u) {
+                if (r & 1u) {
+                    I |= 1u << g;
+                    if (host_popc(z & bgx[g]) & 1) negsign = !negsign;
+                    x ^= bgx[g];
+                    z ^= bgz[g];
+                }
+                r >>= 1;
+            }
+        blade_of[x * kBig + z] = I;
+        sign_of[x * kBig + z] = negsign;
+        if (c == (1u << kBigBase) - 1u) {
+            T.ox = x;
+            T.oz = z;
+        }
+    }
+    for (unsigned z = 0; z < 16; ++z) T.z_pos[z] = position(blade_of[z]);
+    for (unsigned s = 0; s < (1u << k); ++s) T.ext_pos[s] = position(deposit(s));
+    for (unsigned l = 0; l < 64; ++l) {
+        const unsigned x = l & 31u, h = l >> 5;
+        T.lane_pos[l] = position(blade_of[x * kBig + 16 * h]);
+        for (unsigned s = 0; s < (1u << k); ++s) {
+            const unsigned E = deposit(s);
+            unsigned m = 0;
+            for (unsigned zl = 0; zl < 16; ++zl) {
+                const unsigned z = 16 * h + zl, I = blade_of[x * kBig + z];
+                // e_I e_E = (-1)^{pairs (i in I, e in E), i > e} e_{I | E}
+                const unsigned neg1 = (sign_of[x * kBig + z] + (unsigned)reorder_parity(I, E)) & 1u;
+                m |= neg1 << zl;
+                m |= ((neg1 + (unsigned)host_popc(x & z)) & 1u) << (16 + zl);
+                if (position(I) != (T.lane_pos[l] ^ T.z_pos[zl])) return false;  // the labels are linear
+            }
+            T.sgn[s][l] = m;
+        }
+    }
+    T.neg_pairs = T.zero_pairs = 0;
+    for (unsigned s = 0; s < (1u << k); ++s)
+        for (unsigned j = 0; j < (1u << k); ++j) {
+            const unsigned S = deposit(s), J = deposit(j);
+            if (S & J & nul) T.zero_pairs |= 1u << (4 * s + j);
+            else if ((reorder_parity(S, J) + host_popc(S & J & neg)) & 1) T.neg_pairs |= 1u << (4 * s + j);
+        }
+    return true;
+}
+
+// Tables of the signatures in use, built once each; past the bound a table is
+// built per call.
+constexpr size_t kBigTables = 512;
+
+bool big_table(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
+    static std::mutex mu;
+    static std::map<unsigned long long, Rep32Table> cache;
+    const unsigned long long key = ((unsigned long long)n << 48) | ((unsigned long long)nul << 24) | neg;
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        const auto it = cache.find(key);
+        if (it != cache.end()) {
+            T = it->second;
+            return true;
+        }
+    }
+    T = Rep32Table{};
+    if (!big_table_build(n, neg, nul, T)) return false;
+    std::lock_guard<std::mutex> lock(mu);
+    if (cache.size() < kBigTables) cache.emplace(key, T);
+    return true;
+}
+
+// One workgroup per 4 / 2^K rows; the cap only bounds the grid dimension (the
+// kernels walk any batch).
+unsigned big_grid(int k, int64_t batch) {
+    const long long rows = 4 >> k;
+    const long long g = (batch + rows - 1) / rows;
+    return (unsigned)(g < (1LL << 22) ? g : (1LL << 22));
+}
+
+}  // namespace
+
+bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul) {
+    unsigned ext;
+    return op == CLF_OP_GEOM && big_split(n, neg, nul, ext);
+}
+
+int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
+              void* stream) {
+    Rep32Table T;
+    if (!big_table(n, neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid(big_grid(n - kBigBase, batch)), block(256);
+    const bool nt = stream_nt(3.0 * 4.0 * (double)(1LL << n) * (double)batch);
+#define CLF_BIG_FWD(K)                                                                                              \
+    do {                                                                                                            \
+        if (nt) hipLaunchKernelGGL((rep32_fwd_kernel<K, true>), grid, block, 0, s, a, b, c, (long long)batch, T);    \
+        else hipLaunchKernelGGL((rep32_fwd_kernel<K, false>), grid, block, 0, s, a, b, c, (long long)batch, T);      \
+    } while (0)
+    switch (n - kBigBase) {
+        case 0: CLF_BIG_FWD(0); break;
+        case 1: CLF_BIG_FWD(1); break;
+        default: CLF_BIG_FWD(2); break;
+    }
+#undef CLF_BIG_FWD
+    CLF_HIP_CHECK(hipGetLastError());
+    return CLF_OK;
+}
+
+template <int K, bool NT>
+static void launch_rep32_bwd(dim3 grid, hipStream_t s, const float* a, const float* b, const float* gc, int64_t ldg,
+                             float* ga, float* gb, int64_t batch, const Rep32Table& T) {
+    const dim3 block(256);
+    if (ga && gb)
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, true, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
+                           (long long)batch, T);
+    else if (ga)
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, true, false>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
+                           (long long)batch, T);
+    else
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, false, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
+                           (long long)batch, T);
+}
+
+int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
+              float* ga, float* gb, int64_t batch, void* stream) {
+    Rep32Table T;
+    if (!big_table(n, neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
+    hipStream_t s = (hipStream_t)stream;
+    const dim3 grid(big_grid(n - kBigBase, batch));
+    const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 4.0 * (double)(1LL << n) * (double)batch);
+#define CLF_BIG_BWD(K)                                                                    \
+    do {                                                                                  \
+        if (nt) launch_rep32_bwd<K, true>(grid, s, a, b, gc, ldg, ga, gb, batch, T);      \
+        else launch_rep32_bwd<K, false>(grid, s, a, b, gc, ldg, ga, gb, batch, T);        \
+    } while (0)
+    switch (n - kBigBase) {
+        case 0: CLF_BIG_BWD(0); break;
+        case 1: CLF_BIG_BWD(1); break;
+        default: CLF_BIG_BWD(2); break;
+    }
+#undef CLF_BIG_BWD
+    CLF_HIP_CHECK(hipGetLastError());
+    return CLF_OK;
+}
+
+}  // namespace clf
