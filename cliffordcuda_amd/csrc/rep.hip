@@ -735,26 +735,7 @@ static bool rep_table_build(int n, uint32_t neg, RepTable& T) {
         T.e[x * m + z] = I | (negsign ? 0x80000000u : 0u) | (tsign ? 0x40000000u : 0u);
     }
     T.odd_xor = 0;
-    if (m == 16) {
-        // smallest multiple of 4 for which, for every z, the 16 gathers of an
-        // even row (blade offsets I) and of the next odd row (256 + (I ^ h))
-        // fall on 32 distinct LDS banks
-        for (unsigned h = 4; h < 256 && T.odd_xor == 0; h += 4) {
-            bool ok = true;
-            for (unsigned z = 0; z < 16 && ok; ++z) {
-                unsigned used = 0;
-                for (unsigned xx = 0; xx < 16 && ok; ++xx) {
-                    const unsigned I = T.e[xx * 16 + z] & 0xffffu;
-                    const unsigned b0 = I % 32, b1 = (256 + (I ^ h)) % 32;
-                    if ((used >> b0) & 1u) ok = false;
-                    used |= 1u << b0;
-                    if ((used >> b1) & 1u) ok = false;
-                    used |= 1u << b1;
-                }
-            }
-            if (ok) T.odd_xor = h;
-        }
-    }
+    if (m == 16) rep16_odd_xor(T);
     return true;
 }
 
@@ -782,14 +763,19 @@ int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b,
 int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
               float* ga, float* gb, int64_t batch, void* stream);
 
+bool twist_applicable(uint32_t neg, uint32_t nul);
+int twist_fwd(uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch, void* stream);
+int twist_bwd(uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
+              float* gb, int64_t batch, void* stream);
+
 // The matrix path serves the geometric product when the signature allows it
-// (real type, n = 4, 6, 8; every non-degenerate n = 7 signature; split type
-// n = 9, and n = 10 with e_9 null; n = 10, 11, 12 with a real-type base of ten
-// generators); returns false otherwise (the caller uses the per-term kernels).
+// (real type, n = 4, 6, 8; one generator from real type, n = 8; every
+// non-degenerate n = 7 signature; split type n = 9, and n = 10 with e_9 null;
+// n = 10, 11, 12 on 32 x 32 matrices); returns false otherwise (the caller uses
+// the per-term kernels).
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul) {
-    if (n == 9 || n == 10)
-        if (split_applicable(op, n, neg, nul)) return true;
-    if (n >= 10) return rep32_applicable(op, n, neg, nul);
+    if (n >= 9) return split_applicable(op, n, neg, nul) || rep32_applicable(op, n, neg, nul);
+    if (n == 8 && op == CLF_OP_GEOM && twist_applicable(neg, nul)) return true;
     if (n == 7) return op == CLF_OP_GEOM && nul == 0u && rep7_applicable(neg);
     if (op != CLF_OP_GEOM || nul != 0u || n < 4 || n > 2 * kRepMaxLogM) return false;
     RepTable T;
@@ -820,11 +806,11 @@ static long long rep16_bwd_blocks(int64_t batch) {
 
 int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
             void* stream) {
-    if (n >= 10 && rep32_applicable(CLF_OP_GEOM, n, neg, nul)) return rep32_fwd(n, neg, nul, a, b, c, batch, stream);
-    if (n == 9 || n == 10) return split_fwd(n, neg, a, b, c, batch, stream);
+    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_fwd(n, neg, a, b, c, batch, stream);
+    if (n >= 9) return rep32_fwd(n, neg, nul, a, b, c, batch, stream);
     if (n == 7) return rep7_fwd(neg, a, b, c, batch, stream);
     RepTable T;
-    if (!rep_table(n, neg, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no real matrix representation");
+    if (nul || !rep_table(n, neg, T)) return twist_fwd(neg, nul, a, b, c, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     const long long want = rep_blocks(n, batch);
 #define CLF_REP_GRID(K) dim3((unsigned)want)
@@ -858,12 +844,11 @@ int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, f
 
 int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
             float* ga, float* gb, int64_t batch, void* stream) {
-    if (n >= 10 && rep32_applicable(CLF_OP_GEOM, n, neg, nul))
-        return rep32_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
-    if (n == 9 || n == 10) return split_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
+    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
+    if (n >= 9) return rep32_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
     if (n == 7) return rep7_bwd(neg, a, b, gc, ldg, ga, gb, batch, stream);
     RepTable T;
-    if (!rep_table(n, neg, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no real matrix representation");
+    if (nul || !rep_table(n, neg, T)) return twist_bwd(neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     const long long want = rep_blocks(n, batch);
     switch (n) {

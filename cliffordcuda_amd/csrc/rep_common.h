@@ -311,4 +311,26 @@ inline bool rep_generators(int n, uint32_t neg, unsigned* gx, unsigned* gz) {
     return g == n;
 }
 
+// odd_xor of an m = 16 table: the smallest multiple of 4 for which, for every
+// entry z, the 16 gathers of an even row (blade offsets I) and of the next odd
+// row (256 + (I ^ h)) fall on 32 distinct LDS banks (0: none)
+inline void rep16_odd_xor(RepTable& T) {
+    T.odd_xor = 0;
+    for (unsigned h = 4; h < 256 && T.odd_xor == 0; h += 4) {
+        bool ok = true;
+        for (unsigned z = 0; z < 16 && ok; ++z) {
+            unsigned used = 0;
+            for (unsigned xx = 0; xx < 16 && ok; ++xx) {
+                const unsigned I = T.e[xx * 16 + z] & 0xffffu;
+                const unsigned b0 = I % 32, b1 = (256 + (I ^ h)) % 32;
+                if ((used >> b0) & 1u) ok = false;
+                used |= 1u << b0;
+                if ((used >> b1) & 1u) ok = false;
+                used |= 1u << b1;
+            }
+        }
+        if (ok) T.odd_xor = h;
+    }
+}
+
 }  // namespace clf
