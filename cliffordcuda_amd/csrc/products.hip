@@ -4054,19 +4054,16 @@ int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, f
 int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
             float* ga, float* gb, int64_t batch, void* stream);
 
-// The geometric product of real-matrix-type signatures goes through the matrix
-// representation unless CLF_GEOM_PATH=direct asks for the per-term kernels. At
-// n = 11, 12 a few rows stay on the small-batch per-term kernels, which spread
-// a row over more workgroups than the 32 x 32 kernels do (forward + backward,
-// us: n = 11, 1 row 5.4 + 8.4 against 5.5 + 9.0, 16 rows 5.4 + 9.1 against
-// 6.0 + 9.9, 64 rows 10.2 + 18.9 against 6.3 + 10.2; n = 12, 1 row 5.5 + 8.9
-// against 7.5 + 13.1, 16 rows 10.2 + 18.9 against 8.2 + 13.6; n = 10, 1 row
-// 4.9 + 7.6 against 4.2 + 6.2).
+int64_t rep32_few_rows(int n, uint32_t neg, uint32_t nul);
+
+// The geometric product goes through the matrix representation where the
+// signature has one, unless CLF_GEOM_PATH=direct asks for the per-term kernels.
+// A few rows of the larger 32 x 32 forms stay on the small-batch per-term
+// kernels, which spread a row over more workgroups.
 static bool use_rep(int op, int n, uint32_t neg, uint32_t nul, int64_t batch) {
-    if (rep_disabled_by_env()) return false;
+    if (rep_disabled_by_env() || !rep_applicable(op, n, neg, nul)) return false;
     bool lowneg;
-    if ((n == 11 || n == 12) && batch <= (n == 11 ? 16 : 4) && blocked_metric(op, n, neg, nul, lowneg)) return false;
-    return rep_applicable(op, n, neg, nul);
+    return n < 9 || batch > rep32_few_rows(n, neg, nul) || !blocked_metric(op, n, neg, nul, lowneg);
 }
 
 int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c,

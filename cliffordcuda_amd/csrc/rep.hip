@@ -771,7 +771,7 @@ int twist_bwd(uint32_t neg, uint32_t nul, const float* a, const float* b, const 
 // The matrix path serves the geometric product when the signature allows it
 // (real type, n = 4, 6, 8; one generator from real type, n = 8; every
 // non-degenerate n = 7 signature; split type n = 9, and n = 10 with e_9 null;
-// n = 10, 11, 12 on 32 x 32 matrices); returns false otherwise (the caller uses
+// n = 9 .. 12 on 32 x 32 matrices); returns false otherwise (the caller uses
 // the per-term kernels).
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul) {
     if (n >= 9) return split_applicable(op, n, neg, nul) || rep32_applicable(op, n, neg, nul);
@@ -780,6 +780,13 @@ bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul) {
     if (op != CLF_OP_GEOM || nul != 0u || n < 4 || n > 2 * kRepMaxLogM) return false;
     RepTable T;
     return rep_table(n, neg, T);
+}
+
+// Rows up to which the per-term kernels measured faster than rep32's (0 for
+// the signatures that the split representation serves).
+int64_t rep32_rows(int n, uint32_t neg, uint32_t nul);
+int64_t rep32_few_rows(int n, uint32_t neg, uint32_t nul) {
+    return split_applicable(CLF_OP_GEOM, n, neg, nul) ? 0 : rep32_rows(n, neg, nul);
 }
 
 // Workgroups: one per 4 * (64 / m) rows, at most 2048 (8 per CU); the waves

@@ -1,23 +1,26 @@
-// Geometric product of the large algebras (n = 10, 11, 12) through 32 x 32 real
+// Geometric product of the large algebras (n = 9 .. 12) through 32 x 32 real
 // matrices on the matrix cores.
 //
-// Ten of the n generators ("base") form a signature with Cl = M_32(R)
-// (p - q = 0 or 2 mod 8); the other K = n - 10 generators ("ext", any square,
-// null too) extend it. With every blade written e_I e_S (I base, S ext) a row
+// Ten generators ("base") form a signature with Cl = M_32(R) (p - q = 0 or 2
+// mod 8): 10 - D of the n generators and D dummies that no blade of a row
+// holds (their coefficients are staged as zeros), which lets the signatures in
+// that no ten (n = 9: no nine) generators are of real type. The other
+// K = n - 10 + D generators ("ext", any square, null too) extend it. With every blade written e_I e_S (I base, S ext) a row
 // is 2^K base rows x_S, and for (A_S e_S)(B_J e_J):
 //   C_R = sum_{S ^ J = R} sigma(S, J) A_S alpha^{|S|}(B_J),
 // alpha the grade involution of the base (e_S passes B_J's blades) and sigma
 // the ext signs. In the representation phi each term is one 32 x 32 x 32
 // product: 4^K products of 32768 multiply-adds a row instead of 4^n terms
-// (n = 10: 1/32 of them, n = 11: 1/32, n = 12: 1/32). Backward:
+// (without dummies 1/32 of them). Backward:
 //   gA_S = sum_J sigma(S, J) G_{S^J} alpha^{|S|}(B_J)^T,
 //   gB_J = sum_S sigma(S, J) alpha^{|S|}(A_S)^T alpha^{|S|}(G_{S^J}).
 // alpha is the conjugation by the base pseudoscalar, phi = +-P(ox, oz):
 //   alpha(B)[k][j] = (-1)^{popc(oz & (k ^ j))} B[k ^ ox][j ^ ox],
 // so an operand of alpha(B) is B's own read at another column with two signs.
 //
-// Layout. One wave takes one base row (n = 10: four rows per workgroup, n = 11
-// two, n = 12 one; the 2^K waves of a row share their blocks through LDS). Lane
+// Layout. One wave takes one base row (K = 0: four rows per workgroup, K = 1
+// two, K = 2 one; the 2^K waves of a row share their blocks through LDS; the
+// dummies are the top bits of a blade's place there). Lane
 // (h, x) gathers the 16 blades of the labels (x, 16h + zl) (real Pauli products
 // P(x, z) as in rep.hip), runs the 32-point transform over z (16 points in
 // registers, the last stage across the lane halves by permlane swaps) and
@@ -38,8 +41,10 @@
 // matrix issue beside it at n = 11, 12; a workgroup's own latency for a few
 // rows. Measured (us, forward + backward; per-term kernels before): n = 10,
 // 16384 rows 33 + 68 (6.1 and 4.9 TB/s; 352 + 679); n = 11, 4096 rows 26 + 47
-// (3.9 and 3.6 TB/s; 545 + 1180); n = 12, 1024 rows 22 + 40 (660 + 2580), 64
-// rows 8.5 + 14 (34 + 65).
+// (3.9 and 3.6 TB/s; 545 + 1180); n = 12, 1024 rows 22 + 41 (660 + 2580), 64
+// rows 8.5 + 14 (34 + 65). With dummies, 8000 rows: n = 9 17 + 30 (59 + 111),
+// Cl(8,0,1) 38 + 70 (53 + 100), Cl(8,2) 41 + 78 (183 + 350), Cl(8,3) 118 + 231
+// (955 + 2073).
 #include <map>
 #include <mutex>
 
@@ -89,12 +94,26 @@ struct BigRow {
     float4 v[4];
 };
 
-// the wave's 1024 floats of its row
-template <bool NT>
+// places (chunks) in the row's region of the wave's four chunks per lane: the
+// first 4 >> D hold its part of the row, the others the dummies' zeros
+template <int K, int D>
+__device__ __forceinline__ void big_places(unsigned S, unsigned lane, const Rep32Table& T, unsigned (&cpos)[4]) {
+    constexpr unsigned RC = 4u >> D;
+#pragma unroll
+    for (unsigned j = 0; j < 4; ++j)
+        cpos[j] = big_chunk(((j / RC) << (8 + K - D)) | (S * (256u >> D) + 64u * (j % RC) + lane), T);
+}
+
+// the wave's 1024 >> D floats of its row
+template <int D, bool NT>
 __device__ __forceinline__ BigRow big_fetch(const float* __restrict__ src, int lane) {
     BigRow r;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+        if (j >= (4 >> D)) {
+            r.v[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            continue;
+        }
         const float4* q = reinterpret_cast<const float4*>(src) + lane + 64 * j;
         r.v[j] = NT ? load_stream(q) : *q;
     }
@@ -106,14 +125,14 @@ __device__ __forceinline__ void big_stage(float* __restrict__ region, const BigR
     for (int j = 0; j < 4; ++j) reinterpret_cast<float4*>(region)[cpos[j]] = r.v[j];
 }
 
-template <bool NT>
+template <int D, bool NT>
 __device__ __forceinline__ void big_store(float* __restrict__ dst, const float* __restrict__ region,
                                           const unsigned (&cpos)[4], int lane) {
     float4 v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const float4*>(region)[cpos[j]];
+    for (int j = 0; j < (4 >> D); ++j) v[j] = reinterpret_cast<const float4*>(region)[cpos[j]];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < (4 >> D); ++j) {
         float4* q = reinterpret_cast<float4*>(dst) + lane + 64 * j;
         if (NT) store_stream(q, v[j]);
         else *q = v[j];
@@ -252,7 +271,7 @@ __device__ __forceinline__ BigLane big_lane(unsigned lane, const Rep32Table& T) 
     return L;
 }
 
-template <int K, bool NT>
+template <int K, int D, bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep32_fwd_kernel(
     const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, long long batch, Rep32Table T) {
     constexpr unsigned NS = 1u << K;  // base rows per row
@@ -267,15 +286,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
     const unsigned m = T.sgn[S][lane];
     const BigLane L = big_lane(lane, T);
     unsigned cpos[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) cpos[j] = big_chunk(S * 256u + 64u * j + lane, T);
+    big_places<K, D>(S, lane, T, cpos);
 
     for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
         long long row = row0 + (wave >> K);
         const bool live = row < batch;  // rows past the end recompute the last row and are not stored
         row = live ? row : batch - 1;
-        const long long off = (row << (kBigBase + K)) + S * 1024;
-        const BigRow va = big_fetch<NT>(A + off, lane), vb = big_fetch<NT>(B + off, lane);
+        const long long off = (row << (kBigBase + K - D)) + S * (1024u >> D);
+        const BigRow va = big_fetch<D, NT>(A + off, lane), vb = big_fetch<D, NT>(B + off, lane);
         big_stage(ra, va, cpos);
         big_stage(rb, vb, cpos);
         big_sync<K>();
@@ -303,12 +321,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         big_unconvert(acc, ra + S * 1024, m, lane, ta);
         big_scatter(rb, pos, T, ta);
         big_sync<K>();
-        if (live) big_store<NT>(C + off, rb, cpos, lane);
+        if (live) big_store<D, NT>(C + off, rb, cpos, lane);
         big_sync<K>();
     }
 }
 
-template <int K, bool NT, bool WA, bool WB>
+template <int K, int D, bool NT, bool WA, bool WB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rep32_bwd_kernel(
     const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, long long ldg,
     float* __restrict__ GA, float* __restrict__ GB, long long batch, Rep32Table T) {
@@ -325,19 +343,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
     const unsigned m = T.sgn[S][lane];
     const BigLane L = big_lane(lane, T);
     unsigned cpos[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) cpos[j] = big_chunk(S * 256u + 64u * j + lane, T);
+    big_places<K, D>(S, lane, T, cpos);
     const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
     for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
         long long row = row0 + (wave >> K);
         const bool live = row < batch;
         row = live ? row : batch - 1;
-        const long long off = (row << (kBigBase + K)) + S * 1024;
-        const BigRow vg = big_fetch<NT>(GC + ((row & row_mask(ldg)) << (kBigBase + K)) + S * 1024, lane);
+        const long long off = (row << (kBigBase + K - D)) + S * (1024u >> D);
+        const BigRow vg = big_fetch<D, NT>(GC + ((row & row_mask(ldg)) << (kBigBase + K - D)) + S * (1024u >> D), lane);
         BigRow va, vb;
-        if (WA) vb = big_fetch<NT>(B + off, lane);
-        if (WB) va = big_fetch<NT>(A + off, lane);
+        if (WA) vb = big_fetch<D, NT>(B + off, lane);
+        if (WB) va = big_fetch<D, NT>(A + off, lane);
         big_stage(r0, vg, cpos);
         if (WA) big_stage(r1, vb, cpos);
         if (WB) big_stage(r2, va, cpos);
@@ -378,7 +395,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
             big_convert<0>(ta, m, r1 + S * 1024, x, h);
         }
         big_sync<K>();
-        if (WA && live) big_store<NT>(GA + off, r2, cpos, lane);
+        if (WA && live) big_store<D, NT>(GA + off, r2, cpos, lane);
         if (WB) {
             floatx16 acc = zero;
 #pragma unroll 1
@@ -397,7 +414,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
             big_unconvert(acc, r0 + S * 1024, m, lane, ta);
             big_scatter(r1, pos, T, ta);
             big_sync<K>();
-            if (live) big_store<NT>(GB + off, r1, cpos, lane);
+            if (live) big_store<D, NT>(GB + off, r1, cpos, lane);
         }
         big_sync<K>();
     }
@@ -407,37 +424,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
 
 namespace {
 
-// Ten base generators of the metric whose signature is a full real matrix
-// algebra: the ext generators are the first choice, highest generators first,
-// for which no null generator is left and p - q = 0 or 2 (mod 8).
-bool big_split(int n, uint32_t neg, uint32_t nul, unsigned& ext) {
-    const int k = n - kBigBase;
-    if (k < 0 || k > kBigMaxExt) return false;
-    const unsigned full = (1u << n) - 1u;
-    auto real_type = [&](unsigned e) {
-        const unsigned base = full & ~e;
-        if (base & nul) return false;
-        const int q = host_popc(base & neg);
-        const int d = ((kBigBase - 2 * q) % 8 + 8) % 8;
-        return d == 0 || d == 2;
-    };
-    if (k == 0) {
-        ext = 0;
-        return real_type(0u);
-    }
-    for (int a = n - 1; a >= 0; --a) {
-        if (k == 1) {
-            if (real_type(1u << a)) {
-                ext = 1u << a;
+// How a signature is served: the ext generators, the number D of dummies and
+// how many of them are negative. The first choice (fewest dummies, so fewest
+// products; highest ext generators first) for which the base holds no null
+// generator and is of real type.
+struct BigSplit {
+    unsigned ext;
+    int k, d, dneg;
+};
+
+bool big_split(int n, uint32_t neg, uint32_t nul, BigSplit& c) {
+    for (int d = 0; d <= 2; ++d) {
+        const int k = n - kBigBase + d;
+        if (k < 0 || k > kBigMaxExt || (d == 2 && k != 1)) continue;
+        for (unsigned pick = 0; pick < (k == 0 ? 1u : k == 1 ? 16u : 256u); ++pick) {
+            const int a = n - 1 - (int)(pick & 15u), b = n - 1 - (int)(pick >> 4);
+            if ((k >= 1 && a < 0) || (k == 2 && (b < 0 || b <= a))) continue;
+            const unsigned ext = (k >= 1 ? 1u << a : 0u) | (k == 2 ? 1u << b : 0u);
+            const unsigned base = ((1u << n) - 1u) & ~ext;
+            if (base & nul) continue;
+            for (int dneg = 0; dneg <= d; ++dneg) {
+                const int t = ((kBigBase - 2 * (host_popc(base & neg) + dneg)) % 8 + 8) % 8;
+                if (t != 0 && t != 2) continue;
+                c = {ext, k, d, dneg};
                 return true;
             }
-            continue;
         }
-        for (int b = a - 1; b >= 0; --b)
-            if (real_type((1u << a) | (1u << b))) {
-                ext = (1u << a) | (1u << b);
-                return true;
-            }
     }
     return false;
 }
@@ -481,9 +493,8 @@ bool big_independent(unsigned (&basis)[5], int& rank, unsigned v) {
     return true;
 }
 
-bool big_table_build(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
-    unsigned ext = 0;
-    if (!big_split(n, neg, nul, ext)) return false;
+// n, neg: with the dummies as the top generators
+bool big_table_build(int n, uint32_t neg, uint32_t nul, unsigned ext, Rep32Table& T) {
     const int k = n - kBigBase;
     const unsigned full = (1u << n) - 1u, base = full & ~ext;
     unsigned px[kBigBase], pz[kBigBase];
@@ -633,7 +644,7 @@ bool big_table_build(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
 // built per call.
 constexpr size_t kBigTables = 512;
 
-bool big_table(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
+bool big_table(int n, uint32_t neg, uint32_t nul, const BigSplit& c, Rep32Table& T) {
     static std::mutex mu;
     static std::map<unsigned long long, Rep32Table> cache;
     const unsigned long long key = ((unsigned long long)n << 48) | ((unsigned long long)nul << 24) | neg;
@@ -646,7 +657,7 @@ bool big_table(int n, uint32_t neg, uint32_t nul, Rep32Table& T) {
         }
     }
     T = Rep32Table{};
-    if (!big_table_build(n, neg, nul, T)) return false;
+    if (!big_table_build(n + c.d, neg | (((1u << c.dneg) - 1u) << n), nul, c.ext, T)) return false;
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() < kBigTables) cache.emplace(key, T);
     return true;
@@ -663,65 +674,93 @@ unsigned big_grid(int k, int64_t batch) {
 }  // namespace
 
 bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul) {
-    unsigned ext;
-    return op == CLF_OP_GEOM && big_split(n, neg, nul, ext);
+    BigSplit c;
+    return op == CLF_OP_GEOM && big_split(n, neg, nul, c);
 }
 
-int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
-              void* stream) {
-    Rep32Table T;
-    if (!big_table(n, neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
-    hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(big_grid(n - kBigBase, batch)), block(256);
-    const bool nt = stream_nt(3.0 * 4.0 * (double)(1LL << n) * (double)batch);
-#define CLF_BIG_FWD(K)                                                                                              \
-    do {                                                                                                            \
-        if (nt) hipLaunchKernelGGL((rep32_fwd_kernel<K, true>), grid, block, 0, s, a, b, c, (long long)batch, T);    \
-        else hipLaunchKernelGGL((rep32_fwd_kernel<K, false>), grid, block, 0, s, a, b, c, (long long)batch, T);      \
-    } while (0)
-    switch (n - kBigBase) {
-        case 0: CLF_BIG_FWD(0); break;
-        case 1: CLF_BIG_FWD(1); break;
-        default: CLF_BIG_FWD(2); break;
+// Rows up to which the small-batch per-term kernels are faster: a row's 2^K
+// waves of the 32 x 32 kernels are one dependent chain of 2^K products each,
+// the per-term kernels spread it over more workgroups. Forward + backward, us,
+// per-term against 32 x 32: n = 9, K = 1: 300 rows 6.4 + 9.0 against 6.9 + 10.2,
+// 1500 rows 25 + 45 against 10.2 + 17.7; n = 10, K = 1: 64 rows 5.7 + 7.7
+// against 6.7 + 9.5, 300 rows 10.8 + 19.3 against 7.2 + 9.9; n = 11, K = 1: 16
+// rows 5.4 + 9.1 against 6.0 + 9.9, 64 rows 10.2 + 18.9 against 6.3 + 10.2;
+// n = 11, K = 2: 64 rows 8.9 + 15.7 against 8.1 + 13.1; n = 12: 1 row 5.5 + 8.9
+// against 7.5 + 13.1, 16 rows 10.2 + 18.9 against 8.2 + 13.6. K = 0 has no such
+// rows (n = 10, 1 row: 4.9 + 7.6 against 4.2 + 6.2).
+int64_t rep32_rows(int n, uint32_t neg, uint32_t nul) {
+    BigSplit c;
+    if (!big_split(n, neg, nul, c) || c.k == 0) return 0;
+    return n == 9 ? 512 : n == 10 ? 128 : n == 11 ? (c.k == 1 ? 16 : 32) : 4;
+}
+
+// M(K, D) for the (K, D) of c, one of big_split's
+#define CLF_BIG_SWITCH(M)        \
+    switch (4 * c.k + c.d) {     \
+        case 0: M(0, 0); break;  \
+        case 1: M(0, 1); break;  \
+        case 4: M(1, 0); break;  \
+        case 5: M(1, 1); break;  \
+        case 6: M(1, 2); break;  \
+        case 8: M(2, 0); break;  \
+        default: M(2, 1); break; \
     }
+
+template <int K, int D>
+static void launch_rep32_fwd(dim3 grid, hipStream_t s, bool nt, const float* a, const float* b, float* c,
+                             int64_t batch, const Rep32Table& T) {
+    const dim3 block(256);
+    if (nt) hipLaunchKernelGGL((rep32_fwd_kernel<K, D, true>), grid, block, 0, s, a, b, c, (long long)batch, T);
+    else hipLaunchKernelGGL((rep32_fwd_kernel<K, D, false>), grid, block, 0, s, a, b, c, (long long)batch, T);
+}
+
+int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* out, int64_t batch,
+              void* stream) {
+    BigSplit c;
+    Rep32Table T;
+    if (!big_split(n, neg, nul, c) || !big_table(n, neg, nul, c, T))
+        return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
+    const bool nt = stream_nt(3.0 * 4.0 * (double)(1LL << n) * (double)batch);
+#define CLF_BIG_FWD(K, D) \
+    launch_rep32_fwd<K, D>(dim3(big_grid(c.k, batch)), (hipStream_t)stream, nt, a, b, out, batch, T)
+    CLF_BIG_SWITCH(CLF_BIG_FWD)
 #undef CLF_BIG_FWD
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
 
-template <int K, bool NT>
+template <int K, int D, bool NT>
 static void launch_rep32_bwd(dim3 grid, hipStream_t s, const float* a, const float* b, const float* gc, int64_t ldg,
                              float* ga, float* gb, int64_t batch, const Rep32Table& T) {
     const dim3 block(256);
     if (ga && gb)
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, true, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
-                           (long long)batch, T);
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, true, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
+                           gb, (long long)batch, T);
     else if (ga)
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, true, false>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
-                           (long long)batch, T);
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, true, false>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
+                           gb, (long long)batch, T);
     else
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, NT, false, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga, gb,
-                           (long long)batch, T);
+        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, false, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
+                           gb, (long long)batch, T);
 }
 
 int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
               float* ga, float* gb, int64_t batch, void* stream) {
+    BigSplit c;
     Rep32Table T;
-    if (!big_table(n, neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
+    if (!big_split(n, neg, nul, c) || !big_table(n, neg, nul, c, T))
+        return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(big_grid(n - kBigBase, batch));
+    const dim3 grid(big_grid(c.k, batch));
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 4.0 * (double)(1LL << n) * (double)batch);
-#define CLF_BIG_BWD(K)                                                                    \
-    do {                                                                                  \
-        if (nt) launch_rep32_bwd<K, true>(grid, s, a, b, gc, ldg, ga, gb, batch, T);      \
-        else launch_rep32_bwd<K, false>(grid, s, a, b, gc, ldg, ga, gb, batch, T);        \
+#define CLF_BIG_BWD(K, D)                                                                \
+    do {                                                                                 \
+        if (nt) launch_rep32_bwd<K, D, true>(grid, s, a, b, gc, ldg, ga, gb, batch, T);  \
+        else launch_rep32_bwd<K, D, false>(grid, s, a, b, gc, ldg, ga, gb, batch, T);    \
     } while (0)
-    switch (n - kBigBase) {
-        case 0: CLF_BIG_BWD(0); break;
-        case 1: CLF_BIG_BWD(1); break;
-        default: CLF_BIG_BWD(2); break;
-    }
+    CLF_BIG_SWITCH(CLF_BIG_BWD)
 #undef CLF_BIG_BWD
+#undef CLF_BIG_SWITCH
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }

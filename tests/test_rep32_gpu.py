@@ -12,6 +12,8 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-5  # normwise, as for every product: 3 sqrt(2^n) sums of fp32 terms stay below 1e-6
 
 SIGNATURES = [
+    (1,) * 8 + (-1,), (1, -1, 1, -1, 1, 1, 1, 1, -1), (-1, 1) + (1,) * 6 + (-1,), (1,) * 8 + (0,), (0,) + (-1, 1) * 4,
+    (1,) * 8 + (-1,) * 2, (1, 0) + (1,) * 8, (-1,) * 10, (1,) * 8 + (-1,) * 3, (1, -1, 1) * 3 + (0, 0),  # with dummies
     (1,) * 10, (1,) * 9 + (-1,), (-1,) * 4 + (1,) * 6, (1, -1) * 5, (-1,) * 9 + (1,),  # n = 10, real type
     (1,) * 11, (1,) * 10 + (-1,), (1,) * 10 + (0,), (0,) + (1,) * 10, (-1, 1) * 4 + (1, 1, -1),
     (1,) * 5 + (0,) + (-1,) * 5,
@@ -41,7 +43,8 @@ def gpu(metric, a, b, gc):
     return c.detach(), ga, gb
 
 
-@pytest.mark.parametrize("metric", [(1,) * 10, (1,) * 10 + (-1,), (1,) * 12], ids=ids)
+@pytest.mark.parametrize("metric", [(1,) * 8 + (-1,), (-1,) * 2 + (1,) * 7, (1,) * 10, (1,) * 8 + (-1,) * 2,
+                                    (1,) * 10 + (-1,), (1,) * 8 + (-1,) * 3, (1,) * 12], ids=ids)
 @pytest.mark.parametrize("batch", [1, 3, 5])
 def test_against_oracle(metric, batch):
     a, b, gc = inputs(batch, len(metric), 3 + batch)
@@ -55,8 +58,9 @@ def test_against_oracle(metric, batch):
 
 @pytest.mark.parametrize("metric", SIGNATURES, ids=ids)
 def test_equals_per_term_kernels(metric, clf_env):
-    a, b, gc = inputs(11, len(metric), 7)
-    row = gc[:1].cuda().expand(11, -1)  # the gradient of a weighted sum: batch stride 0
+    rows = 515 if len(metric) == 9 else 131 if len(metric) == 10 else 33 + len(metric)  # past the few-rows rule
+    a, b, gc = inputs(rows, len(metric), 7)
+    row = gc[:1].cuda().expand(rows, -1)  # the gradient of a weighted sum: batch stride 0
     got = gpu(metric, a, b, gc.cuda()) + gpu(metric, a, b, row)
     x, y = a.cuda().requires_grad_(), b.cuda().requires_grad_()
     ga, = torch.autograd.grad(cc.geom_prod(x, b.cuda(), metric), x, gc.cuda())
