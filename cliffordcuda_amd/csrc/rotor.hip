@@ -39,10 +39,11 @@
 // and, through cs = Givens(expm(B)), the bivector gradient by reverse-mode
 // through the factorisation (fp64) followed by the Frechet step above.
 //
-// Apply layout: one row is spread over 2^(n-RB) lanes, each holding 2^RB
-// consecutive blades in registers. Planes inside the register bits are pure
-// FMAs; planes touching lane bits exchange partner values with lane shuffles.
-// The plane list is unrolled at compile time per n.
+// Apply layout, n <= 8: one row is spread over 2^(n-RB) lanes, each holding
+// 2^RB consecutive blades in registers. Planes inside the register bits are
+// pure FMAs; planes touching lane bits exchange partner values with lane
+// shuffles. The plane list is unrolled at compile time per n. n = 9 .. 12:
+// rotor_tile.hip.
 #include <utility>
 
 #include "rep_common.h"
@@ -69,9 +70,9 @@ __host__ __device__ constexpr int plane_q(int n, int k) {
     }
     return p + 1 + k;
 }
-// register bits per lane: rows of n <= 8 use 4 lanes (partner exchanges are
-// quad-local DPP permutes), n = 9 .. 12 use 8 .. 64 lanes of 64 blades each
-__host__ __device__ constexpr int rotor_rb(int n) { return n < 4 ? n : (n <= 8 ? n - 2 : 6); }
+// register bits per lane (n <= 8): a row's 4 lanes (one at n < 4), so partner
+// exchanges are quad-local DPP permutes
+__host__ __device__ constexpr int rotor_rb(int n) { return n < 4 ? n : n - 2; }
 // parity of the bits of r strictly between positions p and q (p < q)
 __host__ __device__ constexpr int between_par(unsigned r, int p, int q) {
     int c = 0;
@@ -91,22 +92,13 @@ __device__ __forceinline__ float dpp_mov(float v) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 
-// value of v in lane (lane ^ MASK) for MASK < 64: quad-local bits by DPP quad
-// permutes (full-rate VALU), bits 2..4 by one ds_swizzle in bit-mask mode, bit 5
-// (the other half of the wave) by ds_bpermute
+// value of v in lane (lane ^ MASK) of the quad
 template <unsigned MASK>
 __device__ __forceinline__ float lane_xor(float v) {
-    static_assert(MASK < 64, "lane exchange limited to one wave");
-    float r = v;
-    if constexpr ((MASK & 3u) == 1u) r = dpp_mov<0xB1>(r);       // quad_perm [1,0,3,2]
-    else if constexpr ((MASK & 3u) == 2u) r = dpp_mov<0x4E>(r);  // quad_perm [2,3,0,1]
-    else if constexpr ((MASK & 3u) == 3u) r = dpp_mov<0x1B>(r);  // quad_perm [3,2,1,0]
-    if constexpr ((MASK & 0x1Cu) != 0u) {
-        constexpr int pattern = (int)(((MASK & 0x1Cu) << 10) | 0x1Fu);  // and 0x1F, or 0, xor MASK
-        r = __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(r), pattern));
-    }
-    if constexpr ((MASK & 32u) != 0u) r = __shfl_xor(r, 32, 64);
-    return r;
+    static_assert(MASK >= 1 && MASK < 4, "lane exchange limited to a quad");
+    if constexpr (MASK == 1u) return dpp_mov<0xB1>(v);       // quad_perm [1,0,3,2]
+    else if constexpr (MASK == 2u) return dpp_mov<0x4E>(v);  // quad_perm [2,3,0,1]
+    else return dpp_mov<0x1B>(v);                            // quad_perm [3,2,1,0]
 }
 
 // One plane of the chain, in the form y_I = c x_I - s sig x_J,
@@ -217,9 +209,7 @@ __device__ __forceinline__ void store_row_part(const float (&v)[1 << RB], float*
 }
 
 // y = Lambda(Q) x (FWD) or Lambda(Q)^T x (!FWD), one row per 2^(N-RB) lanes
-// (RB: 2^RB floats of a row per lane; rotor_rb(N), or N - 6 for one wave per
-// row, where a row's planes run on 64 lanes with 2^(N-6) floats each instead
-// of on 2^(N-6) lanes with 64 floats; use_wave_rows picks by n and batch).
+// (n <= 8; the larger n run on rotor_tile.hip).
 // Persistent: the lanes of a row walk rows with a grid stride and load the
 // next row part while the current one is rotated. Rows past the end are never
 // stored; their prefetch re-reads the last row (a cache hit, no branch).
@@ -227,12 +217,11 @@ __device__ __forceinline__ void store_row_part(const float (&v)[1 << RB], float*
 // stay active together and every shuffle partner is active.
 // ldx: floats between the input's rows (2^N, or 0 for one row broadcast over
 // the batch: the transposed action on the gradient of a sum)
-template <int N, bool FWD, int RB = rotor_rb(N)>
+template <int N, bool FWD>
 __global__ __launch_bounds__(256) void rotor_apply_kernel(const float* __restrict__ cs,
                                                            const float* __restrict__ X, float* __restrict__ Y,
                                                            long long batch, long long ldx) {
-    static_assert(RB >= 1 && N - RB <= 6, "a row spans at most one wave");
-    constexpr int LB = N - RB;
+    constexpr int RB = rotor_rb(N), LB = N - RB;
     const unsigned L = threadIdx.x & ((1u << LB) - 1u);
     const long long rows_per_block = 256 >> LB;
     const long long stride = (long long)gridDim.x * rows_per_block;
@@ -344,15 +333,14 @@ __device__ __forceinline__ float wave_sum_f32(float v) {
 // Persistent: each workgroup walks rows with a grid stride, writes gx (if
 // requested) and, if gamma_ws != nullptr, its partial K (C(N,2) floats) to
 // gamma_ws[blockIdx.x * C(N,2)].
-template <int N, int RB = rotor_rb(N)>
+template <int N>
 __global__ __launch_bounds__(256) void rotor_apply_bwd_kernel(const float* __restrict__ cs,
                                                                const float* __restrict__ X,
                                                                const float* __restrict__ GY,
                                                                float* __restrict__ GX,
                                                                float* __restrict__ gamma_ws, long long batch,
                                                                long long ldg) {
-    static_assert(RB >= 1 && N - RB <= 6, "a row spans at most one wave");
-    constexpr int LB = N - RB;
+    constexpr int RB = rotor_rb(N), LB = N - RB;
     constexpr int LPR = 1 << LB;
     constexpr int C = n_planes(N);
     const unsigned L = threadIdx.x & (LPR - 1);
@@ -397,28 +385,18 @@ __global__ __launch_bounds__(256) void rotor_apply_bwd_kernel(const float* __res
         gamma_ws[(long long)blockIdx.x * C + k] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
 }
 
-// ---- the chain with rows staged in LDS (any n up to 12, run-time planes) ----
-// Used for the reference's backward on a caller's cs (every n) and for the
-// n = 12 forward and transposed apply up to 768 rows; the other chain work at
-// n = 11, 12 runs the register kernels with one wave per row (32 and 64
-// floats per lane), which measured faster there. A workgroup stages
-// kLdsBlades floats per array (whole rows; one row at n = 12) and walks the
-// planes with a barrier between planes; each thread owns kLdsBlades / 1024
-// blade pairs of every plane, found by inserting zero bits at p and q into
-// the pair number:
+// ---- the cs backward with rows staged in LDS (any n up to 12, run-time planes) ----
+// The reference's backward on a caller's cs: from (y, gy), gx and the cs
+// gradient (inputs rebuilt with the transposed pair map,
+// grad_c += g_I v_I + g_J v_J, grad_s += sig (g_I v_J - g_J v_I)). A workgroup
+// stages kLdsBlades floats per array (whole rows; one row at n = 12) and walks
+// the planes with a barrier between planes; each thread owns
+// kLdsBlades / 1024 blade pairs of every plane, found by inserting zero bits at
+// p and q into the pair number:
 //   base = deposit(t), I = base | 2^p (p set, q clear), J = base | 2^q.
-// Modes:
-//   LDS_FWD    y = chain(cs) x
-//   LDS_TR     gx = chain(cs)^T gy
-//   LDS_CS_BWD from (y, gy): gx and the cs gradient (the reference's rule:
-//              inputs rebuilt with the transposed pair map,
-//              grad_c += g_I v_I + g_J v_J, grad_s += sig (g_I v_J - g_J v_I))
-//   LDS_GAMMA  from (x, gy): gx = chain^T gy and the statistics
-//              K_pq = sum sig (x_J gx_I - x_I gx_J) of the composite backward
 // Per-plane sums go through a wave reduction into a per-wave LDS slot (no
 // atomics, fixed order), then one partial per workgroup.
 constexpr int kLdsBlades = 4096;
-enum LdsMode { LDS_FWD = 0, LDS_TR = 1, LDS_CS_BWD = 2, LDS_GAMMA = 3 };
 
 __device__ __forceinline__ unsigned deposit2(unsigned t, int p, int q) {
     const unsigned lo = t & ((1u << p) - 1u);
@@ -427,82 +405,33 @@ __device__ __forceinline__ unsigned deposit2(unsigned t, int p, int q) {
     return lo | (mid << (p + 1)) | (hi << (q + 1));
 }
 
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-    for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-template <int MODE>
-__global__ __launch_bounds__(256) void rotor_chain_lds_kernel(int n, const float* __restrict__ cs,
-                                                               const float* __restrict__ A,
-                                                               const float* __restrict__ B, float* __restrict__ OUT,
-                                                               float* __restrict__ parts, long long batch,
-                                                               long long lda, long long ldb) {
-    constexpr bool TWO = (MODE == LDS_CS_BWD || MODE == LDS_GAMMA);
+__global__ __launch_bounds__(256) void rotor_cs_bwd_kernel(int n, const float* __restrict__ cs,
+                                                           const float* __restrict__ Yin,
+                                                           const float* __restrict__ GY, float* __restrict__ GX,
+                                                           float* __restrict__ parts, long long batch,
+                                                           long long ldg) {
     constexpr int kMaxW = 2 * 66;  // 2 C(12, 2)
     __shared__ float va[kLdsBlades];
-    __shared__ float vb[TWO ? kLdsBlades : 1];
-    __shared__ float acc[TWO ? 4 : 1][TWO ? kMaxW : 1];
+    __shared__ float vb[kLdsBlades];
+    __shared__ float acc[4][kMaxW];
     const int D = 1 << n;
     const int C = n * (n - 1) / 2;
     const int rpb = kLdsBlades >> n > 0 ? kLdsBlades >> n : 1;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int pairs = (rpb * D) >> 2;  // per plane in the staged rows
-    if (TWO)
-        for (int e = tid; e < 4 * kMaxW; e += blockDim.x) (&acc[0][0])[e] = 0.f;
+    for (int e = tid; e < 4 * kMaxW; e += blockDim.x) (&acc[0][0])[e] = 0.f;
     for (long long row0 = (long long)blockIdx.x * rpb; row0 < batch; row0 += (long long)gridDim.x * rpb) {
         const long long rows = (batch - row0) < rpb ? (batch - row0) : rpb;
         const int nb = (int)(rows << n);
         __syncthreads();  // the previous group's last plane and stores are done
         for (int e = tid * 4; e < nb; e += blockDim.x * 4) {
-            // rows of A and B are lda / ldb floats apart (2^n, or 0: one row for all)
+            // rows of gy are ldg floats apart (2^n, or 0: one row for all)
             const long long r = row0 + (e >> n), c = e & (D - 1);
-            *reinterpret_cast<float4*>(&va[e]) = *reinterpret_cast<const float4*>(A + r * lda + c);
-            if (TWO) *reinterpret_cast<float4*>(&vb[e]) = *reinterpret_cast<const float4*>(B + r * ldb + c);
+            *reinterpret_cast<float4*>(&va[e]) = *reinterpret_cast<const float4*>(Yin + (r << n) + c);
+            *reinterpret_cast<float4*>(&vb[e]) = *reinterpret_cast<const float4*>(GY + r * ldg + c);
         }
-        if (MODE == LDS_GAMMA) {
-            // gx = chain^T gy on vb (planes last to first), then K from (va = x, vb = gx)
-            for (int k = C - 1; k >= -C; --k) {
-                __syncthreads();
-                const bool stats = k < 0;
-                const int kk = stats ? -1 - k : k;
-                int p = 0, rem = kk;
-                while (rem >= n - 1 - p) {
-                    rem -= n - 1 - p;
-                    ++p;
-                }
-                const int q = p + 1 + rem;
-                const float c = cs[2 * (C - 1 - kk)], sv = cs[2 * (C - 1 - kk) + 1];
-                const unsigned between = ((1u << q) - 1u) & ~((2u << p) - 1u);
-                float part = 0.f;
-                for (int t = tid; t < pairs; t += blockDim.x) {
-                    const int r = t >> (n - 2), tt = t & ((D >> 2) - 1);
-                    const unsigned base = deposit2((unsigned)tt, p, q);
-                    const int I = (r << n) | (int)(base | (1u << p)), J = (r << n) | (int)(base | (1u << q));
-                    const float sig = (__popc(base & between) & 1) ? -1.f : 1.f;
-                    if (r >= rows) continue;
-                    const float gI = vb[I], gJ = vb[J];
-                    if (!stats) {
-                        // transposed pair map: (gI, gJ) <- (c gI - s sig gJ, c gJ + s sig gI)
-                        vb[I] = __builtin_fmaf(c, gI, -sv * sig * gJ);
-                        vb[J] = __builtin_fmaf(c, gJ, sv * sig * gI);
-                    } else {
-                        part = __builtin_fmaf(sig, __builtin_fmaf(va[J], gI, -va[I] * gJ), part);
-                    }
-                }
-                if (stats) {
-                    part = wave_sum_dpp(part);
-                    if (lane == 0) acc[wave][kk] += part;
-                }
-            }
+        for (int k = C - 1; k >= 0; --k) {
             __syncthreads();
-            for (int e = tid * 4; e < nb; e += blockDim.x * 4)
-                if (OUT) *reinterpret_cast<float4*>(OUT + (row0 << n) + e) = *reinterpret_cast<const float4*>(&vb[e]);
-            continue;
-        }
-        for (int step = 0; step < C; ++step) {
-            __syncthreads();
-            const int k = (MODE == LDS_FWD) ? step : C - 1 - step;
             int p = 0, rem = k;
             while (rem >= n - 1 - p) {
                 rem -= n - 1 - p;
@@ -517,47 +446,34 @@ __global__ __launch_bounds__(256) void rotor_chain_lds_kernel(int n, const float
                 if (r >= rows) continue;
                 const unsigned base = deposit2((unsigned)tt, p, q);
                 const int I = (r << n) | (int)(base | (1u << p)), J = (r << n) | (int)(base | (1u << q));
-                const float ss = (__popc(base & between) & 1) ? -sv : sv;
-                const float xI = va[I], xJ = va[J];
-                if (MODE == LDS_FWD) {
-                    va[I] = __builtin_fmaf(c, xI, ss * xJ);
-                    va[J] = __builtin_fmaf(c, xJ, -ss * xI);
-                } else {
-                    // rebuilt input (LDS_CS_BWD) or transposed gradient (LDS_TR)
-                    const float pI = __builtin_fmaf(c, xI, -ss * xJ);
-                    const float pJ = __builtin_fmaf(c, xJ, ss * xI);
-                    va[I] = pI;
-                    va[J] = pJ;
-                    if (MODE == LDS_CS_BWD) {
-                        const float gI = vb[I], gJ = vb[J];
-                        const float sig = (__popc(base & between) & 1) ? -1.f : 1.f;
-                        dc = __builtin_fmaf(gI, pI, __builtin_fmaf(gJ, pJ, dc));
-                        dsum = __builtin_fmaf(sig, __builtin_fmaf(gI, pJ, -gJ * pI), dsum);
-                        vb[I] = __builtin_fmaf(c, gI, -ss * gJ);
-                        vb[J] = __builtin_fmaf(c, gJ, ss * gI);
-                    }
-                }
+                const float sig = (__popc(base & between) & 1) ? -1.f : 1.f;
+                const float ss = sig * sv;
+                const float xI = va[I], xJ = va[J], gI = vb[I], gJ = vb[J];
+                const float pI = __builtin_fmaf(c, xI, -ss * xJ);  // rebuilt input
+                const float pJ = __builtin_fmaf(c, xJ, ss * xI);
+                va[I] = pI;
+                va[J] = pJ;
+                dc = __builtin_fmaf(gI, pI, __builtin_fmaf(gJ, pJ, dc));
+                dsum = __builtin_fmaf(sig, __builtin_fmaf(gI, pJ, -gJ * pI), dsum);
+                vb[I] = __builtin_fmaf(c, gI, -ss * gJ);
+                vb[J] = __builtin_fmaf(c, gJ, ss * gI);
             }
-            if (MODE == LDS_CS_BWD) {
-                dc = wave_sum_dpp(dc);
-                dsum = wave_sum_dpp(dsum);
-                if (lane == 0) {
-                    acc[wave][2 * (C - 1 - k)] += dc;
-                    acc[wave][2 * (C - 1 - k) + 1] += dsum;
-                }
+            dc = wave_sum_f32(dc);
+            dsum = wave_sum_f32(dsum);
+            if (lane == 0) {
+                acc[wave][2 * (C - 1 - k)] += dc;
+                acc[wave][2 * (C - 1 - k) + 1] += dsum;
             }
         }
         __syncthreads();
-        const float* res = (MODE == LDS_CS_BWD) ? vb : va;
-        if (OUT)
+        if (GX)
             for (int e = tid * 4; e < nb; e += blockDim.x * 4)
-                *reinterpret_cast<float4*>(OUT + (row0 << n) + e) = *reinterpret_cast<const float4*>(&res[e]);
+                *reinterpret_cast<float4*>(GX + (row0 << n) + e) = *reinterpret_cast<const float4*>(&vb[e]);
     }
-    if (!TWO || !parts) return;
+    if (!parts) return;
     __syncthreads();
-    const int W = (MODE == LDS_CS_BWD) ? 2 * C : C;
-    for (int e = tid; e < W; e += blockDim.x)
-        parts[(long long)blockIdx.x * W + e] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
+    for (int e = tid; e < 2 * C; e += blockDim.x)
+        parts[(long long)blockIdx.x * 2 * C + e] = (acc[0][e] + acc[1][e]) + (acc[2][e] + acc[3][e]);
 }
 
 // out[e] = sum_p parts[p * width + e] in fp64, one workgroup, deterministic
@@ -1228,7 +1144,7 @@ __global__ __launch_bounds__(1024) void rotor_gamma_biv_kernel(const float* __re
 
 // ---- host side --------------------------------------------------------------
 
-// register-layout kernels: n = 2 .. 10
+// register-layout kernels: n = 2 .. 8
 #define CLF_ROTOR_DISPATCH(n, CALL)       \
     switch (n) {                          \
         case 2: CALL(2); break;           \
@@ -1238,8 +1154,6 @@ __global__ __launch_bounds__(1024) void rotor_gamma_biv_kernel(const float* __re
         case 6: CALL(6); break;           \
         case 7: CALL(7); break;           \
         case 8: CALL(8); break;           \
-        case 9: CALL(9); break;           \
-        case 10: CALL(10); break;         \
         default: break;                   \
     }
 
@@ -1259,8 +1173,6 @@ __global__ __launch_bounds__(1024) void rotor_gamma_biv_kernel(const float* __re
         case 12: CALL(12); break;         \
         default: break;                   \
     }
-
-constexpr int kRegChainMaxN = 10;  // largest n of the default register layout (64 floats on 2^(n-6) lanes)
 
 // one entry per lane up to n = 8 (64 entries), one column per lane above
 template <int N>
@@ -1310,28 +1222,21 @@ static int check_rotor_n(int n) {
 int rotor_state_floats(int n) { return (n >= kRotorMinN && n <= kRotorMaxN) ? state_floats(n) : -1; }
 
 // Workgroups of a backward launch (and so partials in the workspace): the
-// register kernels take 256 >> (lanes per row) rows per workgroup, the
-// LDS-staged kernel kLdsBlades / 2^n rows.
-static bool use_wave_rows_bwd(int n, int64_t batch);
+// register kernels take 256 >> (lanes per row) rows per workgroup.
+bool rotor_tile_serves(int n);
+int rotor_tile_rows(int n);
 
 static int rotor_bwd_grid(int n, int64_t batch) {
-    long long rows_per_block;
-    if (use_wave_rows_bwd(n, batch)) rows_per_block = 4;
-    else if (n <= kRegChainMaxN) rows_per_block = 256 >> (n - rotor_rb(n));
-    else rows_per_block = kLdsBlades >> n > 0 ? kLdsBlades >> n : 1;
+    const long long rows_per_block = rotor_tile_serves(n) ? rotor_tile_rows(n) : 256 >> (n - rotor_rb(n));
     long long g = (batch + rows_per_block - 1) / rows_per_block;
     if (g > 1024) g = 1024;
     if (g < 1) g = 1;
     return (int)g;
 }
 
-static long long lds_groups(int n, int64_t batch) {
-    const long long rpb = kLdsBlades >> n > 0 ? kLdsBlades >> n : 1;
-    return (batch + rpb - 1) / rpb;
-}
-
 static int cs_bwd_grid(int n, int64_t batch) {
-    long long g = lds_groups(n, batch);
+    const long long rpb = kLdsBlades >> n > 0 ? kLdsBlades >> n : 1;
+    long long g = (batch + rpb - 1) / rpb;
     if (g > 1024) g = 1024;
     if (g < 1) g = 1;
     return (int)g;
@@ -1371,22 +1276,6 @@ int rotor_compile_bwd(int n, const float* biv, const float* g_state, float* g_bi
     return CLF_OK;
 }
 
-// LDS-staged chain launch: grid of at most `cap` workgroups and at most the
-// resident workgroups, never more than the row groups.
-template <int MODE>
-static unsigned lds_grid(int n, int64_t batch, long long cap) {
-    long long want = lds_groups(n, batch);
-    if (want > cap) want = cap;
-    return resident_grid((const void*)rotor_chain_lds_kernel<MODE>, 256, 0, want);
-}
-
-template <int MODE>
-static void launch_lds(int n, const float* cs, const float* a, const float* b, float* out, float* parts, int64_t batch,
-                       unsigned grid, hipStream_t s, long long lda, long long ldb) {
-    hipLaunchKernelGGL((rotor_chain_lds_kernel<MODE>), dim3(grid), dim3(256), 0, s, n, cs, a, b, out, parts,
-                       (long long)batch, lda, ldb);
-}
-
 template <int N>
 static void launch_apply_reg(bool fwd, const float* cs, const float* x, float* y, int64_t batch, hipStream_t s,
                              long long ldx) {
@@ -1402,60 +1291,27 @@ static void launch_apply_reg(bool fwd, const float* cs, const float* x, float* y
     }
 }
 
-// One wave per row (four rows per workgroup, 2^(n-6) floats per lane) where
-// it measured faster than the default layouts (rotor_rb: 64 floats on
-// 2^(n-6) lanes; the LDS-staged chain at n = 11, 12). Device time of one
-// forward apply, old -> wave rows: n = 9 19.5 -> 9.2 us at 64 to 2048 rows,
-// 24.2 -> 17.9 at 8192, even at 16384, 56 -> 66 at 32768 rows; n = 10
-// 30 -> 14.5 at 64 rows, 532 -> 455 at 131072; n = 11 43 -> 26.4 at 64 rows,
-// 1535 -> 532 at 65536; n = 12 51.4 -> 62.5 at 64 rows, 57.1 -> 63.8 at
-// 512, 77.9 -> 66.6 at 1024, 1848 -> 1100 at 32768.
-static bool use_wave_rows(int n, int64_t batch) {
-    switch (n) {
-        case 9: return batch <= 12288;
-        case 10:
-        case 11: return true;
-        case 12: return batch > 768;
-        default: return false;
-    }
-}
-
-template <int N>
-static void launch_apply_wave_rows(bool fwd, const float* cs, const float* x, float* y, int64_t batch, hipStream_t s,
-                                   long long ldx) {
-    const dim3 grid((unsigned)((batch + 3) / 4));
-    if (fwd)
-        hipLaunchKernelGGL((rotor_apply_kernel<N, true, N - 6>), grid, dim3(256), 0, s, cs, x, y, (long long)batch,
-                           ldx);
-    else
-        hipLaunchKernelGGL((rotor_apply_kernel<N, false, N - 6>), grid, dim3(256), 0, s, cs, x, y, (long long)batch,
-                           ldx);
-}
+// n = 9 .. 12: tiles of generators (rotor_tile.hip)
+void rotor_tile_apply(int n, bool fwd, const float* cs, const float* x, float* y, int64_t batch, void* stream,
+                      long long ldx);
+int rotor_tile_bwd(int n, const float* cs, const float* x, const float* gy, long long ldg, float* gx, float* parts,
+                   int64_t batch, int wanted, void* stream);
 
 // y = chain(cs) x (fwd) or chain(cs)^T x, any n in range, batch > 0; x's rows
 // are ldx floats apart (2^n, or 0 for one row broadcast over the batch)
 static void launch_chain(int n, bool fwd, const float* cs, const float* x, float* y, int64_t batch, hipStream_t s,
                          long long ldx) {
-    if (use_wave_rows(n, batch)) {
-        switch (n) {
-            case 9: launch_apply_wave_rows<9>(fwd, cs, x, y, batch, s, ldx); break;
-            case 10: launch_apply_wave_rows<10>(fwd, cs, x, y, batch, s, ldx); break;
-            case 11: launch_apply_wave_rows<11>(fwd, cs, x, y, batch, s, ldx); break;
-            default: launch_apply_wave_rows<12>(fwd, cs, x, y, batch, s, ldx); break;
-        }
-    } else if (n <= kRegChainMaxN) {
-#define CLF_CALL(N) launch_apply_reg<N>(fwd, cs, x, y, batch, s, ldx)
-        CLF_ROTOR_DISPATCH(n, CLF_CALL)
-#undef CLF_CALL
-    } else if (fwd) {
-        launch_lds<LDS_FWD>(n, cs, x, nullptr, y, nullptr, batch, lds_grid<LDS_FWD>(n, batch, 1LL << 30), s, ldx, 0);
-    } else {
-        launch_lds<LDS_TR>(n, cs, x, nullptr, y, nullptr, batch, lds_grid<LDS_TR>(n, batch, 1LL << 30), s, ldx, 0);
+    if (rotor_tile_serves(n)) {
+        rotor_tile_apply(n, fwd, cs, x, y, batch, s, ldx);
+        return;
     }
+#define CLF_CALL(N) launch_apply_reg<N>(fwd, cs, x, y, batch, s, ldx)
+    CLF_ROTOR_DISPATCH(n, CLF_CALL)
+#undef CLF_CALL
 }
 
-// Composite backward with the K statistics: the register kernel (n <= 10) or
-// the LDS-staged kernel; returns the number of partials written.
+// Composite backward with the K statistics; returns the number of partials
+// written.
 template <int N>
 static int launch_apply_bwd_reg(const float* cs, const float* x, const float* gy, long long ldg, float* gx, float* ws,
                                 int64_t batch, hipStream_t s) {
@@ -1465,46 +1321,13 @@ static int launch_apply_bwd_reg(const float* cs, const float* x, const float* gy
     return (int)grid;
 }
 
-// The backward with the statistics on one wave per row (2^(n-6) floats per
-// lane) where it measured faster. Device time of one call (gx and the
-// partials), old -> wave rows: n = 9 40.1 -> 23.0 us at 64 rows, 40.8 -> 24.4
-// at 1024, 47.1 -> 50.5 at 8192; n = 10 55.8 -> 33.3 at 64, 58.5 -> 35.9 at
-// 1024, 79.5 -> 81.5 at 8192; n = 11 108 -> 63.5 at 64, 602 -> 178 at 8192
-// (the LDS-staged chain before); n = 12 132 -> 101 at 64, 725 -> 347 at 4096.
-static bool use_wave_rows_bwd(int n, int64_t batch) {
-    if (n == 9 || n == 10) return batch <= 4096;
-    return n == 11 || n == 12;
-}
-
-template <int N>
-static int launch_apply_bwd_wave_rows(const float* cs, const float* x, const float* gy, long long ldg, float* gx,
-                                      float* ws, int64_t batch, hipStream_t s) {
-    const unsigned grid =
-        resident_grid((const void*)rotor_apply_bwd_kernel<N, N - 6>, 256, 0, rotor_bwd_grid(N, batch));
-    hipLaunchKernelGGL((rotor_apply_bwd_kernel<N, N - 6>), dim3(grid), dim3(256), 0, s, cs, x, gy, gx, ws,
-                       (long long)batch, ldg);
-    return (int)grid;
-}
-
 static int launch_gamma(int n, const float* cs, const float* x, const float* gy, long long ldg, float* gx, float* ws,
                         int64_t batch, hipStream_t s) {
+    if (rotor_tile_serves(n)) return rotor_tile_bwd(n, cs, x, gy, ldg, gx, ws, batch, rotor_bwd_grid(n, batch), s);
     int nparts = 0;
-    if (use_wave_rows_bwd(n, batch)) {
-        switch (n) {
-            case 9: nparts = launch_apply_bwd_wave_rows<9>(cs, x, gy, ldg, gx, ws, batch, s); break;
-            case 10: nparts = launch_apply_bwd_wave_rows<10>(cs, x, gy, ldg, gx, ws, batch, s); break;
-            case 11: nparts = launch_apply_bwd_wave_rows<11>(cs, x, gy, ldg, gx, ws, batch, s); break;
-            default: nparts = launch_apply_bwd_wave_rows<12>(cs, x, gy, ldg, gx, ws, batch, s); break;
-        }
-    } else if (n <= kRegChainMaxN) {
 #define CLF_CALL(N) nparts = launch_apply_bwd_reg<N>(cs, x, gy, ldg, gx, ws, batch, s)
-        CLF_ROTOR_DISPATCH(n, CLF_CALL)
+    CLF_ROTOR_DISPATCH(n, CLF_CALL)
 #undef CLF_CALL
-    } else {
-        const unsigned grid = lds_grid<LDS_GAMMA>(n, batch, rotor_bwd_grid(n, batch));
-        launch_lds<LDS_GAMMA>(n, cs, x, gy, gx, ws, batch, grid, s, 1LL << n, ldg);
-        nparts = (int)grid;
-    }
     return nparts;
 }
 
@@ -1642,9 +1465,9 @@ int rotor_cs_apply_bwd(int n, const float* cs, const float* y, const float* gy, 
         if (!g_cs) {
             launch_chain(n, false, cs, gy, gx, batch, s, ldg);
         } else {
-            const unsigned grid = lds_grid<LDS_CS_BWD>(n, batch, cs_bwd_grid(n, batch));
-            launch_lds<LDS_CS_BWD>(n, cs, y, gy, gx, parts, batch, grid, s, 1LL << n, ldg);
-            nparts = (int)grid;
+            nparts = (int)resident_grid((const void*)rotor_cs_bwd_kernel, 256, 0, cs_bwd_grid(n, batch));
+            hipLaunchKernelGGL(rotor_cs_bwd_kernel, dim3((unsigned)nparts), dim3(256), 0, s, n, cs, y, gy, gx, parts,
+                               (long long)batch, ldg);
         }
         CLF_HIP_CHECK(hipGetLastError());
     }
