@@ -1896,6 +1896,13 @@ __device__ __forceinline__ float row16_merge(float x, unsigned h) {
     return h == 0u ? a3 : (h == 15u ? b3 : x);
 }
 
+// A kept output block is formed at its own step: without this the selections
+// of all steps were evaluated after the last one (nothing in between uses
+// them), with every step's accumulators alive until then. At n = 8 (11 steps)
+// that spilled 250 (contractions, wedge, regressive) to 400 registers (inner):
+// backward at 60013 rows lc 372 -> 85 us, wedge 367 -> 96, inner 643 -> 99.
+__device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
+
 template <int N, bool LOWNEG, bool WA, bool WB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void prod_bwd_inner_frame(
     const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, float* __restrict__ GA,
@@ -2094,8 +2101,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
                 const unsigned ms = lane_mask(store_t == t);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    if (WA) ya[e] = bsel(ms, ca[e], ya[e]);
-                    if (WB) yb[e] = bsel(ms, cb[e], yb[e]);
+                    if (WA) {
+                        ya[e] = bsel(ms, ca[e], ya[e]);
+                        pin(ya[e]);
+                    }
+                    if (WB) {
+                        yb[e] = bsel(ms, cb[e], yb[e]);
+                        pin(yb[e]);
+                    }
                 }
             } else if (store_t == t) {
                 store();
@@ -2434,8 +2447,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
                 const float ys = kW ? contr_out_sup<true>(acc, k) : contr_out_sub<LOWNEG, kLC>(acc, k);
                 const float yp = contr_out_sup<!kLC>(acc, k);
                 const float y = K == 1 ? ys : K == 2 ? yp : bsel(msub, ys, yp);
-                if constexpr (Cs::any_first(t)) y1[k] = bsel(m1, y, y1[k]);
-                if constexpr (Cs::any_second(t)) y2[k] = bsel(m2, y, y2[k]);
+                if constexpr (Cs::any_first(t)) {
+                    y1[k] = bsel(m1, y, y1[k]);
+                    pin(y1[k]);
+                }
+                if constexpr (Cs::any_second(t)) {
+                    y2[k] = bsel(m2, y, y2[k]);
+                    pin(y2[k]);
+                }
             }
             if constexpr (Cs::any_first(t)) {
 #pragma unroll
