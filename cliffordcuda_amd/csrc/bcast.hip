@@ -12,6 +12,15 @@
 // gw[m] = sum_{(i,kout) fed by w[m]} sigma * G[i, kout] with G = x^T gy, a
 // split-K MFMA GEMM over the batch followed by a deterministic reduction.
 //
+// Where the per-row kernels have a form made for the op and signature (every
+// masked product with a uniform low metric, the geometric products of a matrix
+// representation) they take fewer operations than the dense matrix: 3^n terms
+// or 2^(3n/2) multiply-adds a row against 4^n. The layer then runs on them, the
+// weight read as one row for every batch row, and the weight gradient as the
+// column sums of the per-row gradients, which each chunk of rows leaves in the
+// workspace. The GEMMs serve the rest (mixed or null low metrics, geometric
+// products without a representation).
+//
 // GEMM kernels: 256 threads, 128 x 128 output tile, K staged through LDS in
 // chunks of 32, each wave a 64 x 64 sub-tile of 2 x 2 v_mfma_f32_32x32x2f32
 // blocks (operand lanes: A[m = l%32][k = l/32], B[k = l/32][n = l%32];
@@ -261,6 +270,56 @@ __global__ __launch_bounds__(256) void bcast_gw_kernel(int op, int side, int n, 
     if (m < D && lane == 0) gw[m] = t;
 }
 
+// ---- column sums of the per-row weight gradients ----------------------------
+
+// parts[b][c] (+)= sum of the rows b takes of column c: 256 >> d4_log rows per
+// pass, eight passes' loads in flight, the row groups added through LDS.
+template <bool ADD>
+__global__ __launch_bounds__(256) void column_sum_kernel(const float4* __restrict__ rows, long long nrows, int d4_log,
+                                                         float4* __restrict__ parts) {
+    __shared__ float4 red[256];
+    const int c = threadIdx.x & ((1 << d4_log) - 1), rg = threadIdx.x >> d4_log, per = 256 >> d4_log;
+    const long long step = (long long)gridDim.x * per;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto add = [&](const float4& v) {
+        acc.x += v.x;
+        acc.y += v.y;
+        acc.z += v.z;
+        acc.w += v.w;
+    };
+    long long r = (long long)blockIdx.x * per + rg;
+    for (; r + 7 * step < nrows; r += 8 * step) {
+        float4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = rows[((r + u * step) << d4_log) + c];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) add(v[u]);
+    }
+    for (; r < nrows; r += step) add(rows[(r << d4_log) + c]);
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    if (rg != 0) return;
+    for (int g = 1; g < per; ++g) add(red[(g << d4_log) + c]);
+    float4* out = parts + ((long long)blockIdx.x << d4_log) + c;
+    if (ADD) add(*out);
+    *out = acc;
+}
+
+// gw[c] = sum of the nparts partials of column c, in fp64: 32 columns per
+// workgroup, eight threads each
+__global__ __launch_bounds__(256) void column_total_kernel(const float* __restrict__ parts, int nparts, int n,
+                                                           float* __restrict__ gw) {
+    __shared__ double red[256];
+    const int c = blockIdx.x * 32 + (threadIdx.x & 31);
+    double t = 0.0;
+    for (int p = threadIdx.x >> 5; p < nparts; p += 8) t += (double)parts[((long long)p << n) + c];
+    red[threadIdx.x] = t;
+    __syncthreads();
+    if (threadIdx.x >= 32) return;
+    for (int g = 1; g < 8; ++g) t += red[g * 32 + threadIdx.x];
+    gw[c] = (float)t;
+}
+
 // ---- host side --------------------------------------------------------------
 
 bool rep_bcast_applicable(int op, int n, uint32_t neg, uint32_t nul);
@@ -277,13 +336,89 @@ static int bcast_splits(int64_t batch, int cap = 128) {
     return (int)s;
 }
 
-// The GEMM path's workspace; it also covers the matrix-representation path's
-// weight-gradient partials (256 floats per workgroup, at most 2048 workgroups
-// and at most 16 * batch floats, below (3 + splits) * 2^(2n) for n >= 7).
+static size_t rows_ws_floats(int n, int64_t batch);
+
+// The larger of the GEMM path's and the rows path's workspace; it also covers
+// the matrix-representation path's weight-gradient partials (256 floats per
+// workgroup, at most 2048 workgroups and at most 16 * batch floats, below
+// (3 + splits) * 2^(2n) for n >= 7).
 size_t bcast_ws_bytes(int n, int64_t batch) {
     if (n < kBcastMinN || n > kMaxN || batch < 0) return 0;
     const size_t DD = (size_t)1 << (2 * n);
-    return (2 + (size_t)bcast_splits(batch) + 1) * DD * sizeof(float);
+    const size_t gemm = (2 + (size_t)bcast_splits(batch) + 1) * DD, rows = rows_ws_floats(n, batch);
+    return (gemm > rows ? gemm : rows) * sizeof(float);
+}
+
+bool product_has_form(int op, int n, uint32_t neg, uint32_t nul);
+int product_fwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b,
+                   int64_t ldb, float* c, int64_t batch, void* stream);
+int product_bwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b,
+                   int64_t ldb, const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
+
+// Rows path: workgroups (and partials) of the column sums, and the bytes of a
+// chunk of rows: the per-row weight gradients of a chunk stay in the 256 MB
+// last-level cache beside the rows streamed, and with the partials they fit the
+// allocation-free entry's scratch.
+constexpr int kSumBlocks = 256;
+constexpr size_t kChunkBytes = (size_t)31 << 20;
+constexpr size_t kBcastScratchBytes = (size_t)32 << 20;
+static_assert(kChunkBytes + kSumBlocks * (sizeof(float) << 10) <= kBcastScratchBytes, "n <= 10 fits the scratch");
+
+static int64_t rows_chunk(int n, int64_t batch) {
+    const int64_t c = (int64_t)(kChunkBytes >> (n + 2));
+    return batch < c ? batch : c;
+}
+
+// the per-row weight gradients of a chunk, the column sums' partials
+static size_t rows_ws_floats(int n, int64_t batch) {
+    return ((size_t)rows_chunk(n, batch) + kSumBlocks) << n;
+}
+
+// GEMMs against the per-row kernels (us, forward + backward): n = 7, 120000
+// rows: geom 48 + 225 -> 27 + 76, wedge 46 + 224 -> 24 + 82, inner 46 + 223 ->
+// 31 + 90; n = 8, 60013 rows: wedge 75 + 238 -> 38 + 110, inner 74 + 239 ->
+// 52 + 122, Cl(7,1) geom 83 + 253 -> 26 + 80, and at 2000 rows inner 26 + 185
+// -> 8 + 29; n = 9, 20000 rows: geom 117 + 290 -> 25 + 88, inner 105 + 267 ->
+// 46 + 141; n = 10, 4096 rows: geom 93 + 257 -> 11 + 38, inner 94 + 257 ->
+// 31 + 109. No form measured slower at any batch. The backward is bound by
+// writing and reading back the per-row weight gradients beside x, gy and gx.
+static bool use_rows(int op, int n, uint32_t neg, uint32_t nul) { return product_has_form(op, n, neg, nul); }
+
+static int rows_fwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* x, const float* w, float* y,
+                    int64_t batch, void* stream) {
+    return side == 0 ? product_fwd_ld(op, n, neg, nul, x, 1, w, 0, y, batch, stream)
+                     : product_fwd_ld(op, n, neg, nul, w, 0, x, 1, y, batch, stream);
+}
+
+static int rows_bwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* x, const float* w,
+                    const float* gy, int64_t ldg, float* gx, float* gw, int64_t batch, float* ws, void* stream) {
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t chunk = gw ? rows_chunk(n, batch) : batch;
+    float* parts = ws + ((size_t)chunk << n);
+    const int per = 256 >> (n - 2);
+    const int64_t groups = (chunk + per - 1) / per;
+    const int nparts = (int)(groups < kSumBlocks ? groups : kSumBlocks);
+    for (int64_t r0 = 0; r0 < batch; r0 += chunk) {
+        const int64_t rows = batch - r0 < chunk ? batch - r0 : chunk;
+        // x is read for the weight gradient alone; the weight stands in where it is not given
+        const float* xs = gw ? x + (r0 << n) : w;
+        const int64_t ldx = gw ? 1 : 0;
+        float* gxs = gx ? gx + (r0 << n) : nullptr;
+        float* gws = gw ? ws : nullptr;
+        const float* gys = gy + r0 * ldg;
+        const int rc =
+            side == 0 ? product_bwd_ld(op, n, neg, nul, xs, ldx, w, 0, gys, ldg, gxs, gws, rows, stream)
+                      : product_bwd_ld(op, n, neg, nul, w, 0, xs, ldx, gys, ldg, gws, gxs, rows, stream);
+        if (rc) return rc;
+        if (!gw) continue;
+        const float4* g4 = reinterpret_cast<const float4*>(ws);
+        float4* p4 = reinterpret_cast<float4*>(parts);
+        if (r0 == 0) hipLaunchKernelGGL((column_sum_kernel<false>), dim3(nparts), dim3(256), 0, s, g4, rows, n - 2, p4);
+        else hipLaunchKernelGGL((column_sum_kernel<true>), dim3(nparts), dim3(256), 0, s, g4, rows, n - 2, p4);
+    }
+    if (gw) hipLaunchKernelGGL(column_total_kernel, dim3(1u << (n - 5)), dim3(256), 0, s, parts, nparts, n, gw);
+    CLF_HIP_CHECK(hipGetLastError());
+    return CLF_OK;
 }
 
 static int check_bcast(int op, int side, int n, uint32_t neg, uint32_t nul, int64_t batch) {
@@ -329,6 +464,8 @@ int bcast_fwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* 
     if ((((uintptr_t)x) | ((uintptr_t)y) | ((uintptr_t)ws)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
     if (rep_bcast_applicable(op, n, neg, nul)) return rep_bcast_fwd(side, n, neg, x, w, y, batch, stream);
+    if (use_rows(op, n, neg, nul) && !(((uintptr_t)w) & 15u))
+        return rows_fwd(op, side, n, neg, nul, x, w, y, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     const int D = 1 << n;
     float* MwT = (float*)ws;
@@ -361,6 +498,8 @@ static int bcast_bwd_launch(int op, int side, int n, uint32_t neg, uint32_t nul,
                             int max_splits, void* stream) {
     if (rep_bcast_applicable(op, n, neg, nul))
         return rep_bcast_bwd(side, n, neg, x, w, gy, ldg, gx, gw, batch, ws, stream);
+    if (batch > 0 && use_rows(op, n, neg, nul) && !(((uintptr_t)w) & 15u))
+        return rows_bwd(op, side, n, neg, nul, x, w, gy, ldg, gx, gw, batch, ws, stream);
     hipStream_t s = (hipStream_t)stream;
     const int D = 1 << n;
     const size_t DD = (size_t)D * D;
@@ -415,7 +554,6 @@ int bcast_bwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* 
 // (different streams or threads) race on it. No kernel relies on its previous
 // contents: every workspace entry a launch reads was written earlier in the
 // same call.
-constexpr size_t kBcastScratchBytes = (size_t)32 << 20;
 static __device__ __align__(256) float scratch[kBcastScratchBytes / sizeof(float)];
 
 constexpr int kScratchMaxDevices = 64;
@@ -458,6 +596,8 @@ int bcast_bwd_noalloc(int op, int side, int n, uint32_t neg, uint32_t nul, const
     size_t need;
     if (rep_bcast_applicable(op, n, neg, nul)) {
         need = rep_bcast_ws_floats(batch) * sizeof(float);
+    } else if (use_rows(op, n, neg, nul)) {
+        need = rows_ws_floats(n, batch) * sizeof(float);
     } else {
         const int cap = noalloc_max_splits(n);
         if (cap < 1)

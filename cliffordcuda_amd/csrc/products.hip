@@ -391,6 +391,7 @@ struct BlkParams {
     int wpr_log;    // small-batch kernels: log2 of the workgroups per row
     unsigned rskew; // blocked kernels: 2-bit slot skew of staged row r at bits 2 (r & 15)
     unsigned negl;  // metric mask, bits 0-3 (the regressive product's dual signs)
+    bool bca, bcb;  // a / b is one row read for every batch row (not on the whole-row, tiled and generic kernels)
 };
 
 // Stage NOPS (2 or 3) row-major operands s0, s1[, s2] for the workgroup's rows
@@ -400,10 +401,11 @@ struct BlkParams {
 template <int NOPS, bool BSLOT = false>
 __device__ __forceinline__ void stage_rows(float4* __restrict__ lds, const float4* __restrict__ s0,
                                            const float4* __restrict__ s1, const float4* __restrict__ s2,
-                                           long long row0, int nrows, int n, long long m2 = -1, unsigned rskew = 0u) {
+                                           long long row0, int nrows, int n, long long m2 = -1, unsigned rskew = 0u,
+                                           long long m0 = -1, long long m1 = -1) {
     // BSLOT: the blocked kernels' slots (bslot with the row skews in rskew), else swz
     // m2 masks s2's float4 index: -1 (packed like s0 and s1) or 2^(n-2) - 1
-    // (one row for all rows: the row offset drops out)
+    // (one row for all rows: the row offset drops out); m0, m1 likewise
     const int d4_log = n - 2;
     const int D4 = 1 << d4_log;
     const int total = nrows << d4_log;
@@ -412,8 +414,10 @@ __device__ __forceinline__ void stage_rows(float4* __restrict__ lds, const float
     for (int base = (int)threadIdx.x; base < total; base += 4 * nt) {
         const int i0 = base, i1 = base + nt, i2 = base + 2 * nt, i3 = base + 3 * nt;
         const int c1 = i1 < total ? i1 : total - 1, c2 = i2 < total ? i2 : total - 1, c3 = i3 < total ? i3 : total - 1;
-        const float4 a0 = s0[g0 + i0], a1 = s0[g0 + c1], a2 = s0[g0 + c2], a3 = s0[g0 + c3];
-        const float4 b0 = s1[g0 + i0], b1 = s1[g0 + c1], b2 = s1[g0 + c2], b3 = s1[g0 + c3];
+        const float4 a0 = s0[(g0 + i0) & m0], a1 = s0[(g0 + c1) & m0], a2 = s0[(g0 + c2) & m0],
+                     a3 = s0[(g0 + c3) & m0];
+        const float4 b0 = s1[(g0 + i0) & m1], b1 = s1[(g0 + c1) & m1], b2 = s1[(g0 + c2) & m1],
+                     b3 = s1[(g0 + c3) & m1];
         float4 e0, e1, e2, e3;
         if constexpr (NOPS == 3) {
             e0 = s2[(g0 + i0) & m2];
@@ -649,7 +653,9 @@ __global__ __launch_bounds__(256) void prod_fwd_split(const float* __restrict__ 
     const unsigned S = 1u << P.split_log;
     const long long row = (long long)(blockIdx.x >> P.wpr_log);
     const unsigned ogrp = blockIdx.x & ((1u << P.wpr_log) - 1u);
-    stage_rows<2>(lds, reinterpret_cast<const float4*>(A), reinterpret_cast<const float4*>(B), nullptr, row, 1, n);
+    const long long one = (1LL << (n - 2)) - 1;
+    stage_rows<2>(lds, reinterpret_cast<const float4*>(A), reinterpret_cast<const float4*>(B), nullptr, row, 1, n, -1,
+                  0u, P.bca ? one : -1, P.bcb ? one : -1);
     __syncthreads();
     const unsigned sl = threadIdx.x & (S - 1u), ol = threadIdx.x >> P.split_log;
     const unsigned G = 256u >> P.split_log;
@@ -700,8 +706,10 @@ __global__ __launch_bounds__(256) void prod_bwd_split(const float* __restrict__ 
     const unsigned S = 1u << P.split_log;
     const long long row = (long long)(blockIdx.x >> P.wpr_log);
     const unsigned ogrp = blockIdx.x & ((1u << P.wpr_log) - 1u);
+    const long long one = (1LL << (n - 2)) - 1;
     stage_rows<3>(lds, reinterpret_cast<const float4*>(A), reinterpret_cast<const float4*>(B),
-                  reinterpret_cast<const float4*>(GC), row, 1, n, P.ldg4 ? -1LL : (1LL << (n - 2)) - 1);
+                  reinterpret_cast<const float4*>(GC), row, 1, n, P.ldg4 ? -1LL : one, 0u, P.bca ? one : -1,
+                  P.bcb ? one : -1);
     __syncthreads();
     const unsigned sl = threadIdx.x & (S - 1u), ol = threadIdx.x >> P.split_log;
     const unsigned G = 256u >> P.split_log;
@@ -1544,13 +1552,13 @@ __global__ __launch_bounds__(256) void prod_fwd_bal(const float* __restrict__ A,
     long long grp = (long long)blockIdx.x * 4 + wave;
     const BalLane L = bal_lane(n, lane);
     const int d4_log = n - 2;
-    BalPre pa = bal_fetch(bal_src(A, grp, P.batch, n, R), L, d4_log);
-    BalPre pb = bal_fetch(bal_src(B, grp, P.batch, n, R), L, d4_log);
+    BalPre pa = bal_fetch(bal_src(A, grp, P.batch, n, R, P.bca), L, d4_log);
+    BalPre pb = bal_fetch(bal_src(B, grp, P.batch, n, R, P.bcb), L, d4_log);
     for (; grp < ngrp; grp += gstride) {
         bal_stage(sa, pa, L);
         bal_stage(sb, pb, L);
-        pa = bal_fetch(bal_src(A, grp + gstride, P.batch, n, R), L, d4_log);
-        pb = bal_fetch(bal_src(B, grp + gstride, P.batch, n, R), L, d4_log);
+        pa = bal_fetch(bal_src(A, grp + gstride, P.batch, n, R, P.bca), L, d4_log);
+        pb = bal_fetch(bal_src(B, grp + gstride, P.batch, n, R, P.bcb), L, d4_log);
         wave_lds_sync();
         const long long row = grp * R + r;
         float4* out = row < P.batch ? reinterpret_cast<float4*>(C) + (row << (n - 2)) : nullptr;
@@ -1634,8 +1642,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
     const int d4_log = n - 2;
     const bool gbc = P.ldg4 == 0;  // gc: one row for all rows
     BalPre pa, pb;
-    if (want_b) pa = bal_fetch(bal_src(A, grp, P.batch, n, R), L, d4_log);
-    if (want_a) pb = bal_fetch(bal_src(B, grp, P.batch, n, R), L, d4_log);
+    if (want_b) pa = bal_fetch(bal_src(A, grp, P.batch, n, R, P.bca), L, d4_log);
+    if (want_a) pb = bal_fetch(bal_src(B, grp, P.batch, n, R, P.bcb), L, d4_log);
     BalPre pg = bal_fetch(bal_src(GC, grp, P.batch, n, R, gbc), L, d4_log);
     for (; grp < ngrp; grp += gstride) {
         const long long row = grp * R + r;
@@ -1644,7 +1652,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
         pg = bal_fetch(bal_src(GC, grp + gstride, P.batch, n, R, gbc), L, d4_log);
         if (want_a) {  // uniform: a kernel argument
             bal_stage(sb, pb, L);
-            pb = bal_fetch(bal_src(B, grp + gstride, P.batch, n, R), L, d4_log);
+            pb = bal_fetch(bal_src(B, grp + gstride, P.batch, n, R, P.bcb), L, d4_log);
             wave_lds_sync();
             float4* out = row_ok ? reinterpret_cast<float4*>(GA) + (row << (n - 2)) : nullptr;
             if constexpr (kDeals) {
@@ -1663,7 +1671,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
         }
         if (want_b) {
             bal_stage(sa, pa, L);
-            pa = bal_fetch(bal_src(A, grp + gstride, P.batch, n, R), L, d4_log);
+            pa = bal_fetch(bal_src(A, grp + gstride, P.batch, n, R, P.bca), L, d4_log);
             wave_lds_sync();
             float4* out = row_ok ? reinterpret_cast<float4*>(GB) + (row << (n - 2)) : nullptr;
             if constexpr (kDeals) {
@@ -1932,8 +1940,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
     const bool gbc = P.ldg4 == 0;
     // the group's loads are in flight while the step table is built
     BalPre pa, pb, pg;
-    if (WB) pa = bal_fetch(bal_src(A, grp, P.batch, N, R), L, N - 2);
-    if (WA) pb = bal_fetch(bal_src(B, grp, P.batch, N, R), L, N - 2);
+    if (WB) pa = bal_fetch(bal_src(A, grp, P.batch, N, R, P.bca), L, N - 2);
+    if (WA) pb = bal_fetch(bal_src(B, grp, P.batch, N, R, P.bcb), L, N - 2);
     pg = bal_fetch(bal_src(GC, grp, P.batch, N, R, gbc), L, N - 2);
     // entry: block offsets (gc block o ^ p; partner p, its slot order reversed
     // in sub mode), sub flag, the high-part signs, the parities of p and o, and
@@ -2312,8 +2320,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void p
         }
         return p;
     };
-    const BalPre pa = fetch(A, false, 0);
-    const BalPre pb = fetch(B, false, 1);
+    const BalPre pa = fetch(A, P.bca, 0);
+    const BalPre pb = fetch(B, P.bcb, 1);
     const BalPre pg = fetch(GC, gbc, 2);
     // entry: gc block offset (o ^ p), partner offset (a at +0, b at +4 KB; slot
     // order reversed in sub mode), then the step's flip bits: pair sign S,
@@ -2569,14 +2577,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         unsigned lo = (unsigned)lane;  // opaque: the loop keeps no lane-derived pointers
         asm volatile("" : "+v"(lo));
         const BalLane L = bal_lane(N, (int)lo);
-        const BalSrc sa = bal_src(A, g, P.batch, N, R);
+        const BalSrc sa = bal_src(A, g, P.batch, N, R, P.bca);
         if constexpr (NULLTOP) {  // a0 only: chunks 0, 1 of the row
             pa.v[0] = sa.g0[L.ff[0]];
             pa.v[1] = sa.g0[L.ff[1]];
         } else {
             pa = bal_fetch(sa, L, N - 2);
         }
-        pb = bal_fetch(bal_src(B, g, P.batch, N, R), L, N - 2);
+        pb = bal_fetch(bal_src(B, g, P.batch, N, R, P.bcb), L, N - 2);
         pg = bal_fetch(bal_src(GC, g, P.batch, N, R, P.ldg4 == 0), L, N - 2);
     };
     fetch(grp < ngrp ? grp : ngrp - 1);
@@ -2813,8 +2821,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void p
         unsigned lo = (unsigned)lane;  // opaque: the loop keeps no lane-derived pointers
         asm volatile("" : "+v"(lo));
         const BalLane L = bal_lane(N, (int)lo);
-        pa = bal_fetch(bal_src(A, g, P.batch, N, R), L, N - 2);
-        pb = bal_fetch(bal_src(B, g, P.batch, N, R), L, N - 2);
+        pa = bal_fetch(bal_src(A, g, P.batch, N, R, P.bca), L, N - 2);
+        pb = bal_fetch(bal_src(B, g, P.batch, N, R, P.bcb), L, N - 2);
         pg = bal_fetch(bal_src(GC, g, P.batch, N, R, P.ldg4 == 0), L, N - 2);
     };
     fetch(grp < ngrp ? grp : ngrp - 1);
@@ -3084,14 +3092,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void p
         unsigned lo = (unsigned)lane;  // opaque: the loop keeps no lane-derived addresses
         asm volatile("" : "+v"(lo));
         const BalLane L = bal_lane(N, (int)lo);
-        const BalSrc sa = bal_src(A, g, P.batch, N, R);
+        const BalSrc sa = bal_src(A, g, P.batch, N, R, P.bca);
         if constexpr (NULLTOP) {
             pa.v[0] = sa.g0[L.ff[0]];
             pa.v[1] = sa.g0[L.ff[1]];
         } else {
             pa = bal_fetch(sa, L, N - 2);
         }
-        pb = bal_fetch(bal_src(B, g, P.batch, N, R), L, N - 2);
+        pb = bal_fetch(bal_src(B, g, P.batch, N, R, P.bcb), L, N - 2);
     };
     fetch(grp < ngrp ? grp : ngrp - 1);
     // entries: a byte offset (bits 0-13), b byte offset (14-27), high sign (28), cross parity |ih| (29)
@@ -3307,8 +3315,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(OP == OP_WE
     const long long ngrp = (P.batch + R - 1) / R;
     const long long grp = (long long)blockIdx.x * 4 + wave;
     const BalLane L = bal_lane<kFwd7RowX>(N, lane);
-    const BalPre pa = bal_fetch(bal_src(A, grp, P.batch, N, R), L, N - 2);
-    const BalPre pb = bal_fetch(bal_src(B, grp, P.batch, N, R), L, N - 2);
+    const BalPre pa = bal_fetch(bal_src(A, grp, P.batch, N, R, P.bca), L, N - 2);
+    const BalPre pb = bal_fetch(bal_src(B, grp, P.batch, N, R, P.bcb), L, N - 2);
     if (wave == 0 && lane < 32) {
         const unsigned th = (unsigned)lane & full, trs = row_x<kFwd7RowX>((unsigned)lane >> 3);
 #pragma unroll
@@ -3774,8 +3782,10 @@ static void launch_out7(hipStream_t s, bool ln, const float* a, const float* b, 
         Q.batch = (g0 + gn) * 8 < P.batch ? gn * 8 : P.batch - g0 * 8;
         const long long off = g0 * 8 * 128;
         const dim3 grid((unsigned)((gn + 3) / 4));
-        if (ln) hipLaunchKernelGGL((prod_fwd_out7<OP, true>), grid, dim3(256), 0, s, a + off, b + off, c + off, Q);
-        else hipLaunchKernelGGL((prod_fwd_out7<OP, false>), grid, dim3(256), 0, s, a + off, b + off, c + off, Q);
+        if (ln) hipLaunchKernelGGL((prod_fwd_out7<OP, true>), grid, dim3(256), 0, s, a + (P.bca ? 0 : off),
+                                   b + (P.bcb ? 0 : off), c + off, Q);
+        else hipLaunchKernelGGL((prod_fwd_out7<OP, false>), grid, dim3(256), 0, s, a + (P.bca ? 0 : off),
+                                   b + (P.bcb ? 0 : off), c + off, Q);
     }
 }
 
@@ -3793,7 +3803,8 @@ static void launch_frame3(hipStream_t s, const float* A, const float* B, const f
         const long long groups = (Q.batch + R - 1) / R;
         const dim3 g((unsigned)((groups + 3) / 4));
         const long long off = r0 * D;
-        hipLaunchKernelGGL((prod_bwd_inner_frame<N, LN, WA, WB>), g, dim3(256), 0, s, A + off, B + off,
+        hipLaunchKernelGGL((prod_bwd_inner_frame<N, LN, WA, WB>), g, dim3(256), 0, s, A + (P.bca ? 0 : off),
+                           B + (P.bcb ? 0 : off),
                            GCp + (P.ldg4 ? off : 0), GA ? GA + off : nullptr, GB ? GB + off : nullptr, Q);
     }
 }
@@ -3850,7 +3861,8 @@ static void launch_contr3(hipStream_t s, const float* A, const float* B, const f
         const long long groups = (Q.batch + R - 1) / R;
         const dim3 g((unsigned)((groups + 3) / 4));
         const long long off = r0 * D;
-        hipLaunchKernelGGL((prod_bwd_contr_frame<OP, N, LN>), g, dim3(256), 0, s, A + off, B + off,
+        hipLaunchKernelGGL((prod_bwd_contr_frame<OP, N, LN>), g, dim3(256), 0, s, A + (P.bca ? 0 : off),
+                           B + (P.bcb ? 0 : off),
                            GCp + (P.ldg4 ? off : 0), GA ? GA + off : nullptr, GB ? GB + off : nullptr, Q);
     }
 }
@@ -3915,7 +3927,8 @@ static void launch_inner5_t(hipStream_t s, const float* A, const float* B, const
         const long long groups = (Q.batch + R - 1) / R;
         const dim3 g(resident_grid((const void*)prod_bwd_inner5<LN, NT>, 256, 0, (groups + 3) / 4));
         const long long off = r0 * D;
-        hipLaunchKernelGGL((prod_bwd_inner5<LN, NT>), g, dim3(256), 0, s, A + off, B + off,
+        hipLaunchKernelGGL((prod_bwd_inner5<LN, NT>), g, dim3(256), 0, s, A + (P.bca ? 0 : off),
+                           B + (P.bcb ? 0 : off),
                            GCp + (P.ldg4 ? off : 0), GA ? GA + off : nullptr, GB ? GB + off : nullptr, Q);
     }
 }
@@ -3943,7 +3956,8 @@ static void launch_contr5_t(hipStream_t s, const float* A, const float* B, const
         const long long groups = (Q.batch + R - 1) / R;
         const dim3 g(resident_grid((const void*)prod_bwd_contr5<OP, LN, NT>, 256, 0, (groups + 3) / 4));
         const long long off = r0 * D;
-        hipLaunchKernelGGL((prod_bwd_contr5<OP, LN, NT>), g, dim3(256), 0, s, A + off, B + off,
+        hipLaunchKernelGGL((prod_bwd_contr5<OP, LN, NT>), g, dim3(256), 0, s, A + (P.bca ? 0 : off),
+                           B + (P.bcb ? 0 : off),
                            GCp + (P.ldg4 ? off : 0), GA ? GA + off : nullptr, GB ? GB + off : nullptr, Q);
     }
 }
@@ -3959,7 +3973,8 @@ static void launch_fcontr5_t(hipStream_t s, const float* A, const float* B, floa
         const long long groups = (Q.batch + R - 1) / R;
         const dim3 g(resident_grid((const void*)prod_fwd_contr5<OP, LN, NT>, 256, 0, (groups + 3) / 4));
         const long long off = r0 * D;
-        hipLaunchKernelGGL((prod_fwd_contr5<OP, LN, NT>), g, dim3(256), 0, s, A + off, B + off, C + off, Q);
+        hipLaunchKernelGGL((prod_fwd_contr5<OP, LN, NT>), g, dim3(256), 0, s, A + (P.bca ? 0 : off),
+                           B + (P.bcb ? 0 : off), C + off, Q);
     }
 }
 
@@ -4068,12 +4083,22 @@ static void launch_bwd(dim3 g, dim3 b, size_t lds, hipStream_t s, const float* A
 
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul);
 bool rep_disabled_by_env();
-int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
-            void* stream);
-int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
-            float* ga, float* gb, int64_t batch, void* stream);
-
+int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+            int64_t batch, void* stream);
+int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
+            const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
 int64_t rep32_few_rows(int n, uint32_t neg, uint32_t nul);
+
+// Whether the op has kernels made for the signature: a matrix representation
+// for the geometric product, a uniform low metric for the others (false: the
+// geometric product's 4^n terms, or the per-coefficient kernels).
+bool product_has_form(int op, int n, uint32_t neg, uint32_t nul) {
+    bool lowneg;
+    if (rep_disabled_by_env() || options().product_path != PATH_DEFAULT) return false;
+    if (op == CLF_OP_GEOM) return rep_applicable(op, n, neg, nul);
+    // (the inner product's backward with a null generator runs the whole-row kernel below n = 8)
+    return n >= 7 && n <= 10 && blocked_metric(op, n, neg, nul, lowneg) && !(op == CLF_OP_INNER && n == 7 && nul);
+}
 
 // The geometric product goes through the matrix representation where the
 // signature has one, unless CLF_GEOM_PATH=direct asks for the per-term kernels.
@@ -4085,8 +4110,10 @@ static bool use_rep(int op, int n, uint32_t neg, uint32_t nul, int64_t batch) {
     return n < 9 || batch > rep32_few_rows(n, neg, nul) || !blocked_metric(op, n, neg, nul, lowneg);
 }
 
-int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c,
-                int64_t batch, void* stream) {
+// lda, ldb: 0 if a / b is one row read for every batch row (where
+// product_has_form holds), nonzero: packed rows
+int product_fwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b,
+                   int64_t ldb, float* c, int64_t batch, void* stream) {
     int rc = check_common(op, n, neg, nul, batch);
     if (rc) return rc;
     if (batch == 0) return CLF_OK;
@@ -4094,10 +4121,13 @@ int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
     if (c == a || c == b) return set_error(CLF_ERR_ARG, "output must not alias an input");
     if ((((uintptr_t)a) | ((uintptr_t)b) | ((uintptr_t)c)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
-    if (use_rep(op, n, neg, nul, batch)) return rep_fwd(n, neg, nul, a, b, c, batch, stream);
+    if (use_rep(op, n, neg, nul, lda && ldb ? batch : INT64_MAX))
+        return rep_fwd(n, neg, nul, a, lda, b, ldb, c, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     BlkParams P{};
     P.batch = batch;
+    P.bca = lda == 0;
+    P.bcb = ldb == 0;
     bool ln = false, nt5 = false;
     dim3 g, bl;
     size_t lds = 0;
@@ -4136,6 +4166,8 @@ int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
             case OP_REGR: launch_fwd_bal<OP_REGR, false>(s, a, b, c, P); break;
         }
 #undef CLF_FWD_BAL
+    } else if (P.bca || P.bcb) {
+        return set_error(CLF_ERR_UNSUPPORTED, "this product takes packed rows");
     } else if (!force_generic && !force_tiled && blocked_plan(op, n, neg, nul, 2, P, ln, g, bl, lds)) {
 #define CLF_FWD_CASE(OPV)                                              \
     case OPV:                                                          \
@@ -4175,8 +4207,8 @@ int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
 
 // gc's rows are ldg floats apart: 2^n (packed) or 0 (one row broadcast over
 // the batch, e.g. the gradient of a sum)
-int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc,
-                int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
+int product_bwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b,
+                   int64_t ldb, const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
     int rc = check_common(op, n, neg, nul, batch);
     if (rc) return rc;
     if (ldg != 0 && ldg != (1LL << n)) return set_error(CLF_ERR_ARG, "gc row stride must be 0 or 2^n");
@@ -4186,11 +4218,14 @@ int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
         return set_error(CLF_ERR_ARG, "gradient outputs must not alias inputs or each other");
     if ((((uintptr_t)a) | ((uintptr_t)b) | ((uintptr_t)gc) | ((uintptr_t)ga) | ((uintptr_t)gb)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
-    if (use_rep(op, n, neg, nul, batch)) return rep_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
+    if (use_rep(op, n, neg, nul, lda && ldb ? batch : INT64_MAX))
+        return rep_bwd(n, neg, nul, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     BlkParams P{};
     P.batch = batch;
     P.ldg4 = ldg >> 2;
+    P.bca = lda == 0;
+    P.bcb = ldb == 0;
     bool ln = false, nt5 = false;
     dim3 g, bl;
     size_t lds = 0;
@@ -4233,6 +4268,8 @@ int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
             case OP_REGR: launch_bwd_bal<OP_REGR, false>(s, a, b, gc, ga, gb, P); break;
         }
 #undef CLF_BWD_BAL
+    } else if (P.bca || P.bcb) {
+        return set_error(CLF_ERR_UNSUPPORTED, "this product takes packed rows");
     } else if (!force_generic && !force_tiled && blocked_plan(op, n, neg, nul, 3, P, ln, g, bl, lds)) {
 #define CLF_BWD_CASE(OPV)                                                      \
     case OPV:                                                                  \
@@ -4273,6 +4310,16 @@ int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const
     }
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
+}
+
+int product_fwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c,
+                int64_t batch, void* stream) {
+    return product_fwd_ld(op, n, neg, nul, a, 1, b, 1, c, batch, stream);
+}
+
+int product_bwd(int op, int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc,
+                int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
+    return product_bwd_ld(op, n, neg, nul, a, 1, b, 1, gc, ldg, ga, gb, batch, stream);
 }
 
 }  // namespace clf

@@ -750,23 +750,28 @@ bool rep_table(int n, uint32_t neg, RepTable& T) {
 
 bool split_applicable(int op, int n, uint32_t neg, uint32_t nul);
 bool rep7_applicable(uint32_t neg);
-int rep7_fwd(uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream);
-int rep7_bwd(uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga, float* gb,
-             int64_t batch, void* stream);
-int split_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream);
-int split_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
-              float* gb, int64_t batch, void* stream);
+// lda, ldb of the functions below: 0 if a / b is one row read for every batch
+// row, nonzero: packed rows
+int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
+             void* stream);
+int rep7_bwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc, int64_t ldg,
+             float* ga, float* gb, int64_t batch, void* stream);
+int split_fwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
+              void* stream);
+int split_bwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc,
+              int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
 
 bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul);
-int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
-              void* stream);
-int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
-              float* ga, float* gb, int64_t batch, void* stream);
+int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+              int64_t batch, void* stream);
+int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
+              const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
 
 bool twist_applicable(uint32_t neg, uint32_t nul);
-int twist_fwd(uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch, void* stream);
-int twist_bwd(uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
-              float* gb, int64_t batch, void* stream);
+int twist_fwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+              int64_t batch, void* stream);
+int twist_bwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc,
+              int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
 
 // The matrix path serves the geometric product when the signature allows it
 // (real type, n = 4, 6, 8; one generator from real type, n = 8; every
@@ -811,13 +816,15 @@ static long long rep16_bwd_blocks(int64_t batch) {
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 
-int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch,
-            void* stream) {
-    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_fwd(n, neg, a, b, c, batch, stream);
-    if (n >= 9) return rep32_fwd(n, neg, nul, a, b, c, batch, stream);
-    if (n == 7) return rep7_fwd(neg, a, b, c, batch, stream);
+// (real-type n <= 8 takes packed rows only; its broadcast form is rep_bcast_fwd)
+int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+            int64_t batch, void* stream) {
+    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_fwd(n, neg, a, lda, b, ldb, c, batch, stream);
+    if (n >= 9) return rep32_fwd(n, neg, nul, a, lda, b, ldb, c, batch, stream);
+    if (n == 7) return rep7_fwd(neg, a, lda, b, ldb, c, batch, stream);
     RepTable T;
-    if (nul || !rep_table(n, neg, T)) return twist_fwd(neg, nul, a, b, c, batch, stream);
+    if (nul || !rep_table(n, neg, T)) return twist_fwd(neg, nul, a, lda, b, ldb, c, batch, stream);
+    if (!lda || !ldb) return set_error(CLF_ERR_UNSUPPORTED, "real-type products take packed rows");
     hipStream_t s = (hipStream_t)stream;
     const long long want = rep_blocks(n, batch);
 #define CLF_REP_GRID(K) dim3((unsigned)want)
@@ -849,13 +856,15 @@ int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, f
     return CLF_OK;
 }
 
-int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
-            float* ga, float* gb, int64_t batch, void* stream) {
-    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
-    if (n >= 9) return rep32_bwd(n, neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
-    if (n == 7) return rep7_bwd(neg, a, b, gc, ldg, ga, gb, batch, stream);
+int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
+            const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
+    if (split_applicable(CLF_OP_GEOM, n, neg, nul))
+        return split_bwd(n, neg, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
+    if (n >= 9) return rep32_bwd(n, neg, nul, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
+    if (n == 7) return rep7_bwd(neg, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
     RepTable T;
-    if (nul || !rep_table(n, neg, T)) return twist_bwd(neg, nul, a, b, gc, ldg, ga, gb, batch, stream);
+    if (nul || !rep_table(n, neg, T)) return twist_bwd(neg, nul, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
+    if (!lda || !ldb) return set_error(CLF_ERR_UNSUPPORTED, "real-type products take packed rows");
     hipStream_t s = (hipStream_t)stream;
     const long long want = rep_blocks(n, batch);
     switch (n) {

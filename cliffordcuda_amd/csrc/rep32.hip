@@ -104,6 +104,12 @@ __device__ __forceinline__ void big_places(unsigned S, unsigned lane, const Rep3
         cpos[j] = big_chunk(((j / RC) << (8 + K - D)) | (S * (256u >> D) + 64u * (j % RC) + lane), T);
 }
 
+// first float of the wave's part of a row; ld 0: one row read for every batch row
+template <int K, int D>
+__device__ __forceinline__ long long big_off(long long row, long long ld, unsigned S) {
+    return ((row & row_mask(ld)) << (kBigBase + K - D)) + S * (1024u >> D);
+}
+
 // the wave's 1024 >> D floats of its row
 template <int D, bool NT>
 __device__ __forceinline__ BigRow big_fetch(const float* __restrict__ src, int lane) {
@@ -273,7 +279,8 @@ __device__ __forceinline__ BigLane big_lane(unsigned lane, const Rep32Table& T) 
 
 template <int K, int D, bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep32_fwd_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, long long batch, Rep32Table T) {
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb, float* __restrict__ C,
+    long long batch, Rep32Table T) {
     constexpr unsigned NS = 1u << K;  // base rows per row
     constexpr int kRows = 4 >> K;     // rows per workgroup
     __shared__ __attribute__((aligned(4096))) float lds[2][4 * 1024];
@@ -292,8 +299,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         long long row = row0 + (wave >> K);
         const bool live = row < batch;  // rows past the end recompute the last row and are not stored
         row = live ? row : batch - 1;
-        const long long off = (row << (kBigBase + K - D)) + S * (1024u >> D);
-        const BigRow va = big_fetch<D, NT>(A + off, lane), vb = big_fetch<D, NT>(B + off, lane);
+        const long long off = big_off<K, D>(row, 1, S);
+        const BigRow va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
+        const BigRow vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
         big_stage(ra, va, cpos);
         big_stage(rb, vb, cpos);
         big_sync<K>();
@@ -328,8 +336,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
 
 template <int K, int D, bool NT, bool WA, bool WB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rep32_bwd_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, long long ldg,
-    float* __restrict__ GA, float* __restrict__ GB, long long batch, Rep32Table T) {
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
+    const float* __restrict__ GC, long long ldg, float* __restrict__ GA, float* __restrict__ GB, long long batch,
+    Rep32Table T) {
     constexpr unsigned NS = 1u << K;
     constexpr int kRows = 4 >> K;
     __shared__ __attribute__((aligned(4096))) float lds[3][4 * 1024];
@@ -350,11 +359,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
         long long row = row0 + (wave >> K);
         const bool live = row < batch;
         row = live ? row : batch - 1;
-        const long long off = (row << (kBigBase + K - D)) + S * (1024u >> D);
-        const BigRow vg = big_fetch<D, NT>(GC + ((row & row_mask(ldg)) << (kBigBase + K - D)) + S * (1024u >> D), lane);
+        const long long off = big_off<K, D>(row, 1, S);
+        const BigRow vg = big_fetch<D, NT>(GC + big_off<K, D>(row, ldg, S), lane);
         BigRow va, vb;
-        if (WA) vb = big_fetch<D, NT>(B + off, lane);
-        if (WB) va = big_fetch<D, NT>(A + off, lane);
+        if (WA) vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
+        if (WB) va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
         big_stage(r0, vg, cpos);
         if (WA) big_stage(r1, vb, cpos);
         if (WB) big_stage(r2, va, cpos);
@@ -707,22 +716,26 @@ int64_t rep32_rows(int n, uint32_t neg, uint32_t nul) {
     }
 
 template <int K, int D>
-static void launch_rep32_fwd(dim3 grid, hipStream_t s, bool nt, const float* a, const float* b, float* c,
-                             int64_t batch, const Rep32Table& T) {
+static void launch_rep32_fwd(dim3 grid, hipStream_t s, bool nt, const float* a, int64_t lda, const float* b,
+                             int64_t ldb, float* c, int64_t batch, const Rep32Table& T) {
     const dim3 block(256);
-    if (nt) hipLaunchKernelGGL((rep32_fwd_kernel<K, D, true>), grid, block, 0, s, a, b, c, (long long)batch, T);
-    else hipLaunchKernelGGL((rep32_fwd_kernel<K, D, false>), grid, block, 0, s, a, b, c, (long long)batch, T);
+    if (nt)
+        hipLaunchKernelGGL((rep32_fwd_kernel<K, D, true>), grid, block, 0, s, a, (long long)lda, b, (long long)ldb, c,
+                           (long long)batch, T);
+    else
+        hipLaunchKernelGGL((rep32_fwd_kernel<K, D, false>), grid, block, 0, s, a, (long long)lda, b, (long long)ldb, c,
+                           (long long)batch, T);
 }
 
-int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, float* out, int64_t batch,
-              void* stream) {
+int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* out,
+              int64_t batch, void* stream) {
     BigSplit c;
     Rep32Table T;
     if (!big_split(n, neg, nul, c) || !big_table(n, neg, nul, c, T))
         return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
     const bool nt = stream_nt(3.0 * 4.0 * (double)(1LL << n) * (double)batch);
 #define CLF_BIG_FWD(K, D) \
-    launch_rep32_fwd<K, D>(dim3(big_grid(c.k, batch)), (hipStream_t)stream, nt, a, b, out, batch, T)
+    launch_rep32_fwd<K, D>(dim3(big_grid(c.k, batch)), (hipStream_t)stream, nt, a, lda, b, ldb, out, batch, T)
     CLF_BIG_SWITCH(CLF_BIG_FWD)
 #undef CLF_BIG_FWD
     CLF_HIP_CHECK(hipGetLastError());
@@ -730,22 +743,20 @@ int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b,
 }
 
 template <int K, int D, bool NT>
-static void launch_rep32_bwd(dim3 grid, hipStream_t s, const float* a, const float* b, const float* gc, int64_t ldg,
-                             float* ga, float* gb, int64_t batch, const Rep32Table& T) {
-    const dim3 block(256);
-    if (ga && gb)
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, true, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
-                           gb, (long long)batch, T);
-    else if (ga)
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, true, false>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
-                           gb, (long long)batch, T);
-    else
-        hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, false, true>), grid, block, 0, s, a, b, gc, (long long)ldg, ga,
-                           gb, (long long)batch, T);
+static void launch_rep32_bwd(dim3 grid, hipStream_t s, const float* a, int64_t lda, const float* b, int64_t ldb,
+                             const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch,
+                             const Rep32Table& T) {
+#define CLF_BIG_BWD_W(WA, WB)                                                                                     \
+    hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, WA, WB>), grid, dim3(256), 0, s, a, (long long)lda, b,          \
+                       (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
+    if (ga && gb) CLF_BIG_BWD_W(true, true);
+    else if (ga) CLF_BIG_BWD_W(true, false);
+    else CLF_BIG_BWD_W(false, true);
+#undef CLF_BIG_BWD_W
 }
 
-int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg,
-              float* ga, float* gb, int64_t batch, void* stream) {
+int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
+              const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
     BigSplit c;
     Rep32Table T;
     if (!big_split(n, neg, nul, c) || !big_table(n, neg, nul, c, T))
@@ -753,10 +764,10 @@ int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, const float* b,
     hipStream_t s = (hipStream_t)stream;
     const dim3 grid(big_grid(c.k, batch));
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 4.0 * (double)(1LL << n) * (double)batch);
-#define CLF_BIG_BWD(K, D)                                                                \
-    do {                                                                                 \
-        if (nt) launch_rep32_bwd<K, D, true>(grid, s, a, b, gc, ldg, ga, gb, batch, T);  \
-        else launch_rep32_bwd<K, D, false>(grid, s, a, b, gc, ldg, ga, gb, batch, T);    \
+#define CLF_BIG_BWD(K, D)                                                                          \
+    do {                                                                                           \
+        if (nt) launch_rep32_bwd<K, D, true>(grid, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);  \
+        else launch_rep32_bwd<K, D, false>(grid, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);    \
     } while (0)
     CLF_BIG_SWITCH(CLF_BIG_BWD)
 #undef CLF_BIG_BWD

@@ -255,7 +255,8 @@ __device__ __forceinline__ void product_q7(float* __restrict__ rel, const float 
 // ONE: the grid covers the batch (one group per wave), so no next group is
 // prefetched (the same in the backward)
 template <bool PAIR, bool NT, bool ONE>
-__global__ __launch_bounds__(256) void rep7_fwd_kernel(const float* __restrict__ A, const float* __restrict__ B,
+__global__ __launch_bounds__(256) void rep7_fwd_kernel(
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
                                                         float* __restrict__ C, long long batch, Rep7Table T) {
     constexpr int D = PAIR ? 2 : 3;
     // per wave: staged a | b, later the relayout (over both), then c in the b
@@ -275,8 +276,8 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(const float* __restrict__
     const long long stride = (long long)gridDim.x * 16;
     const long long rfirst = ((long long)blockIdx.x * 4 + wave) * 4;
     long long row0 = rfirst;
-    Pre7 pa = fetch7<NT>(A, row0, batch, lane);
-    Pre7 pb = fetch7<NT>(B, row0, batch, lane);
+    Pre7 pa = fetch7<NT>(A, row0, batch, lane, lda);
+    Pre7 pb = fetch7<NT>(B, row0, batch, lane, ldb);
     for (; row0 < batch; row0 += stride) {
         stage7(sa, pa, lane, oddc);
         if (row0 != rfirst) {  // uniform: the previous group's c leaves the b slot first
@@ -286,8 +287,8 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(const float* __restrict__
         }
         stage7(sb, pb, lane, oddc);
         if (!ONE) {
-            pa = fetch7<NT>(A, row0 + stride, batch, lane);
-            pb = fetch7<NT>(B, row0 + stride, batch, lane);
+            pa = fetch7<NT>(A, row0 + stride, batch, lane, lda);
+            pb = fetch7<NT>(B, row0 + stride, batch, lane, ldb);
         }
         wave_lds_sync();
         if constexpr (PAIR) {
@@ -320,7 +321,8 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(const float* __restrict__
 // slot, so few converted operands are live at once.
 template <bool PAIR, bool NT, bool WA, bool WB, bool ONE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep7_bwd_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, long long ldg,
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
+    const float* __restrict__ GC, long long ldg,
     float* __restrict__ GA, float* __restrict__ GB, long long batch, Rep7Table T) {
     constexpr int D = PAIR ? 2 : 3;
     constexpr int L = 1 << D;
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
     const long long stride = (long long)gridDim.x * 16;
     const long long rfirst = ((long long)blockIdx.x * 4 + wave) * 4;
     long long row0 = rfirst;
-    Pre7 pb = fetch7<NT>(B, row0, batch, lane);
+    Pre7 pb = fetch7<NT>(B, row0, batch, lane, ldb);
     Pre7 pg = fetch7<NT>(GC, row0, batch, lane, ldg);
     for (; row0 < batch; row0 += stride) {
         // the table values are re-derived where they are used rather than kept
@@ -348,7 +350,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         for (int k = 0; k < 8; ++k) asm volatile("" : "+v"(ent[k]));
         stage7(sg, pg, lane, oddc);
         stage7(sx, pb, lane, oddc);
-        const Pre7 pa = fetch7<NT>(A, row0, batch, lane);
+        const Pre7 pa = fetch7<NT>(A, row0, batch, lane, lda);
         // the previous group's gb leaves the scratch slot (stored after this wait)
         if (WB && row0 != rfirst) store7<NT>(GB, sr, row0 - stride, batch, lane, oddc);  // uniform
         wave_lds_sync();
@@ -373,7 +375,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         stage7(sx, pa, lane, oddc);
         if (!ONE) {
             pg = fetch7<NT>(GC, row0 + stride, batch, lane, ldg);
-            pb = fetch7<NT>(B, row0 + stride, batch, lane);
+            pb = fetch7<NT>(B, row0 + stride, batch, lane, ldb);
         }
         if (WA) store7<NT>(GA, sr, row0, batch, lane, oddc);  // after this group's second wait
         wave_lds_sync();
@@ -566,7 +568,8 @@ static unsigned rep7_grid(int64_t batch) {
     return (unsigned)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
-int rep7_fwd(uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream) {
+int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
+             void* stream) {
     Rep7Table T;
     if (!rep7_table(neg & 0x7fu, T)) return set_error(CLF_ERR_UNSUPPORTED, "no n = 7 matrix representation found");
     const bool pair = (host_popc(neg & 0x7fu) & 1) != 0;
@@ -574,10 +577,13 @@ int rep7_fwd(uint32_t neg, const float* a, const float* b, float* c, int64_t bat
     const dim3 g(rep7_grid(batch));
     const bool one = (long long)g.x * 16 >= batch;
     const bool nt = stream_nt(3.0 * 512.0 * (double)batch);
-#define CLF_REP7_FWD(P, NT)                                                                                        \
-    do {                                                                                                          \
-        if (one) hipLaunchKernelGGL((rep7_fwd_kernel<P, NT, true>), g, dim3(256), 0, s, a, b, c, (long long)batch, T); \
-        else hipLaunchKernelGGL((rep7_fwd_kernel<P, NT, false>), g, dim3(256), 0, s, a, b, c, (long long)batch, T); \
+#define CLF_REP7_FWD_ONE(P, NT, ONE)                                                                             \
+    hipLaunchKernelGGL((rep7_fwd_kernel<P, NT, ONE>), g, dim3(256), 0, s, a, (long long)lda, b, (long long)ldb, c, \
+                       (long long)batch, T)
+#define CLF_REP7_FWD(P, NT)                     \
+    do {                                        \
+        if (one) CLF_REP7_FWD_ONE(P, NT, true); \
+        else CLF_REP7_FWD_ONE(P, NT, false);    \
     } while (0)
     if (pair) {
         if (nt) CLF_REP7_FWD(true, true);
@@ -587,12 +593,13 @@ int rep7_fwd(uint32_t neg, const float* a, const float* b, float* c, int64_t bat
         else CLF_REP7_FWD(false, false);
     }
 #undef CLF_REP7_FWD
+#undef CLF_REP7_FWD_ONE
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
 
-int rep7_bwd(uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga, float* gb,
-             int64_t batch, void* stream) {
+int rep7_bwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc, int64_t ldg,
+             float* ga, float* gb, int64_t batch, void* stream) {
     Rep7Table T;
     if (!rep7_table(neg & 0x7fu, T)) return set_error(CLF_ERR_UNSUPPORTED, "no n = 7 matrix representation found");
     const bool pair = (host_popc(neg & 0x7fu) & 1) != 0;
@@ -601,14 +608,13 @@ int rep7_bwd(uint32_t neg, const float* a, const float* b, const float* gc, int6
     const bool one = (long long)g.x * 16 >= batch;
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 512.0 * (double)batch);
     if (!ga && !gb) return CLF_OK;
-#define CLF_REP7_BWD(P, NT, WA, WB)                                                                        \
-    do {                                                                                                  \
-        if (one)                                                                                          \
-            hipLaunchKernelGGL((rep7_bwd_kernel<P, NT, WA, WB, true>), g, dim3(256), 0, s, a, b, gc,       \
-                               (long long)ldg, ga, gb, (long long)batch, T);                              \
-        else                                                                                              \
-            hipLaunchKernelGGL((rep7_bwd_kernel<P, NT, WA, WB, false>), g, dim3(256), 0, s, a, b, gc,      \
-                               (long long)ldg, ga, gb, (long long)batch, T);                              \
+#define CLF_REP7_BWD_ONE(P, NT, WA, WB, ONE)                                                                  \
+    hipLaunchKernelGGL((rep7_bwd_kernel<P, NT, WA, WB, ONE>), g, dim3(256), 0, s, a, (long long)lda, b,        \
+                       (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
+#define CLF_REP7_BWD(P, NT, WA, WB)                     \
+    do {                                                \
+        if (one) CLF_REP7_BWD_ONE(P, NT, WA, WB, true); \
+        else CLF_REP7_BWD_ONE(P, NT, WA, WB, false);    \
     } while (0)
 #define CLF_REP7_BWD_W(P, NT)                 \
     do {                                      \
@@ -625,6 +631,7 @@ int rep7_bwd(uint32_t neg, const float* a, const float* b, const float* gc, int6
     }
 #undef CLF_REP7_BWD_W
 #undef CLF_REP7_BWD
+#undef CLF_REP7_BWD_ONE
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }

@@ -115,7 +115,8 @@ __device__ __forceinline__ void twist_unconvert(const float (&w)[16], float rho,
 
 template <bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void twist16_fwd_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, float* __restrict__ C, long long batch, TwistTable T) {
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb, float* __restrict__ C,
+    long long batch, TwistTable T) {
     __shared__ float lds[4][2 * 4 * 256];  // staged a | staged b; the relayout over a and the start of b, then c over b
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const unsigned x = lane & 15u;
@@ -129,8 +130,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
     for (int z = 0; z < 16; ++z) ent[z] = T.rep.e[x * 16 + z] ^ oddx;
     const long long stride = (long long)gridDim.x * 16;
     for (long long row0 = ((long long)blockIdx.x * 4 + wave) * 4; row0 < batch; row0 += stride) {
-        const Pre16 pa = fetch16<NT>(A, row0, batch, lane);
-        const Pre16 pb = fetch16<NT>(B, row0, batch, lane);
+        const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
+        const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
 #pragma unroll
         for (int z = 0; z < 16; ++z) asm volatile("" : "+v"(ent[z]));  // addresses re-derived where they are used
         stage16(sa, pa, lane, oddc);
@@ -154,8 +155,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
 
 template <bool NT, bool WA, bool WB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void twist16_bwd_kernel(
-    const float* __restrict__ A, const float* __restrict__ B, const float* __restrict__ GC, long long ldg,
-    float* __restrict__ GA, float* __restrict__ GB, long long batch, TwistTable T) {
+    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
+    const float* __restrict__ GC, long long ldg, float* __restrict__ GA, float* __restrict__ GB, long long batch,
+    TwistTable T) {
     __shared__ float lds[4][2 * 4 * 256 + kRelayoutFloats];  // gc | b, then a | relayout and rows of each gradient
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const unsigned x = lane & 15u;
@@ -171,12 +173,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     const long long stride = (long long)gridDim.x * 16;
     for (long long row0 = ((long long)blockIdx.x * 4 + wave) * 4; row0 < batch; row0 += stride) {
         const Pre16 pg = fetch16<NT>(GC, row0, batch, lane, ldg);
-        const Pre16 pb = fetch16<NT>(B, row0, batch, lane);
+        const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
 #pragma unroll
         for (int z = 0; z < 16; ++z) asm volatile("" : "+v"(ent[z]));
         stage16(s0, pg, lane, oddc);
         if (WA) stage16(s1, pb, lane, oddc);
-        const Pre16 pa = fetch16<NT>(A, row0, batch, lane);
+        const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
         wave_lds_sync();
         if (WA) {
             const Parts g = twist_convert<0>(s0 + rb * 256, ent);
@@ -331,39 +333,40 @@ static dim3 twist_grid(int64_t batch) {
     return dim3((unsigned)(g < (1LL << 24) ? g : (1LL << 24)));
 }
 
-int twist_fwd(uint32_t neg, uint32_t nul, const float* a, const float* b, float* c, int64_t batch, void* stream) {
+int twist_fwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
+              int64_t batch, void* stream) {
     TwistTable T;
     if (!twist_table(neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature is not one generator from M_16(R)");
     hipStream_t s = (hipStream_t)stream;
     if (stream_nt(3.0 * 1024.0 * (double)batch))
-        hipLaunchKernelGGL((twist16_fwd_kernel<true>), twist_grid(batch), dim3(256), 0, s, a, b, c, (long long)batch,
-                           T);
+        hipLaunchKernelGGL((twist16_fwd_kernel<true>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b,
+                           (long long)ldb, c, (long long)batch, T);
     else
-        hipLaunchKernelGGL((twist16_fwd_kernel<false>), twist_grid(batch), dim3(256), 0, s, a, b, c, (long long)batch,
-                           T);
+        hipLaunchKernelGGL((twist16_fwd_kernel<false>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b,
+                           (long long)ldb, c, (long long)batch, T);
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
 
-int twist_bwd(uint32_t neg, uint32_t nul, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
-              float* gb, int64_t batch, void* stream) {
+int twist_bwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc,
+              int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
     TwistTable T;
     if (!twist_table(neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature is not one generator from M_16(R)");
     hipStream_t s = (hipStream_t)stream;
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 1024.0 * (double)batch);
-#define CLF_TWIST_BWD(WA, WB)                                                                                    \
-    do {                                                                                                         \
-        if (nt)                                                                                                  \
-            hipLaunchKernelGGL((twist16_bwd_kernel<true, WA, WB>), twist_grid(batch), dim3(256), 0, s, a, b, gc,  \
-                               (long long)ldg, ga, gb, (long long)batch, T);                                     \
-        else                                                                                                     \
-            hipLaunchKernelGGL((twist16_bwd_kernel<false, WA, WB>), twist_grid(batch), dim3(256), 0, s, a, b, gc, \
-                               (long long)ldg, ga, gb, (long long)batch, T);                                     \
+#define CLF_TWIST_BWD2(NT, WA, WB)                                                                               \
+    hipLaunchKernelGGL((twist16_bwd_kernel<NT, WA, WB>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b, \
+                       (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
+#define CLF_TWIST_BWD(WA, WB)                \
+    do {                                     \
+        if (nt) CLF_TWIST_BWD2(true, WA, WB);  \
+        else CLF_TWIST_BWD2(false, WA, WB);    \
     } while (0)
     if (ga && gb) CLF_TWIST_BWD(true, true);
     else if (ga) CLF_TWIST_BWD(true, false);
     else if (gb) CLF_TWIST_BWD(false, true);
 #undef CLF_TWIST_BWD
+#undef CLF_TWIST_BWD2
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }

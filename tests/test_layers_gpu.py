@@ -181,3 +181,43 @@ def test_layer_small_batches():
             ref = O.layer_forward("geom", x.detach().double().cpu(), layer.weight.detach().double().cpu())
             assert rel_err(y, ref) <= TOL
         layer.weight.grad = None
+
+
+@pytest.mark.parametrize("op,metric,rows", [
+    ("geom", (1,) * 7, 1), ("inner", (1,) * 7, 63489), ("regressive", (1,) * 7, 17), ("lc", (-1,) * 4 + (1, 1, 0), 33),
+    ("geom", (1,) * 7 + (-1,), 31745), ("wedge", (1,) * 8, 2049), ("inner", (1,) * 5 + (0, -1, 1), 300),
+    ("geom", (1,) * 9, 9), ("geom", (1,) * 8 + (-1,), 15873), ("inner", (1,) * 9, 15872), ("rc", (1,) * 9, 5),
+    ("geom", (1,) * 9 + (0,), 65), ("geom", (1,) * 8 + (-1, 1), 7936), ("lc", (1,) * 9 + (0,), 7937),
+    ("wedge", (-1,) * 10, 3)])
+@pytest.mark.parametrize("side", [0, 1])
+def test_rows_path_edges(op, metric, rows, side):
+    """The layers on the per-row kernels, at remainders of their row groups and
+    one row below, at and above a chunk of weight gradients (31 MiB of rows):
+    values and input gradient equal the per-row product's on the expanded
+    weight, the weight gradient its fp64 column sums; one gradient at a time
+    gives the same as both. TOL is normwise: sums of at most 1024 terms a row
+    and 32 x 2 rows a partial stay below 1e-6."""
+    D = 1 << len(metric)
+    g = torch.Generator(device="cuda").manual_seed(rows + side)
+    x, gy = (torch.randn(rows, D, device="cuda", generator=g) for _ in range(2))
+    w = torch.randn(1, D, device="cuda", generator=g)
+    print(f"[case] rows path op={op} metric={metric} rows={rows} side={side}", flush=True)
+    x1, w1 = x.clone().requires_grad_(), w.clone().requires_grad_()
+    y = bcast.bcast_product(op, x1, w1, metric, side=side)
+    gx, gw = torch.autograd.grad(y, (x1, w1), gy)
+    x2, w2 = x.clone().requires_grad_(), w.expand(rows, D).contiguous().requires_grad_()
+    fn = {"geom": cc.geom_prod, "wedge": cc.wedge_prod, "inner": cc.inner_prod, "lc": cc.left_contraction,
+          "rc": cc.right_contraction, "regressive": cc.regressive_prod}[op]
+    y2 = fn(x2, w2, metric) if side == 0 else fn(w2, x2, metric)
+    gx2, gw2 = torch.autograd.grad(y2, (x2, w2), gy)
+    assert rel_err(y, y2) <= TOL
+    assert rel_err(gx, gx2) <= TOL
+    assert rel_err(gw, gw2.double().sum(0, keepdim=True)) <= TOL
+    y3 = bcast.bcast_product(op, x, w1, metric, side=side)
+    assert torch.equal(torch.autograd.grad(y3, w1, gy)[0], gw)
+    y4 = bcast.bcast_product(op, x1, w, metric, side=side)
+    assert rel_err(torch.autograd.grad(y4, x1, gy)[0], gx) <= TOL
+    g0 = torch.autograd.grad(bcast.bcast_product(op, x1, w1, metric, side=side).sum(), (x1, w1))
+    r0 = torch.autograd.grad(fn(x2, w2, metric).sum() if side == 0 else fn(w2, x2, metric).sum(), (x2, w2))
+    assert rel_err(g0[0], r0[0]) <= TOL
+    assert rel_err(g0[1], r0[1].double().sum(0, keepdim=True)) <= TOL
