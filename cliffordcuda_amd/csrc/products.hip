@@ -391,8 +391,129 @@ struct BlkParams {
     int wpr_log;    // small-batch kernels: log2 of the workgroups per row
     unsigned rskew; // blocked kernels: 2-bit slot skew of staged row r at bits 2 (r & 15)
     unsigned negl;  // metric mask, bits 0-3 (the regressive product's dual signs)
+    unsigned null;  // null mask, bits 0-3 (mixed low metrics)
     bool bca, bcb;  // a / b is one row read for every batch row (not on the whole-row, tiled and generic kernels)
 };
+
+// ---- mixed low metrics ----
+// Low generators of different squares: a term's low sign is the Euclidean one
+// times m(il & jl), m(e) = the product of the squares over e's bits, a kernel
+// argument that the compile-time patterns cannot hold. A contraction's common
+// part is its smaller index, so m goes onto that operand (or that output) once
+// per index, and an index with m = 0 is passed over by a scalar branch. The
+// geometric product takes the 16 dressings m(e & .) of one operand from each
+// other, generator by generator: 120 multiplies beside the 256 FMAs.
+// Against a thread per coefficient with the sign computed for each of its 2^n
+// terms (us, forward + backward, inner): n = 4, 60000 rows 22 + 39 -> 7 + 8;
+// n = 5 71 + 125 -> 8 + 13; n = 6 263 + 475 -> 15 + 31; n = 7, 15000 rows 268 +
+// 475 -> 12 + 25; n = 8, 60013 rows 3894 + 7060 -> 117 + 261; n = 12, 2 rows
+// 1057 + 2242 -> 711 + 1293, so they take every batch that fits their LDS. Bound
+// by the lanes of a wave whose partner blocks the op drops (a quarter to a half
+// of the steps), from n = 7 on; below that by memory.
+enum { LOW_POS = 0, LOW_NEG = 1, LOW_MIX = 2 };
+
+struct LowMetric {
+    float m[16];
+};
+
+__device__ __forceinline__ LowMetric low_metric(const BlkParams& P) {
+    LowMetric lo;
+#pragma unroll
+    for (unsigned e = 0; e < 16u; ++e)
+        lo.m[e] = (e & P.null) ? 0.f : (__popc(e & P.negl) & 1) ? -1.f : 1.f;
+    return lo;
+}
+
+template <class F, int... E>
+__device__ __forceinline__ void each_of(std::integer_sequence<int, E...>, F&& f) {
+    (f(std::integral_constant<int, E>{}), ...);
+}
+template <class F>
+__device__ __forceinline__ void each16(F&& f) {
+    each_of(std::make_integer_sequence<int, 16>{}, f);
+}
+
+// The contraction VAR (LV_LC: il inside jl, LV_RC: jl inside il; STRICT: not
+// equal) with e the smaller index and f the larger. MODE 0: acc[e ^ f] += s m(e)
+// u[e] v[f] (u the smaller index's operand, v the larger's); 1, the gradient of
+// the smaller: acc[e] += m(e) sum s u[f] v[e ^ f]; 2, of the larger: acc[f] +=
+// s m(e) u[e] v[e ^ f] (v the upstream gradient).
+template <int VAR, int MODE, bool STRICT = false>
+__device__ __forceinline__ void mix_contr(float (&acc)[16], const float (&u)[16], const float (&v)[16],
+                                          const LowMetric& lo) {
+    each16([&](auto ec) __attribute__((always_inline)) {
+        constexpr int E = decltype(ec)::value;
+        const float m = lo.m[E];
+        if (m == 0.f) return;  // uniform
+        const float x = MODE == 1 ? 0.f : m * u[E];
+        float t = 0.f;
+        each16([&](auto fc) __attribute__((always_inline)) {
+            constexpr int F = decltype(fc)::value;
+            if constexpr ((E & ~F) == 0 && !(STRICT && E == F)) {
+                constexpr int s = VAR == LV_LC ? low_sign(VAR, false, (unsigned)E, (unsigned)F) : low_sign(VAR, false, (unsigned)F, (unsigned)E);
+                if constexpr (MODE == 0) acc[E ^ F] = __builtin_fmaf(s > 0 ? x : -x, v[F], acc[E ^ F]);
+                else if constexpr (MODE == 1) t = __builtin_fmaf(s > 0 ? u[F] : -u[F], v[E ^ F], t);
+                else acc[F] = __builtin_fmaf(s > 0 ? x : -x, v[E ^ F], acc[F]);
+            }
+        });
+        if constexpr (MODE == 1) acc[E] = __builtin_fmaf(m, t, acc[E]);
+    });
+}
+
+// The geometric product; d: the operand that is dressed, on the way to index E
+// with generators below K done. MODE 0: acc[il ^ jl] += s v[il] d[jl]; 1:
+// acc[il] += s d[jl] v[il ^ jl]; 2: acc[jl] += s d[il] v[il ^ jl].
+template <int MODE, int K = 0, int E = 0>
+__device__ __forceinline__ void mix_geom(float (&acc)[16], const float (&d)[16], const float (&v)[16],
+                                         const LowMetric& lo) {
+    if constexpr (K == 4) {
+        each16([&](auto fc) __attribute__((always_inline)) {
+            constexpr int F = decltype(fc)::value;
+            constexpr int s = MODE == 2 ? low_sign(LV_GEOM, false, (unsigned)F, (unsigned)E) : low_sign(LV_GEOM, false, (unsigned)E, (unsigned)F);
+            if constexpr (MODE == 0) acc[E ^ F] = __builtin_fmaf(s > 0 ? v[E] : -v[E], d[F], acc[E ^ F]);
+            else acc[E] = __builtin_fmaf(s > 0 ? d[F] : -d[F], v[E ^ F], acc[E]);
+        });
+    } else {
+        mix_geom<MODE, K + 1, E>(acc, d, v, lo);
+        float w[16];
+        const float m = lo.m[1 << K];
+        each16([&](auto fc) __attribute__((always_inline)) {
+            constexpr int F = decltype(fc)::value;
+            w[F] = (F >> K) & 1 ? m * d[F] : d[F];
+        });
+        mix_geom<MODE, K + 1, E | (1 << K)>(acc, w, v, lo);
+    }
+}
+
+template <int OP>
+__device__ __forceinline__ void mix_fwd(float (&acc)[16], const float (&a)[16], const float (&b)[16], unsigned ih,
+                                        unsigned jh, const LowMetric& lo) {
+    if constexpr (OP == OP_GEOM) mix_geom<0>(acc, b, a, lo);
+    else if constexpr (OP == OP_LC) mix_contr<LV_LC, 0>(acc, a, b, lo);
+    else if constexpr (OP == OP_RC) mix_contr<LV_RC, 0>(acc, b, a, lo);
+    else {
+        const bool l = (ih & ~jh) == 0u, r = (jh & ~ih) == 0u;
+        if (l) mix_contr<LV_LC, 0>(acc, a, b, lo);
+        if (l && r) mix_contr<LV_RC, 0, true>(acc, b, a, lo);
+        else if (r) mix_contr<LV_RC, 0>(acc, b, a, lo);
+    }
+}
+
+template <int OP>
+__device__ __forceinline__ void mix_ga(float (&acc)[16], const float (&b)[16], const float (&g)[16],
+                                       const LowMetric& lo) {
+    if constexpr (OP == OP_GEOM) mix_geom<1>(acc, b, g, lo);
+    else if constexpr (OP == OP_LC) mix_contr<LV_LC, 1>(acc, b, g, lo);
+    else mix_contr<LV_RC, 2>(acc, b, g, lo);
+}
+
+template <int OP>
+__device__ __forceinline__ void mix_gb(float (&acc)[16], const float (&a)[16], const float (&g)[16],
+                                       const LowMetric& lo) {
+    if constexpr (OP == OP_GEOM) mix_geom<2>(acc, a, g, lo);
+    else if constexpr (OP == OP_LC) mix_contr<LV_LC, 2>(acc, a, g, lo);
+    else mix_contr<LV_RC, 1>(acc, a, g, lo);
+}
 
 // Stage NOPS (2 or 3) row-major operands s0, s1[, s2] for the workgroup's rows
 // into LDS (swizzled). Each thread issues all its loads (up to four float4 per
@@ -442,7 +563,7 @@ __device__ __forceinline__ void stage_rows(float4* __restrict__ lds, const float
     }
 }
 
-template <int OP, bool LOWNEG>
+template <int OP, int LOW>
 __global__ __launch_bounds__(256) void prod_fwd_blk(const float* __restrict__ A, const float* __restrict__ B,
                                                      float* __restrict__ C, BlkParams P) {
     extern __shared__ float4 lds[];
@@ -463,6 +584,7 @@ __global__ __launch_bounds__(256) void prod_fwd_blk(const float* __restrict__ A,
     float4* out = reinterpret_cast<float4*>(C) + ((row0 + r) << (n - 2));
     const unsigned fullh = NB - 1u;
 
+    const LowMetric lo = low_metric(P);
     for (int kk = 0; kk < P.kpl; ++kk) {
         const unsigned kh = lane_blk + ((unsigned)kk << P.lpr_log);
         float acc[16];
@@ -476,7 +598,8 @@ __global__ __launch_bounds__(256) void prod_fwd_blk(const float* __restrict__ A,
             load_blk_s(la, ih, bslot(ih, t), av);
             load_blk_s(lb, jh, bslot(jh, t), bv);
             apply_flips(bv, hs.mask, hs.mask ^ (cross_pi<OP>(ih, P.nm1) << 31));
-            fwd_block_dispatch<OP, LOWNEG>(acc, av, bv, ih, jh);
+            if constexpr (LOW == LOW_MIX) mix_fwd<OP>(acc, av, bv, ih, jh, lo);
+            else fwd_block_dispatch<OP, LOW == LOW_NEG>(acc, av, bv, ih, jh);
         }
         if (OP == OP_REGR) {
             const unsigned ob = fullh ^ kh;
@@ -498,11 +621,11 @@ __global__ __launch_bounds__(256) void prod_fwd_blk(const float* __restrict__ A,
 // subsets (the other way round), then m = h (both patterns). A lane whose
 // class has fewer partners than another lane's idles for the difference; the
 // wave stops a class when no lane has partners left.
-template <int CLASS, bool LOWNEG>
+template <int CLASS, int LOW>
 __device__ __forceinline__ void inner_pair(const float4* __restrict__ la, const float4* __restrict__ lb,
                                            const float4* __restrict__ lg, unsigned h, unsigned m, unsigned fullh,
                                            bool do_a, bool do_b, float (&ga)[16], float (&gb)[16],
-                                           const BlkParams& P, unsigned t) {
+                                           const BlkParams& P, unsigned t, const LowMetric& lo) {
     // CLASS 0: m strict superset of h; 1: strict subset; 2: m = h
     constexpr int VA = CLASS == 0 ? LV_LC : CLASS == 1 ? LV_RC : LV_INNER;
     constexpr int VB = CLASS == 0 ? LV_RC : CLASS == 1 ? LV_LC : LV_INNER;
@@ -517,7 +640,12 @@ __device__ __forceinline__ void inner_pair(const float4* __restrict__ la, const 
         float bv[16];
         load_blk_s(lb, m, bslot(m, t), bv);
         apply_flips(bv, sa.mask, sa.mask ^ (cross_pi<OP_INNER>(h, P.nm1) << 31));
-        lowblock_ga<VA, LOWNEG>(ga, bv, g);
+        if constexpr (LOW != LOW_MIX) {
+            lowblock_ga<VA, LOW == LOW_NEG>(ga, bv, g);
+        } else {
+            if constexpr (CLASS != 1) mix_contr<LV_LC, 1>(ga, bv, g, lo);
+            if constexpr (CLASS != 0) mix_contr<LV_RC, 2, CLASS == 2>(ga, bv, g, lo);
+        }
     }
     if (do_b) {
         const unsigned pm = cross_pi<OP_INNER>(m, P.nm1) << 31;
@@ -526,34 +654,39 @@ __device__ __forceinline__ void inner_pair(const float4* __restrict__ la, const 
         apply_flips(av, sb.mask, sb.mask ^ pm);
 #pragma unroll
         for (int e = 0; e < 16; ++e) gt[e] = (cpopc((unsigned)e) & 1) ? flip(g[e], pm) : g[e];
-        lowblock_gb<VB, LOWNEG>(gb, av, gt);
+        if constexpr (LOW != LOW_MIX) {
+            lowblock_gb<VB, LOW == LOW_NEG>(gb, av, gt);
+        } else {
+            if constexpr (CLASS != 0) mix_contr<LV_LC, 2>(gb, av, gt, lo);
+            if constexpr (CLASS != 1) mix_contr<LV_RC, 1, CLASS == 2>(gb, av, gt, lo);
+        }
     }
 }
 
-template <bool LOWNEG>
+template <int LOW>
 __device__ __forceinline__ void inner_bwd_blocks(const float4* __restrict__ la, const float4* __restrict__ lb,
                                                  const float4* __restrict__ lg, unsigned h, unsigned fullh,
                                                  bool want_a, bool want_b, float (&ga)[16], float (&gb)[16],
-                                                 const BlkParams& P, unsigned t) {
+                                                 const BlkParams& P, unsigned t, const LowMetric& lo) {
     const unsigned co = fullh & ~h;
     // strict supersets m = h | S, S a nonempty subset of co, in increasing order
     const int nsup = (1 << __popc(co)) - 1;
     unsigned S = 0u;
     for (int k = 0; __any(k < nsup); ++k) {
         S = (S - co) & co;
-        inner_pair<0, LOWNEG>(la, lb, lg, h, h | S, fullh, want_a && k < nsup, want_b && k < nsup, ga, gb, P, t);
+        inner_pair<0, LOW>(la, lb, lg, h, h | S, fullh, want_a && k < nsup, want_b && k < nsup, ga, gb, P, t, lo);
     }
     // strict subsets m of h (the empty set first)
     const int nsub = (1 << __popc(h)) - 1;
     unsigned T = 0u;
     for (int k = 0; __any(k < nsub); ++k) {
-        inner_pair<1, LOWNEG>(la, lb, lg, h, T, fullh, want_a && k < nsub, want_b && k < nsub, ga, gb, P, t);
+        inner_pair<1, LOW>(la, lb, lg, h, T, fullh, want_a && k < nsub, want_b && k < nsub, ga, gb, P, t, lo);
         T = (T - h) & h;
     }
-    inner_pair<2, LOWNEG>(la, lb, lg, h, h, fullh, want_a, want_b, ga, gb, P, t);
+    inner_pair<2, LOW>(la, lb, lg, h, h, fullh, want_a, want_b, ga, gb, P, t, lo);
 }
 
-template <int OP, bool LOWNEG>
+template <int OP, int LOW>
 __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A, const float* __restrict__ B,
                                                      const float* __restrict__ GC, float* __restrict__ GA,
                                                      float* __restrict__ GB, BlkParams P) {
@@ -577,6 +710,7 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
     const unsigned fullh = NB - 1u;
     const bool want_a = GA != nullptr, want_b = GB != nullptr;
 
+    const LowMetric lo = low_metric(P);
     for (int kk = 0; kk < P.kpl; ++kk) {
         const unsigned h = lane_blk + ((unsigned)kk << P.lpr_log);
         const unsigned pi_h = cross_pi<OP>(h, P.nm1);
@@ -587,7 +721,7 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
             gb[e] = 0.f;
         }
         if constexpr (OP == OP_INNER) {
-            inner_bwd_blocks<LOWNEG>(la, lb, lg, h, fullh, want_a, want_b, ga, gb, P, t);
+            inner_bwd_blocks<LOW>(la, lb, lg, h, fullh, want_a, want_b, ga, gb, P, t, lo);
         } else
         for (unsigned m = 0; m < NB; ++m) {
             const unsigned x = h ^ m;
@@ -602,7 +736,8 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
                 float bv[16];
                 load_blk_s(lb, m, bslot(m, t), bv);
                 apply_flips(bv, sa.mask, sa.mask ^ (pi_h << 31));
-                ga_block_dispatch<OP, LOWNEG>(ga, bv, g, h, m);
+                if constexpr (LOW == LOW_MIX) mix_ga<OP>(ga, bv, g, lo);
+                else ga_block_dispatch<OP, LOW == LOW_NEG>(ga, bv, g, h, m);
             }
             if (do_b) {
                 const unsigned pm = cross_pi<OP>(m, P.nm1) << 31;
@@ -611,7 +746,8 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
                 apply_flips(av, sb.mask, sb.mask ^ pm);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) gt[e] = (cpopc((unsigned)e) & 1) ? flip(g[e], pm) : g[e];
-                gb_block_dispatch<OP, LOWNEG>(gb, av, gt, m, h);
+                if constexpr (LOW == LOW_MIX) mix_gb<OP>(gb, av, gt, lo);
+                else gb_block_dispatch<OP, LOW == LOW_NEG>(gb, av, gt, m, h);
             }
         }
         const long long base = (row0 + r) << (n - 2);
@@ -3690,6 +3826,7 @@ static void block_sign_params(int n, uint32_t neg, uint32_t nul, BlkParams& P) {
     P.nm1 = (n - 1) & 1;
     P.mu = popc_rt(neg) & 1;
     P.negl = neg & 15u;
+    P.null = nul & 15u;
 }
 
 constexpr size_t kBlockedLdsMax = 48 * 1024;
@@ -3708,9 +3845,8 @@ static unsigned blocked_row_skew(int n) {
     return 0u;
 }
 
-static bool blocked_plan(int op, int n, uint32_t neg, uint32_t nul, int nops, BlkParams& P, bool& lowneg,
-                         dim3& grid, dim3& block, size_t& lds_bytes) {
-    if (!blocked_metric(op, n, neg, nul, lowneg)) return false;
+static bool blocked_launch(int n, uint32_t neg, uint32_t nul, int nops, BlkParams& P, dim3& grid, dim3& block,
+                           size_t& lds_bytes) {
     const int nh = n - 4;
     const int NB = 1 << nh;
     const int lpr = NB < 64 ? NB : 64;
@@ -3730,6 +3866,21 @@ static bool blocked_plan(int op, int n, uint32_t neg, uint32_t nul, int nops, Bl
     block = dim3(64 * nwaves);
     lds_bytes = (size_t)P.rows_per_wg * row_bytes;
     return true;
+}
+
+static bool blocked_plan(int op, int n, uint32_t neg, uint32_t nul, int nops, BlkParams& P, bool& lowneg,
+                         dim3& grid, dim3& block, size_t& lds_bytes) {
+    if (!blocked_metric(op, n, neg, nul, lowneg)) return false;
+    return blocked_launch(n, neg, nul, nops, P, grid, block, lds_bytes);
+}
+
+// low generators of different squares, or null ones (blocked_metric fails): the
+// per-coefficient kernels keep n < 4 and rows beyond the LDS
+static bool mixed_plan(int op, int n, uint32_t neg, uint32_t nul, int nops, BlkParams& P, dim3& grid, dim3& block,
+                       size_t& lds_bytes) {
+    bool lowneg;
+    if (n < 4 || blocked_metric(op, n, neg, nul, lowneg)) return false;
+    return blocked_launch(n, neg, nul, nops, P, grid, block, lds_bytes);
 }
 
 // Grid cap of the grid-stride kernels (tiled, per-coefficient): well inside
@@ -4069,16 +4220,16 @@ static void launch_bwd_bal(hipStream_t s, const float* A, const float* B, const 
     hipLaunchKernelGGL((prod_bwd_bal<OP, LN>), g, dim3(256), 0, s, A, B, GCp, GA, GB, P);
 }
 
-template <int OP, bool LN>
+template <int OP, int LOW>
 static void launch_fwd(dim3 g, dim3 b, size_t lds, hipStream_t s, const float* A, const float* B, float* C,
                        const BlkParams& P) {
-    hipLaunchKernelGGL((prod_fwd_blk<OP, LN>), g, b, lds, s, A, B, C, P);
+    hipLaunchKernelGGL((prod_fwd_blk<OP, LOW>), g, b, lds, s, A, B, C, P);
 }
 
-template <int OP, bool LN>
+template <int OP, int LOW>
 static void launch_bwd(dim3 g, dim3 b, size_t lds, hipStream_t s, const float* A, const float* B, const float* GCp,
                        float* GA, float* GB, const BlkParams& P) {
-    hipLaunchKernelGGL((prod_bwd_blk<OP, LN>), g, b, lds, s, A, B, GCp, GA, GB, P);
+    hipLaunchKernelGGL((prod_bwd_blk<OP, LOW>), g, b, lds, s, A, B, GCp, GA, GB, P);
 }
 
 bool rep_applicable(int op, int n, uint32_t neg, uint32_t nul);
@@ -4091,7 +4242,7 @@ int64_t rep32_few_rows(int n, uint32_t neg, uint32_t nul);
 
 // Whether the op has kernels made for the signature: a matrix representation
 // for the geometric product, a uniform low metric for the others (false: the
-// geometric product's 4^n terms, or the per-coefficient kernels).
+// geometric product's 4^n terms, or the mixed low metrics' kernels).
 bool product_has_form(int op, int n, uint32_t neg, uint32_t nul) {
     bool lowneg;
     if (rep_disabled_by_env() || options().product_path != PATH_DEFAULT) return false;
@@ -4171,16 +4322,16 @@ int product_fwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
     } else if (!force_generic && !force_tiled && blocked_plan(op, n, neg, nul, 2, P, ln, g, bl, lds)) {
 #define CLF_FWD_CASE(OPV)                                              \
     case OPV:                                                          \
-        if (ln) launch_fwd<OPV, true>(g, bl, lds, s, a, b, c, P);      \
-        else launch_fwd<OPV, false>(g, bl, lds, s, a, b, c, P);        \
+        if (ln) launch_fwd<OPV, LOW_NEG>(g, bl, lds, s, a, b, c, P);   \
+        else launch_fwd<OPV, LOW_POS>(g, bl, lds, s, a, b, c, P);      \
         break;
         switch (op) {
             CLF_FWD_CASE(OP_GEOM)
             CLF_FWD_CASE(OP_INNER)
             CLF_FWD_CASE(OP_LC)
             CLF_FWD_CASE(OP_RC)
-            case OP_WEDGE: launch_fwd<OP_WEDGE, false>(g, bl, lds, s, a, b, c, P); break;
-            case OP_REGR: launch_fwd<OP_REGR, false>(g, bl, lds, s, a, b, c, P); break;
+            case OP_WEDGE: launch_fwd<OP_WEDGE, LOW_POS>(g, bl, lds, s, a, b, c, P); break;
+            case OP_REGR: launch_fwd<OP_REGR, LOW_POS>(g, bl, lds, s, a, b, c, P); break;
         }
 #undef CLF_FWD_CASE
     } else if (!force_generic && tiled_plan(op, n, neg, nul, P, ln, g)) {
@@ -4194,6 +4345,11 @@ int product_fwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
             case OP_REGR: CLF_FWD_TILED(OP_REGR, false); break;
         }
 #undef CLF_FWD_TILED
+    } else if (!force_generic && mixed_plan(op, n, neg, nul, 2, P, g, bl, lds)) {
+        if (op == OP_GEOM) launch_fwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, c, P);
+        else if (op == OP_INNER) launch_fwd<OP_INNER, LOW_MIX>(g, bl, lds, s, a, b, c, P);
+        else if (op == OP_LC) launch_fwd<OP_LC, LOW_MIX>(g, bl, lds, s, a, b, c, P);
+        else launch_fwd<OP_RC, LOW_MIX>(g, bl, lds, s, a, b, c, P);
     } else {
         const long long total = batch << n;
         const long long want = (total + 255) / 256;
@@ -4273,16 +4429,16 @@ int product_bwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
     } else if (!force_generic && !force_tiled && blocked_plan(op, n, neg, nul, 3, P, ln, g, bl, lds)) {
 #define CLF_BWD_CASE(OPV)                                                      \
     case OPV:                                                                  \
-        if (ln) launch_bwd<OPV, true>(g, bl, lds, s, a, b, gc, ga, gb, P);     \
-        else launch_bwd<OPV, false>(g, bl, lds, s, a, b, gc, ga, gb, P);       \
+        if (ln) launch_bwd<OPV, LOW_NEG>(g, bl, lds, s, a, b, gc, ga, gb, P);  \
+        else launch_bwd<OPV, LOW_POS>(g, bl, lds, s, a, b, gc, ga, gb, P);     \
         break;
         switch (op) {
             CLF_BWD_CASE(OP_GEOM)
             CLF_BWD_CASE(OP_INNER)
             CLF_BWD_CASE(OP_LC)
             CLF_BWD_CASE(OP_RC)
-            case OP_WEDGE: launch_bwd<OP_WEDGE, false>(g, bl, lds, s, a, b, gc, ga, gb, P); break;
-            case OP_REGR: launch_bwd<OP_REGR, false>(g, bl, lds, s, a, b, gc, ga, gb, P); break;
+            case OP_WEDGE: launch_bwd<OP_WEDGE, LOW_POS>(g, bl, lds, s, a, b, gc, ga, gb, P); break;
+            case OP_REGR: launch_bwd<OP_REGR, LOW_POS>(g, bl, lds, s, a, b, gc, ga, gb, P); break;
         }
 #undef CLF_BWD_CASE
     } else if (!force_generic && tiled_plan(op, n, neg, nul, P, ln, g)) {
@@ -4297,6 +4453,11 @@ int product_bwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
             case OP_REGR: CLF_BWD_TILED(OP_REGR, false); break;
         }
 #undef CLF_BWD_TILED
+    } else if (!force_generic && mixed_plan(op, n, neg, nul, 3, P, g, bl, lds)) {
+        if (op == OP_GEOM) launch_bwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
+        else if (op == OP_INNER) launch_bwd<OP_INNER, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
+        else if (op == OP_LC) launch_bwd<OP_LC, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
+        else launch_bwd<OP_RC, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
     } else {
         const long long total = batch << n;
         const long long want = (total + 255) / 256;
