@@ -410,7 +410,10 @@ struct BlkParams {
 // 1057 + 2242 -> 711 + 1293, so they take every batch that fits their LDS. Bound
 // by the lanes of a wave whose partner blocks the op drops (a quarter to a half
 // of the steps), from n = 7 on; below that by memory.
-enum { LOW_POS = 0, LOW_NEG = 1, LOW_MIX = 2 };
+// LOW_NULL: the geometric product's variant with a null generator among them
+// (its branches cost registers: 21 + 33 us at n = 6, 60000 rows, against 14 + 29
+// with the null terms multiplied by 0, which would turn an infinity into NaN).
+enum { LOW_POS = 0, LOW_NEG = 1, LOW_MIX = 2, LOW_NULL = 3 };
 
 struct LowMetric {
     float m[16];
@@ -461,34 +464,42 @@ __device__ __forceinline__ void mix_contr(float (&acc)[16], const float (&u)[16]
 }
 
 // The geometric product; d: the operand that is dressed, on the way to index E
-// with generators below K done. MODE 0: acc[il ^ jl] += s v[il] d[jl]; 1:
+// with generators below K done; SKIP: the null generators in E, whose blades of the
+// dressed operand are passed over (a uniform choice per level). MODE 0: acc[il ^ jl] += s v[il] d[jl]; 1:
 // acc[il] += s d[jl] v[il ^ jl]; 2: acc[jl] += s d[il] v[il ^ jl].
-template <int MODE, int K = 0, int E = 0>
+template <int MODE, bool NUL, int K = 0, int E = 0, int SKIP = 0>
 __device__ __forceinline__ void mix_geom(float (&acc)[16], const float (&d)[16], const float (&v)[16],
                                          const LowMetric& lo) {
     if constexpr (K == 4) {
         each16([&](auto fc) __attribute__((always_inline)) {
             constexpr int F = decltype(fc)::value;
             constexpr int s = MODE == 2 ? low_sign(LV_GEOM, false, (unsigned)F, (unsigned)E) : low_sign(LV_GEOM, false, (unsigned)E, (unsigned)F);
-            if constexpr (MODE == 0) acc[E ^ F] = __builtin_fmaf(s > 0 ? v[E] : -v[E], d[F], acc[E ^ F]);
+            if constexpr ((F & SKIP) != 0) return;
+            else if constexpr (MODE == 0) acc[E ^ F] = __builtin_fmaf(s > 0 ? v[E] : -v[E], d[F], acc[E ^ F]);
             else acc[E] = __builtin_fmaf(s > 0 ? d[F] : -d[F], v[E ^ F], acc[E]);
         });
     } else {
-        mix_geom<MODE, K + 1, E>(acc, d, v, lo);
-        float w[16];
+        mix_geom<MODE, NUL, K + 1, E, SKIP>(acc, d, v, lo);
         const float m = lo.m[1 << K];
+        if constexpr (NUL) {
+            if (m == 0.f) {
+                mix_geom<MODE, NUL, K + 1, E | (1 << K), SKIP | (1 << K)>(acc, d, v, lo);
+                return;
+            }
+        }
+        float w[16];
         each16([&](auto fc) __attribute__((always_inline)) {
             constexpr int F = decltype(fc)::value;
             w[F] = (F >> K) & 1 ? m * d[F] : d[F];
         });
-        mix_geom<MODE, K + 1, E | (1 << K)>(acc, w, v, lo);
+        mix_geom<MODE, NUL, K + 1, E | (1 << K), SKIP>(acc, w, v, lo);
     }
 }
 
-template <int OP>
+template <int OP, bool NUL>
 __device__ __forceinline__ void mix_fwd(float (&acc)[16], const float (&a)[16], const float (&b)[16], unsigned ih,
                                         unsigned jh, const LowMetric& lo) {
-    if constexpr (OP == OP_GEOM) mix_geom<0>(acc, b, a, lo);
+    if constexpr (OP == OP_GEOM) mix_geom<0, NUL>(acc, b, a, lo);
     else if constexpr (OP == OP_LC) mix_contr<LV_LC, 0>(acc, a, b, lo);
     else if constexpr (OP == OP_RC) mix_contr<LV_RC, 0>(acc, b, a, lo);
     else {
@@ -499,18 +510,18 @@ __device__ __forceinline__ void mix_fwd(float (&acc)[16], const float (&a)[16], 
     }
 }
 
-template <int OP>
+template <int OP, bool NUL>
 __device__ __forceinline__ void mix_ga(float (&acc)[16], const float (&b)[16], const float (&g)[16],
                                        const LowMetric& lo) {
-    if constexpr (OP == OP_GEOM) mix_geom<1>(acc, b, g, lo);
+    if constexpr (OP == OP_GEOM) mix_geom<1, NUL>(acc, b, g, lo);
     else if constexpr (OP == OP_LC) mix_contr<LV_LC, 1>(acc, b, g, lo);
     else mix_contr<LV_RC, 2>(acc, b, g, lo);
 }
 
-template <int OP>
+template <int OP, bool NUL>
 __device__ __forceinline__ void mix_gb(float (&acc)[16], const float (&a)[16], const float (&g)[16],
                                        const LowMetric& lo) {
-    if constexpr (OP == OP_GEOM) mix_geom<2>(acc, a, g, lo);
+    if constexpr (OP == OP_GEOM) mix_geom<2, NUL>(acc, a, g, lo);
     else if constexpr (OP == OP_LC) mix_contr<LV_LC, 2>(acc, a, g, lo);
     else mix_contr<LV_RC, 1>(acc, a, g, lo);
 }
@@ -598,7 +609,7 @@ __global__ __launch_bounds__(256) void prod_fwd_blk(const float* __restrict__ A,
             load_blk_s(la, ih, bslot(ih, t), av);
             load_blk_s(lb, jh, bslot(jh, t), bv);
             apply_flips(bv, hs.mask, hs.mask ^ (cross_pi<OP>(ih, P.nm1) << 31));
-            if constexpr (LOW == LOW_MIX) mix_fwd<OP>(acc, av, bv, ih, jh, lo);
+            if constexpr (LOW >= LOW_MIX) mix_fwd<OP, LOW == LOW_NULL>(acc, av, bv, ih, jh, lo);
             else fwd_block_dispatch<OP, LOW == LOW_NEG>(acc, av, bv, ih, jh);
         }
         if (OP == OP_REGR) {
@@ -736,7 +747,7 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
                 float bv[16];
                 load_blk_s(lb, m, bslot(m, t), bv);
                 apply_flips(bv, sa.mask, sa.mask ^ (pi_h << 31));
-                if constexpr (LOW == LOW_MIX) mix_ga<OP>(ga, bv, g, lo);
+                if constexpr (LOW >= LOW_MIX) mix_ga<OP, LOW == LOW_NULL>(ga, bv, g, lo);
                 else ga_block_dispatch<OP, LOW == LOW_NEG>(ga, bv, g, h, m);
             }
             if (do_b) {
@@ -746,7 +757,7 @@ __global__ __launch_bounds__(256) void prod_bwd_blk(const float* __restrict__ A,
                 apply_flips(av, sb.mask, sb.mask ^ pm);
 #pragma unroll
                 for (int e = 0; e < 16; ++e) gt[e] = (cpopc((unsigned)e) & 1) ? flip(g[e], pm) : g[e];
-                if constexpr (LOW == LOW_MIX) mix_gb<OP>(gb, av, gt, lo);
+                if constexpr (LOW >= LOW_MIX) mix_gb<OP, LOW == LOW_NULL>(gb, av, gt, lo);
                 else gb_block_dispatch<OP, LOW == LOW_NEG>(gb, av, gt, m, h);
             }
         }
@@ -4346,7 +4357,8 @@ int product_fwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
         }
 #undef CLF_FWD_TILED
     } else if (!force_generic && mixed_plan(op, n, neg, nul, 2, P, g, bl, lds)) {
-        if (op == OP_GEOM) launch_fwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, c, P);
+        if (op == OP_GEOM && P.null) launch_fwd<OP_GEOM, LOW_NULL>(g, bl, lds, s, a, b, c, P);
+        else if (op == OP_GEOM) launch_fwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, c, P);
         else if (op == OP_INNER) launch_fwd<OP_INNER, LOW_MIX>(g, bl, lds, s, a, b, c, P);
         else if (op == OP_LC) launch_fwd<OP_LC, LOW_MIX>(g, bl, lds, s, a, b, c, P);
         else launch_fwd<OP_RC, LOW_MIX>(g, bl, lds, s, a, b, c, P);
@@ -4454,7 +4466,8 @@ int product_bwd_ld(int op, int n, uint32_t neg, uint32_t nul, const float* a, in
         }
 #undef CLF_BWD_TILED
     } else if (!force_generic && mixed_plan(op, n, neg, nul, 3, P, g, bl, lds)) {
-        if (op == OP_GEOM) launch_bwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
+        if (op == OP_GEOM && P.null) launch_bwd<OP_GEOM, LOW_NULL>(g, bl, lds, s, a, b, gc, ga, gb, P);
+        else if (op == OP_GEOM) launch_bwd<OP_GEOM, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
         else if (op == OP_INNER) launch_bwd<OP_INNER, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
         else if (op == OP_LC) launch_bwd<OP_LC, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);
         else launch_bwd<OP_RC, LOW_MIX>(g, bl, lds, s, a, b, gc, ga, gb, P);

@@ -56,3 +56,19 @@ def test_against_oracle(op, m, clf_env):
     clf_env.setenv("CLF_PRODUCT_PATH", "generic")
     for x, r in zip(got, grads(op, metric, ad, bd, gd)):
         assert rel_err(x, r) <= TOL
+
+
+@pytest.mark.parametrize("op", list(FN))
+@pytest.mark.parametrize("m", ["0+-+", "+0-00-+"])
+def test_null_terms_are_passed_over(op, m, clf_env):
+    """A term that a null generator takes away is not formed: an infinite
+    coefficient reaches the same outputs as in the per-coefficient kernels."""
+    metric = signature(m)
+    g = torch.Generator().manual_seed(1)
+    D = 1 << len(m)
+    a, b, gc = (torch.randn(D, D, generator=g).cuda() for _ in range(3))
+    a.diagonal().fill_(float("inf"))  # row r: coefficient r
+    got = grads(op, metric, a, b, gc)
+    clf_env.setenv("CLF_PRODUCT_PATH", "generic")
+    for x, r in zip(got, grads(op, metric, a, b, gc)):
+        assert torch.equal(x.isfinite(), r.isfinite())
