@@ -3,8 +3,8 @@
 //
 // Ten generators ("base") form a signature with Cl = M_32(R) (p - q = 0 or 2
 // mod 8): 10 - D of the n generators and D dummies that no blade of a row
-// holds (their coefficients are staged as zeros), which lets the signatures in
-// that no ten (n = 9: no nine) generators are of real type. The other
+// holds (their coefficients are staged as zeros), which lets in the signatures
+// of which no ten (n = 9: no nine) generators are of real type. The other
 // K = n - 10 + D generators ("ext", any square, null too) extend it. With every blade written e_I e_S (I base, S ext) a row
 // is 2^K base rows x_S, and for (A_S e_S)(B_J e_J):
 //   C_R = sum_{S ^ J = R} sigma(S, J) A_S alpha^{|S|}(B_J),
