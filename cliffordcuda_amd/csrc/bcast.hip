@@ -306,17 +306,25 @@ __global__ __launch_bounds__(256) void column_sum_kernel(const float4* __restric
 }
 
 // gw[c] = sum of the nparts partials of column c, in fp64: 32 columns per
-// workgroup, eight threads each
-__global__ __launch_bounds__(256) void column_total_kernel(const float* __restrict__ parts, int nparts, int n,
-                                                           float* __restrict__ gw) {
-    __shared__ double red[256];
+// workgroup, 32 threads each with eight loads in flight (eight threads each,
+// one load after the other, measured 9.3 us for 256 partials of 256 columns)
+__global__ __launch_bounds__(1024) void column_total_kernel(const float* __restrict__ parts, int nparts, int n,
+                                                            float* __restrict__ gw) {
+    __shared__ double red[1024];
     const int c = blockIdx.x * 32 + (threadIdx.x & 31);
     double t = 0.0;
-    for (int p = threadIdx.x >> 5; p < nparts; p += 8) t += (double)parts[((long long)p << n) + c];
+    for (int p = threadIdx.x >> 5; p < nparts; p += 256) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p + 32 * u < nparts ? parts[((long long)(p + 32 * u) << n) + c] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t += (double)v[u];
+    }
     red[threadIdx.x] = t;
     __syncthreads();
     if (threadIdx.x >= 32) return;
-    for (int g = 1; g < 8; ++g) t += red[g * 32 + threadIdx.x];
+#pragma unroll
+    for (int g = 1; g < 32; ++g) t += red[g * 32 + threadIdx.x];
     gw[c] = (float)t;
 }
 
@@ -416,7 +424,7 @@ static int rows_bwd(int op, int side, int n, uint32_t neg, uint32_t nul, const f
         if (r0 == 0) hipLaunchKernelGGL((column_sum_kernel<false>), dim3(nparts), dim3(256), 0, s, g4, rows, n - 2, p4);
         else hipLaunchKernelGGL((column_sum_kernel<true>), dim3(nparts), dim3(256), 0, s, g4, rows, n - 2, p4);
     }
-    if (gw) hipLaunchKernelGGL(column_total_kernel, dim3(1u << (n - 5)), dim3(256), 0, s, parts, nparts, n, gw);
+    if (gw) hipLaunchKernelGGL(column_total_kernel, dim3(1u << (n - 5)), dim3(1024), 0, s, parts, nparts, n, gw);
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
