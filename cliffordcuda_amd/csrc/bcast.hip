@@ -388,7 +388,8 @@ static size_t rows_ws_floats(int n, int64_t batch) {
 // 52 + 122, Cl(7,1) geom 83 + 253 -> 26 + 80, and at 2000 rows inner 26 + 185
 // -> 8 + 29; n = 9, 20000 rows: geom 117 + 290 -> 25 + 88, inner 105 + 267 ->
 // 46 + 141; n = 10, 4096 rows: geom 93 + 257 -> 11 + 38, inner 94 + 257 ->
-// 31 + 109. No form measured slower at any batch. The backward is bound by
+// 31 + 109 (before column_total_kernel's loads in flight, 5 to 10 less since).
+// No form measured slower at any batch. The backward is bound by
 // writing and reading back the per-row weight gradients beside x, gy and gx.
 static bool use_rows(int op, int n, uint32_t neg, uint32_t nul) { return product_has_form(op, n, neg, nul); }
 
