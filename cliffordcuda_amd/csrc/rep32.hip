@@ -5,8 +5,9 @@
 // mod 8): 10 - D of the n generators and D dummies that no blade of a row
 // holds (their coefficients are staged as zeros), which lets in the signatures
 // of which no ten (n = 9: no nine) generators are of real type. The other
-// K = n - 10 + D generators ("ext", any square, null too) extend it. With every blade written e_I e_S (I base, S ext) a row
-// is 2^K base rows x_S, and for (A_S e_S)(B_J e_J):
+// K = n - 10 + D generators ("ext", any square, null too) extend it. With every
+// blade written e_I e_S (I base, S ext) a row is 2^K base rows x_S, and for
+// (A_S e_S)(B_J e_J):
 //   C_R = sum_{S ^ J = R} sigma(S, J) A_S alpha^{|S|}(B_J),
 // alpha the grade involution of the base (e_S passes B_J's blades) and sigma
 // the ext signs. In the representation phi each term is one 32 x 32 x 32
@@ -36,19 +37,25 @@
 // the chunk index under a host-chosen mask) so that the 32 gathers of a step
 // fall on 32 banks.
 //
+// Rows whose coefficients are not of one scale are formed term by term in the
+// same launch (geom_terms.h). The test costs about 90 of 740 vector instructions
+// of a forward wave.
+//
 // Bound: 12 (forward) and 20 (backward) 2^n bytes a row over HBM against 4^K
-// 1024 matrix-core cycles a row forward and twice that backward: HBM at n = 10,
-// matrix issue beside it at n = 11, 12; a workgroup's own latency for a few
-// rows. Measured (us, forward + backward; per-term kernels before): n = 10,
-// 16384 rows 33 + 68 (6.1 and 4.9 TB/s; 352 + 679); n = 11, 4096 rows 26 + 47
-// (3.9 and 3.6 TB/s; 545 + 1180); n = 12, 1024 rows 22 + 41 (660 + 2580), 64
-// rows 8.5 + 14 (34 + 65). With dummies, 8000 rows: n = 9 17 + 30 (59 + 111),
-// Cl(8,0,1) 38 + 70 (53 + 100), Cl(8,2) 41 + 78 (183 + 350), Cl(8,3) 118 + 231
-// (955 + 2073).
+// 1024 matrix-core cycles a row forward and twice that backward; vector
+// instructions beside them (the test added 3 to 10 %); a workgroup's own latency
+// for a few rows. Measured (us, forward + backward; before: the per-term kernels),
+// N(0, 1) rows: n = 10, 16384 rows 37 + 75 (5.4 and 4.5 TB/s; 358 + 690); n = 11,
+// 4096 rows 27.5 + 50 (3.7 and 3.4 TB/s; 542 + 1180); n = 12, 1024 rows 22.7 + 41
+// (660 + 2580), 64 rows 9 + 15 (35 + 63). With dummies, 8000 rows: n = 9 20 + 36
+// (62 + 115), Cl(7,2) 48 + 86 (57 + 105), Cl(8,2) 45 + 84 (184 + 355), Cl(8,3)
+// 123 + 244 (950 + 2070). Rows that all go by their terms: n = 9 68 + 148, Cl(7,2)
+// 67 + 136, n = 10 431 + 893, n = 11 422 + 852, n = 12 440 + 913 and 32 + 67,
+// Cl(8,2) 211 + 439, Cl(8,3) 792 + 1604.
 #include <map>
 #include <mutex>
 
-#include "rep_common.h"
+#include "geom_terms.h"
 
 namespace clf {
 
@@ -64,6 +71,7 @@ struct Rep32Table {
     unsigned chunk_mask[3];         // chunk group bit t is flipped by the parity of chunk & chunk_mask[t]
     unsigned ox, oz;                // label of the base pseudoscalar
     unsigned neg_pairs, zero_pairs; // ext signs: bit 4 S + J
+    TermSpec terms;                 // for the rows that are not of one scale
 };
 
 // word of element (r, p), split into its xor-linear row part and p itself
@@ -124,6 +132,66 @@ __device__ __forceinline__ BigRow big_fetch(const float* __restrict__ src, int l
         r.v[j] = NT ? load_stream(q) : *q;
     }
     return r;
+}
+
+// Which of the wave's parts of its rows are not of one scale (geom_terms.h), bit
+// i for rows[i]. Each part is converted by itself and two parts' products meet
+// in plain sums, so the parts of a row may differ in scale.
+template <int D, int COUNT>
+__device__ __forceinline__ unsigned big_uneven(const BigRow* const (&rows)[COUNT]) {
+    unsigned bad = 0;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+        float q = 0.f;
+#pragma unroll
+        for (int j = 0; j < (4 >> D); ++j) q += sumsq4(rows[i]->v[j]);
+        q = wave_total(q);
+        const float level = even_level(q, kBigBase - D);
+        int large = 0;
+#pragma unroll
+        for (int j = 0; j < (4 >> D); ++j) large += even_large(rows[i]->v[j], level);
+        bad |= even_range(q) && even_count(large, 1024 >> D) ? 0u : 1u << i;
+    }
+    return __builtin_amdgcn_readfirstlane(bad);
+}
+
+// The or of the row's waves' marks; every wave writes its own before a big_sync
+// and calls this after it.
+template <int K>
+__device__ __forceinline__ unsigned big_marks(const unsigned (&marks)[4], unsigned first, unsigned own) {
+    if constexpr (K == 0) return own;
+    unsigned m = 0;
+#pragma unroll
+    for (unsigned s = 0; s < (1u << K); ++s) m |= marks[first + s];
+    return __builtin_amdgcn_readfirstlane(m);
+}
+
+// Whether no row of the workgroup (K = 0: of the wave) has use for its matrices
+template <int K, class All>
+__device__ __forceinline__ bool big_skip(const unsigned (&marks)[4], bool own, All&& all) {
+    if constexpr (K == 0) return own;
+    constexpr unsigned NS = 1u << K;
+    bool skip = true;
+#pragma unroll
+    for (unsigned r = 0; r < 4; r += NS) {
+        unsigned m = 0;
+#pragma unroll
+        for (unsigned s = 0; s < NS; ++s) m |= marks[r + s];
+        skip = skip && all(m);
+    }
+    return __builtin_amdgcn_readfirstlane(skip);
+}
+
+// one row by its terms: the lanes of the row's waves (of all its workgroups),
+// 2^log to a block
+template <int K, int D, int MODE>
+__device__ __forceinline__ void big_terms(const float* __restrict__ X, long long ldx, const float* __restrict__ Y,
+                                          long long ldy, float* __restrict__ out, long long row, unsigned S,
+                                          unsigned lane, const TermSpec& t, int log) {
+    const unsigned per = 6 - log;  // a wave's blocks, log2
+    const unsigned h = ((blockIdx.y << K | S) << per) | (lane & ((1u << per) - 1u));
+    term_block<MODE>(X + big_off<K, D>(row, ldx, 0), Y + big_off<K, D>(row, ldy, 0), out + big_off<K, D>(row, 1, 0), h,
+                     t, lane >> per, log);
 }
 
 __device__ __forceinline__ void big_stage(float* __restrict__ region, const BigRow& r, const unsigned (&cpos)[4]) {
@@ -280,10 +348,11 @@ __device__ __forceinline__ BigLane big_lane(unsigned lane, const Rep32Table& T) 
 template <int K, int D, bool NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep32_fwd_kernel(
     const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb, float* __restrict__ C,
-    long long batch, Rep32Table T) {
+    long long batch, int terms_log, Rep32Table T) {
     constexpr unsigned NS = 1u << K;  // base rows per row
     constexpr int kRows = 4 >> K;     // rows per workgroup
     __shared__ __attribute__((aligned(4096))) float lds[2][4 * 1024];
+    __shared__ unsigned marks[4];
     const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const unsigned x = lane & 31u, h = lane >> 5;
     const unsigned S = wave & (NS - 1u), first = wave - S;
@@ -294,21 +363,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
     const BigLane L = big_lane(lane, T);
     unsigned cpos[4];
     big_places<K, D>(S, lane, T, cpos);
-
-    for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
-        long long row = row0 + (wave >> K);
-        const bool live = row < batch;  // rows past the end recompute the last row and are not stored
-        row = live ? row : batch - 1;
-        const long long off = big_off<K, D>(row, 1, S);
-        const BigRow va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
-        const BigRow vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
-        big_stage(ra, va, cpos);
-        big_stage(rb, vb, cpos);
-        big_sync<K>();
-        float ta[16], tb[16];
-        big_gather(ra, pos, T, ta);
-        big_gather(rb, pos, T, tb);
-        big_sync<K>();
+    long long row = (long long)blockIdx.x * kRows + (wave >> K);
+    const bool live = row < batch;  // rows past the end recompute the last row and are not stored
+    row = live ? row : batch - 1;
+    const long long off = big_off<K, D>(row, 1, S);
+    const BigRow va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
+    const BigRow vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
+    big_stage(ra, va, cpos);
+    big_stage(rb, vb, cpos);
+    big_sync<K>();
+    float ta[16], tb[16];
+    big_gather(ra, pos, T, ta);
+    big_gather(rb, pos, T, tb);
+    const unsigned own = big_uneven<D, 2>({&va, &vb});
+    if (K > 0 && lane == 0) marks[wave] = own;
+    big_sync<K>();
+    const unsigned by_terms = big_marks<K>(marks, first, own);
+    if (blockIdx.y == 0 && !big_skip<K>(marks, own != 0u, [](unsigned r) { return r != 0u; })) {
         big_convert<16>(ta, m, ra + S * 1024, x, h);
         big_convert<0>(tb, m, rb + S * 1024, x, h);
         big_sync<K>();
@@ -329,19 +400,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         big_unconvert(acc, ra + S * 1024, m, lane, ta);
         big_scatter(rb, pos, T, ta);
         big_sync<K>();
-        if (live) big_store<D, NT>(C + off, rb, cpos, lane);
-        big_sync<K>();
+        if (live && !by_terms) big_store<D, NT>(C + off, rb, cpos, lane);
     }
+    if (live && by_terms) big_terms<K, D, TERM_C>(A, lda, B, ldb, C, row, S, lane, T.terms, terms_log);
 }
+
+constexpr unsigned kMarkGA = 1 | 2, kMarkGB = 1 | 4;  // rows (gc, b, a) that a gradient needs of one scale
 
 template <int K, int D, bool NT, bool WA, bool WB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void rep32_bwd_kernel(
     const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
     const float* __restrict__ GC, long long ldg, float* __restrict__ GA, float* __restrict__ GB, long long batch,
-    Rep32Table T) {
+    int terms_log, Rep32Table T) {
     constexpr unsigned NS = 1u << K;
     constexpr int kRows = 4 >> K;
     __shared__ __attribute__((aligned(4096))) float lds[3][4 * 1024];
+    __shared__ unsigned marks[4];
     const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     const unsigned x = lane & 31u, h = lane >> 5;
     const unsigned S = wave & (NS - 1u), first = wave - S;
@@ -354,25 +428,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
     unsigned cpos[4];
     big_places<K, D>(S, lane, T, cpos);
     const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-
-    for (long long row0 = (long long)blockIdx.x * kRows; row0 < batch; row0 += (long long)gridDim.x * kRows) {
-        long long row = row0 + (wave >> K);
-        const bool live = row < batch;
-        row = live ? row : batch - 1;
-        const long long off = big_off<K, D>(row, 1, S);
-        const BigRow vg = big_fetch<D, NT>(GC + big_off<K, D>(row, ldg, S), lane);
-        BigRow va, vb;
-        if (WA) vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
-        if (WB) va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
-        big_stage(r0, vg, cpos);
-        if (WA) big_stage(r1, vb, cpos);
-        if (WB) big_stage(r2, va, cpos);
-        big_sync<K>();
-        float tg[16], ta[16], tb[16];
-        big_gather(r0, pos, T, tg);
-        if (WA) big_gather(r1, pos, T, tb);
-        if (WB) big_gather(r2, pos, T, ta);
-        big_sync<K>();
+    long long row = (long long)blockIdx.x * kRows + (wave >> K);
+    const bool live = row < batch;
+    row = live ? row : batch - 1;
+    const long long off = big_off<K, D>(row, 1, S);
+    const BigRow vg = big_fetch<D, NT>(GC + big_off<K, D>(row, ldg, S), lane);
+    BigRow va, vb;
+    if (WA) vb = big_fetch<D, NT>(B + big_off<K, D>(row, ldb, S), lane);
+    if (WB) va = big_fetch<D, NT>(A + big_off<K, D>(row, lda, S), lane);
+    big_stage(r0, vg, cpos);
+    if (WA) big_stage(r1, vb, cpos);
+    if (WB) big_stage(r2, va, cpos);
+    big_sync<K>();
+    float tg[16], ta[16], tb[16];
+    big_gather(r0, pos, T, tg);
+    if (WA) big_gather(r1, pos, T, tb);
+    if (WB) big_gather(r2, pos, T, ta);
+    unsigned own;  // gc, b, a
+    if constexpr (WA && WB) own = big_uneven<D, 3>({&vg, &vb, &va});
+    else if constexpr (WA) own = big_uneven<D, 2>({&vg, &vb});
+    else own = big_uneven<D, 2>({&vg, &va}) != 0u ? kMarkGB : 0u;
+    if (K > 0 && lane == 0) marks[wave] = own;
+    big_sync<K>();
+    const unsigned by_terms = big_marks<K>(marks, first, own);
+    const auto all = [](unsigned r) { return (!WA || (r & kMarkGA)) && (!WB || (r & kMarkGB)); };
+    if (blockIdx.y == 0 && !big_skip<K>(marks, all(own), all)) {
         if (WA) {
             // gA_S = sum_J sigma(S, J) G_{S^J} alpha^{|S|}(B_J)^T
             big_convert<16>(tg, m, r0 + S * 1024, x, h);
@@ -404,7 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
             big_convert<0>(ta, m, r1 + S * 1024, x, h);
         }
         big_sync<K>();
-        if (WA && live) big_store<D, NT>(GA + off, r2, cpos, lane);
+        if (WA && live && !(by_terms & kMarkGA)) big_store<D, NT>(GA + off, r2, cpos, lane);
         if (WB) {
             floatx16 acc = zero;
 #pragma unroll 1
@@ -423,10 +503,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void r
             big_unconvert(acc, r0 + S * 1024, m, lane, ta);
             big_scatter(r1, pos, T, ta);
             big_sync<K>();
-            if (live) big_store<D, NT>(GB + off, r1, cpos, lane);
+            if (live && !(by_terms & kMarkGB)) big_store<D, NT>(GB + off, r1, cpos, lane);
         }
-        big_sync<K>();
     }
+    if (!live) return;
+    if (WA && (by_terms & kMarkGA)) big_terms<K, D, TERM_GA>(B, ldb, GC, ldg, GA, row, S, lane, T.terms, terms_log);
+    if (WB && (by_terms & kMarkGB)) big_terms<K, D, TERM_GB>(A, lda, GC, ldg, GB, row, S, lane, T.terms, terms_log);
 }
 
 // ---- host side --------------------------------------------------------------
@@ -667,17 +749,30 @@ bool big_table(int n, uint32_t neg, uint32_t nul, const BigSplit& c, Rep32Table&
     }
     T = Rep32Table{};
     if (!big_table_build(n + c.d, neg | (((1u << c.dneg) - 1u) << n), nul, c.ext, T)) return false;
+    if (!term_spec(n, neg, nul, T.terms)) return false;  // (ten of one square or two always hold four of one)
     std::lock_guard<std::mutex> lock(mu);
     if (cache.size() < kBigTables) cache.emplace(key, T);
     return true;
 }
 
-// One workgroup per 4 / 2^K rows; the cap only bounds the grid dimension (the
-// kernels walk any batch).
-unsigned big_grid(int k, int64_t batch) {
-    const long long rows = 4 >> k;
-    const long long g = (batch + rows - 1) / rows;
-    return (unsigned)(g < (1LL << 22) ? g : (1LL << 22));
+// One workgroup per 4 / 2^K rows (no row loop in the kernels: nothing that only
+// the term sums need is held across the matrix part), at most 2^22 in a launch,
+// well inside the 2^32 work-items of one launch dimension. Few rows get more
+// workgroups, which share a row's term sums if it needs them and end otherwise:
+// enough for two on each CU, and at most 16 lanes for a block.
+// launch(r0, rows, grid, lanes of a block log2) runs for each chunk of rows.
+template <class Launch>
+void big_chunks(int n, int k, int64_t batch, Launch&& launch) {
+    const int64_t per = 4 >> k, most = per << 22;
+    for (int64_t r0 = 0; r0 < batch; r0 += most) {
+        const int64_t rows = batch - r0 < most ? batch - r0 : most, groups = (rows + per - 1) / per;
+        int log = 6 + k - (n - 4), more = 0;
+        while (log < 4 && groups << (more + 1) <= 512) {
+            ++log;
+            ++more;
+        }
+        launch(r0, rows, dim3((unsigned)groups, 1u << more), log);
+    }
 }
 
 }  // namespace
@@ -716,15 +811,18 @@ int64_t rep32_rows(int n, uint32_t neg, uint32_t nul) {
     }
 
 template <int K, int D>
-static void launch_rep32_fwd(dim3 grid, hipStream_t s, bool nt, const float* a, int64_t lda, const float* b,
-                             int64_t ldb, float* c, int64_t batch, const Rep32Table& T) {
-    const dim3 block(256);
-    if (nt)
-        hipLaunchKernelGGL((rep32_fwd_kernel<K, D, true>), grid, block, 0, s, a, (long long)lda, b, (long long)ldb, c,
-                           (long long)batch, T);
-    else
-        hipLaunchKernelGGL((rep32_fwd_kernel<K, D, false>), grid, block, 0, s, a, (long long)lda, b, (long long)ldb, c,
-                           (long long)batch, T);
+static void launch_rep32_fwd(int n, hipStream_t s, bool nt, const float* a, int64_t lda, const float* b, int64_t ldb,
+                             float* c, int64_t batch, const Rep32Table& T) {
+    big_chunks(n, K, batch, [&](int64_t r0, int64_t rows, dim3 grid, int log) {
+        const int64_t off = r0 << n;
+        const float *ar = a + (lda ? off : 0), *br = b + (ldb ? off : 0);
+        if (nt)
+            hipLaunchKernelGGL((rep32_fwd_kernel<K, D, true>), grid, dim3(256), 0, s, ar, (long long)lda, br,
+                               (long long)ldb, c + off, (long long)rows, log, T);
+        else
+            hipLaunchKernelGGL((rep32_fwd_kernel<K, D, false>), grid, dim3(256), 0, s, ar, (long long)lda, br,
+                               (long long)ldb, c + off, (long long)rows, log, T);
+    });
 }
 
 int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* out,
@@ -735,7 +833,7 @@ int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, co
         return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
     const bool nt = stream_nt(3.0 * 4.0 * (double)(1LL << n) * (double)batch);
 #define CLF_BIG_FWD(K, D) \
-    launch_rep32_fwd<K, D>(dim3(big_grid(c.k, batch)), (hipStream_t)stream, nt, a, lda, b, ldb, out, batch, T)
+    launch_rep32_fwd<K, D>(n, (hipStream_t)stream, nt, a, lda, b, ldb, out, batch, T)
     CLF_BIG_SWITCH(CLF_BIG_FWD)
 #undef CLF_BIG_FWD
     CLF_HIP_CHECK(hipGetLastError());
@@ -743,16 +841,21 @@ int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, co
 }
 
 template <int K, int D, bool NT>
-static void launch_rep32_bwd(dim3 grid, hipStream_t s, const float* a, int64_t lda, const float* b, int64_t ldb,
+static void launch_rep32_bwd(int n, hipStream_t s, const float* a, int64_t lda, const float* b, int64_t ldb,
                              const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch,
                              const Rep32Table& T) {
-#define CLF_BIG_BWD_W(WA, WB)                                                                                     \
-    hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, WA, WB>), grid, dim3(256), 0, s, a, (long long)lda, b,          \
-                       (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
-    if (ga && gb) CLF_BIG_BWD_W(true, true);
-    else if (ga) CLF_BIG_BWD_W(true, false);
-    else CLF_BIG_BWD_W(false, true);
+    big_chunks(n, K, batch, [&](int64_t r0, int64_t rows, dim3 grid, int log) {
+        const int64_t off = r0 << n;
+        const float *ar = a + (lda ? off : 0), *br = b + (ldb ? off : 0), *gr = gc + (ldg ? off : 0);
+        float *gar = ga ? ga + off : nullptr, *gbr = gb ? gb + off : nullptr;
+#define CLF_BIG_BWD_W(WA, WB)                                                                                 \
+    hipLaunchKernelGGL((rep32_bwd_kernel<K, D, NT, WA, WB>), grid, dim3(256), 0, s, ar, (long long)lda, br,    \
+                       (long long)ldb, gr, (long long)ldg, gar, gbr, (long long)rows, log, T)
+        if (ga && gb) CLF_BIG_BWD_W(true, true);
+        else if (ga) CLF_BIG_BWD_W(true, false);
+        else CLF_BIG_BWD_W(false, true);
 #undef CLF_BIG_BWD_W
+    });
 }
 
 int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
@@ -762,12 +865,11 @@ int rep32_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, co
     if (!big_split(n, neg, nul, c) || !big_table(n, neg, nul, c, T))
         return set_error(CLF_ERR_UNSUPPORTED, "signature has no 32 x 32 base");
     hipStream_t s = (hipStream_t)stream;
-    const dim3 grid(big_grid(c.k, batch));
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 4.0 * (double)(1LL << n) * (double)batch);
 #define CLF_BIG_BWD(K, D)                                                                          \
     do {                                                                                           \
-        if (nt) launch_rep32_bwd<K, D, true>(grid, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);  \
-        else launch_rep32_bwd<K, D, false>(grid, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);    \
+        if (nt) launch_rep32_bwd<K, D, true>(n, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);  \
+        else launch_rep32_bwd<K, D, false>(n, s, a, lda, b, ldb, gc, ldg, ga, gb, batch, T);    \
     } while (0)
     CLF_BIG_SWITCH(CLF_BIG_BWD)
 #undef CLF_BIG_BWD
