@@ -21,11 +21,17 @@
 // The combinations of parts are taken before the shuffles.
 //
 // Layout, LDS slots and relayout as in rep.hip (four rows per wave, one group
-// per wave). Bound: 12 and 20 KB a row over HBM against 1024 / 2048 matrix-core
-// cycles and about 400 / 800 VALU instructions per four rows.
+// per wave). Rows that are not of one scale are formed term by term in the same
+// launch (geom_terms.h).
+//
+// Bound: 3 and 5 KB a row over HBM, 1024 / 2048 matrix-core cycles and about 500 /
+// 960 vector instructions per four rows (the scale test is 100 / 160 of them).
+// Measured (us, forward + backward, 50001 N(0, 1) rows): Cl(7,1) 31 + 59 (27 + 53
+// without the test; the per-term kernels 91 + 170), Cl(7,0,1) 30 + 55 (28 + 49;
+// 78 + 150); rows that all go by their terms 150 + 240 and 118 + 205.
 #include <mutex>
 
-#include "rep_common.h"
+#include "geom_terms.h"
 
 namespace clf {
 
@@ -33,7 +39,78 @@ struct TwistTable {
     RepTable rep;   // entries of part 0, then of part 1
     float lambda;   // e_s^2 over its square in the representation
     int d;          // u^2 = -1
+    int s;          // e_s
+    TermSpec terms; // for the rows that are not of one scale
 };
+
+// Which of a wave's rows are not of one scale (geom_terms.h), bit j for row j.
+// With e_s null the result's part without e_s is a0 b0 alone, so each part of a
+// row has to hold its share of large coefficients.
+__device__ __forceinline__ unsigned twist_uneven(const Pre16& p, const TwistTable& T, int lane) {
+    // sums of squares, row j's total in the lanes 16j .. 16j + 15
+    float q0 = sumsq4(p.v[0]), q1 = sumsq4(p.v[1]), q2 = sumsq4(p.v[2]), q3 = sumsq4(p.v[3]);
+    permlane_swap32(q0, q2);
+    permlane_swap32(q1, q3);
+    float u = q0 + q2, v = q1 + q3;
+    permlane_swap16(u, v);
+    const float q = row16_sum(u + v);
+    const unsigned long long ranged = __ballot(even_range(q));
+    const unsigned level = __float_as_uint(even_level(q, 8));
+    unsigned bad = 0;
+    if (T.lambda != 0.f) {  // uniform
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (!even_count(even_large(p.v[j], __uint_as_float(__builtin_amdgcn_readlane(level, 16 * j))), 256))
+                bad |= 1u << j;
+    } else {
+        // the lanes (s >= 2) or components that hold blades with e_s
+        const unsigned long long with = T.s < 2 ? 0ull : __ballot((lane >> (T.s - 2)) & 1);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float lev = __uint_as_float(__builtin_amdgcn_readlane(level, 16 * j));
+            const float c[4] = {p.v[j].x, p.v[j].y, p.v[j].z, p.v[j].w};
+            int all = 0, part = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const unsigned long long large = __ballot(__builtin_fabsf(c[k]) >= lev);
+                all += __popcll(large);
+                part += __popcll(large & (T.s >= 2 ? with : (k >> T.s) & 1 ? ~0ull : 0ull));
+            }
+            if (!even_count(part, 128) || !even_count(all - part, 128)) bad |= 1u << j;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (!((ranged >> (16 * j)) & 1ull)) bad |= 1u << j;
+    return bad;
+}
+
+// store16 for the rows that are not in `bad`
+template <bool NT>
+__device__ __forceinline__ void twist_store(float* __restrict__ dst, const float* __restrict__ src, long long row0,
+                                            long long batch, int lane, unsigned oddc, unsigned bad) {
+    float4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const float4*>(src + j * 256)[(j & 1) ? (lane ^ oddc) : lane];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (row0 + j >= batch || ((bad >> j) & 1u)) continue;  // uniform
+        float4* q = reinterpret_cast<float4*>(dst + ((row0 + j) << 8)) + lane;
+        if (NT) store_stream(q, v[j]);
+        else *q = v[j];
+    }
+}
+
+// the rows of `bad` by their terms, a block per lane of the row's sixteen
+template <int MODE>
+__device__ __forceinline__ void twist_terms(const float* __restrict__ X, long long ldx, const float* __restrict__ Y,
+                                            long long ldy, float* __restrict__ out, long long row0, long long batch,
+                                            int lane, unsigned bad, const TermSpec& t) {
+    const long long row = row0 + (lane >> 4);
+    if (row >= batch || !((bad >> (lane >> 4)) & 1u)) return;
+    term_block<MODE>(X + ((row & row_mask(ldx)) << 8), Y + ((row & row_mask(ldy)) << 8), out + (row << 8),
+                     lane & 15u, t);
+}
 
 __device__ __forceinline__ void wht8(const float (&t)[16], int half, float (&v)[8]) {
 #pragma unroll
@@ -128,29 +205,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void t
     unsigned ent[16];
 #pragma unroll
     for (int z = 0; z < 16; ++z) ent[z] = T.rep.e[x * 16 + z] ^ oddx;
-    const long long stride = (long long)gridDim.x * 16;
-    for (long long row0 = ((long long)blockIdx.x * 4 + wave) * 4; row0 < batch; row0 += stride) {
-        const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
-        const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
-#pragma unroll
-        for (int z = 0; z < 16; ++z) asm volatile("" : "+v"(ent[z]));  // addresses re-derived where they are used
-        stage16(sa, pa, lane, oddc);
-        stage16(sb, pb, lane, oddc);
-        wave_lds_sync();
-        const Parts a = twist_convert<0>(sa + rb * 256, ent);
-        const Parts b = twist_convert<1>(sb + rb * 256, ent);
-        wave_lds_sync();
-        const floatx16 acc = twist_products(a, b, 1.f, 1.f, 1.f, T.lambda, sigma);
-        relayout_store(sa, acc, lane);
-        wave_lds_sync();
-        float wc[16];
-        relayout_load(sa, rb, x, wc);
-        wave_lds_sync();
-        twist_unconvert(wc, rho, sb + rb * 256, ent);
-        wave_lds_sync();
-        store16<NT>(C, sb, row0, batch, lane, oddc);
-        wave_lds_sync();
-    }
+    const long long row0 = ((long long)blockIdx.x * 4 + wave) * 4;
+    if (row0 >= batch) return;  // whole waves; no barrier follows
+    const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
+    const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
+    stage16(sa, pa, lane, oddc);
+    stage16(sb, pb, lane, oddc);
+    wave_lds_sync();
+    const Parts a = twist_convert<0>(sa + rb * 256, ent);
+    const Parts b = twist_convert<1>(sb + rb * 256, ent);
+    const unsigned bad = twist_uneven(pa, T, lane) | twist_uneven(pb, T, lane);
+    wave_lds_sync();
+    const floatx16 acc = twist_products(a, b, 1.f, 1.f, 1.f, T.lambda, sigma);
+    relayout_store(sa, acc, lane);
+    wave_lds_sync();
+    float wc[16];
+    relayout_load(sa, rb, x, wc);
+    wave_lds_sync();
+    twist_unconvert(wc, rho, sb + rb * 256, ent);
+    wave_lds_sync();
+    twist_store<NT>(C, sb, row0, batch, lane, oddc, bad);
+    if (bad) twist_terms<TERM_C>(A, lda, B, ldb, C, row0, batch, lane, bad, T.terms);
 }
 
 template <bool NT, bool WA, bool WB>
@@ -170,46 +245,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     unsigned ent[16];
 #pragma unroll
     for (int z = 0; z < 16; ++z) ent[z] = T.rep.e[x * 16 + z] ^ oddx;
-    const long long stride = (long long)gridDim.x * 16;
-    for (long long row0 = ((long long)blockIdx.x * 4 + wave) * 4; row0 < batch; row0 += stride) {
-        const Pre16 pg = fetch16<NT>(GC, row0, batch, lane, ldg);
-        const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
-#pragma unroll
-        for (int z = 0; z < 16; ++z) asm volatile("" : "+v"(ent[z]));
-        stage16(s0, pg, lane, oddc);
-        if (WA) stage16(s1, pb, lane, oddc);
-        const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
+    const long long row0 = ((long long)blockIdx.x * 4 + wave) * 4;
+    if (row0 >= batch) return;  // whole waves; no barrier follows
+    const Pre16 pg = fetch16<NT>(GC, row0, batch, lane, ldg);
+    const Pre16 pb = fetch16<NT>(B, row0, batch, lane, ldb);
+    stage16(s0, pg, lane, oddc);
+    if (WA) stage16(s1, pb, lane, oddc);
+    const Pre16 pa = fetch16<NT>(A, row0, batch, lane, lda);
+    const unsigned bad_g = twist_uneven(pg, T, lane);
+    const unsigned bad_a = WA ? bad_g | twist_uneven(pb, T, lane) : 0u;  // ga's rows by terms
+    wave_lds_sync();
+    if (WA && bad_a != 15u) {
+        const Parts g = twist_convert<0>(s0 + rb * 256, ent);
+        const Parts b = twist_convert<0>(s1 + rb * 256, ent);
+        const floatx16 acc = twist_products(g, b, 1.f, T.lambda, 1.f, 1.f, sigma);
+        relayout_store(sr, acc, lane);
         wave_lds_sync();
-        if (WA) {
-            const Parts g = twist_convert<0>(s0 + rb * 256, ent);
-            const Parts b = twist_convert<0>(s1 + rb * 256, ent);
-            const floatx16 acc = twist_products(g, b, 1.f, T.lambda, 1.f, 1.f, sigma);
-            relayout_store(sr, acc, lane);
-            wave_lds_sync();
-            float w[16];
-            relayout_load(sr, rb, x, w);
-            wave_lds_sync();
-            twist_unconvert(w, rho, sr + rb * 256, ent);
-        }
+        float w[16];
+        relayout_load(sr, rb, x, w);
         wave_lds_sync();
-        if (WB) stage16(s1, pa, lane, oddc);
-        if (WA) store16<NT>(GA, sr, row0, batch, lane, oddc);
-        wave_lds_sync();
-        if (WB) {
-            const Parts a = twist_convert<1>(s1 + rb * 256, ent);
-            const Parts g = twist_convert<1>(s0 + rb * 256, ent);
-            const floatx16 acc = twist_products(a, g, 1.f, 1.f, T.lambda, 1.f, sigma);
-            relayout_store(sr, acc, lane);
-            wave_lds_sync();
-            float w[16];
-            relayout_load(sr, rb, x, w);
-            wave_lds_sync();
-            twist_unconvert(w, rho, sr + rb * 256, ent);
-            wave_lds_sync();
-            store16<NT>(GB, sr, row0, batch, lane, oddc);
-        }
-        wave_lds_sync();
+        twist_unconvert(w, rho, sr + rb * 256, ent);
     }
+    wave_lds_sync();
+    const unsigned bad_b = WB ? bad_g | twist_uneven(pa, T, lane) : 0u;
+    if (WB) stage16(s1, pa, lane, oddc);
+    if (WA) twist_store<NT>(GA, sr, row0, batch, lane, oddc, bad_a);
+    wave_lds_sync();
+    if (WB && bad_b != 15u) {
+        const Parts a = twist_convert<1>(s1 + rb * 256, ent);
+        const Parts g = twist_convert<1>(s0 + rb * 256, ent);
+        const floatx16 acc = twist_products(a, g, 1.f, 1.f, T.lambda, 1.f, sigma);
+        relayout_store(sr, acc, lane);
+        wave_lds_sync();
+        float w[16];
+        relayout_load(sr, rb, x, w);
+        wave_lds_sync();
+        twist_unconvert(w, rho, sr + rb * 256, ent);
+        wave_lds_sync();
+        twist_store<NT>(GB, sr, row0, batch, lane, oddc, bad_b);
+    }
+    if (WA && bad_a) twist_terms<TERM_GA>(B, ldb, GC, ldg, GA, row0, batch, lane, bad_a, T.terms);
+    if (WB && bad_b) twist_terms<TERM_GB>(A, lda, GC, ldg, GB, row0, batch, lane, bad_b, T.terms);
 }
 
 // ---- host side --------------------------------------------------------------
@@ -307,7 +383,8 @@ bool twist_build(uint32_t neg, uint32_t nul, TwistTable& T) {
         T.rep.e[x * 16 + slot] = I | (negsign ? 0x80000000u : 0u) | (tsign ? 0x40000000u : 0u);
     }
     rep16_odd_xor(T.rep);
-    return true;
+    T.s = s;
+    return term_spec(kTwistN, neg, nul, T.terms);
 }
 
 }  // namespace
@@ -327,10 +404,15 @@ bool twist_applicable(uint32_t neg, uint32_t nul) {
     return twist_table(neg, nul, T);
 }
 
-// One workgroup per 16 rows; the cap only bounds the grid dimension.
-static dim3 twist_grid(int64_t batch) {
-    const long long g = (batch + 15) / 16;
-    return dim3((unsigned)(g < (1LL << 24) ? g : (1LL << 24)));
+// One workgroup per 16 rows, at most 2^22 in a launch (well inside the 2^32
+// work-items of one launch dimension); launch(r0, rows, grid) for each chunk.
+template <class Launch>
+static void twist_chunks(int64_t batch, Launch&& launch) {
+    const int64_t most = 16LL << 22;
+    for (int64_t r0 = 0; r0 < batch; r0 += most) {
+        const int64_t rows = batch - r0 < most ? batch - r0 : most;
+        launch(r0, rows, dim3((unsigned)((rows + 15) / 16)));
+    }
 }
 
 int twist_fwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
@@ -338,12 +420,17 @@ int twist_fwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const flo
     TwistTable T;
     if (!twist_table(neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature is not one generator from M_16(R)");
     hipStream_t s = (hipStream_t)stream;
-    if (stream_nt(3.0 * 1024.0 * (double)batch))
-        hipLaunchKernelGGL((twist16_fwd_kernel<true>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b,
-                           (long long)ldb, c, (long long)batch, T);
-    else
-        hipLaunchKernelGGL((twist16_fwd_kernel<false>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b,
-                           (long long)ldb, c, (long long)batch, T);
+    const bool nt = stream_nt(3.0 * 1024.0 * (double)batch);
+    twist_chunks(batch, [&](int64_t r0, int64_t rows, dim3 grid) {
+        const int64_t off = r0 << kTwistN;
+        const float *ar = a + (lda ? off : 0), *br = b + (ldb ? off : 0);
+        if (nt)
+            hipLaunchKernelGGL((twist16_fwd_kernel<true>), grid, dim3(256), 0, s, ar, (long long)lda, br,
+                               (long long)ldb, c + off, (long long)rows, T);
+        else
+            hipLaunchKernelGGL((twist16_fwd_kernel<false>), grid, dim3(256), 0, s, ar, (long long)lda, br,
+                               (long long)ldb, c + off, (long long)rows, T);
+    });
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
@@ -354,19 +441,24 @@ int twist_bwd(uint32_t neg, uint32_t nul, const float* a, int64_t lda, const flo
     if (!twist_table(neg, nul, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature is not one generator from M_16(R)");
     hipStream_t s = (hipStream_t)stream;
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 1024.0 * (double)batch);
-#define CLF_TWIST_BWD2(NT, WA, WB)                                                                               \
-    hipLaunchKernelGGL((twist16_bwd_kernel<NT, WA, WB>), twist_grid(batch), dim3(256), 0, s, a, (long long)lda, b, \
-                       (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
-#define CLF_TWIST_BWD(WA, WB)                \
-    do {                                     \
+    twist_chunks(batch, [&](int64_t r0, int64_t rows, dim3 grid) {
+        const int64_t off = r0 << kTwistN;
+        const float *ar = a + (lda ? off : 0), *br = b + (ldb ? off : 0), *gr = gc + (ldg ? off : 0);
+        float *gar = ga ? ga + off : nullptr, *gbr = gb ? gb + off : nullptr;
+#define CLF_TWIST_BWD2(NT, WA, WB)                                                                       \
+    hipLaunchKernelGGL((twist16_bwd_kernel<NT, WA, WB>), grid, dim3(256), 0, s, ar, (long long)lda, br,   \
+                       (long long)ldb, gr, (long long)ldg, gar, gbr, (long long)rows, T)
+#define CLF_TWIST_BWD(WA, WB)                  \
+    do {                                       \
         if (nt) CLF_TWIST_BWD2(true, WA, WB);  \
         else CLF_TWIST_BWD2(false, WA, WB);    \
     } while (0)
-    if (ga && gb) CLF_TWIST_BWD(true, true);
-    else if (ga) CLF_TWIST_BWD(true, false);
-    else if (gb) CLF_TWIST_BWD(false, true);
+        if (ga && gb) CLF_TWIST_BWD(true, true);
+        else if (ga) CLF_TWIST_BWD(true, false);
+        else if (gb) CLF_TWIST_BWD(false, true);
 #undef CLF_TWIST_BWD
 #undef CLF_TWIST_BWD2
+    });
     CLF_HIP_CHECK(hipGetLastError());
     return CLF_OK;
 }
