@@ -383,13 +383,16 @@ static size_t rows_ws_floats(int n, int64_t batch) {
 }
 
 // GEMMs against the per-row kernels (us, forward + backward): n = 7, 120000
-// rows: geom 48 + 225 -> 27 + 76, wedge 46 + 224 -> 24 + 82, inner 46 + 223 ->
-// 31 + 90; n = 8, 60013 rows: wedge 75 + 238 -> 38 + 110, inner 74 + 239 ->
-// 52 + 122, Cl(7,1) geom 83 + 253 -> 26 + 80, and at 2000 rows inner 26 + 185
-// -> 8 + 29; n = 9, 20000 rows: geom 117 + 290 -> 25 + 88, inner 105 + 267 ->
-// 46 + 141; n = 10, 4096 rows: geom 93 + 257 -> 11 + 38, inner 94 + 257 ->
-// 31 + 109 (before column_total_kernel's loads in flight, 5 to 10 less since).
-// No form measured slower at any batch. The backward is bound by
+// rows: wedge 46 + 224 -> 24 + 82, inner 46 + 223 -> 31 + 90; n = 8, 60013 rows:
+// wedge 75 + 238 -> 38 + 110, inner 74 + 239 -> 52 + 122, and at 2000 rows inner
+// 26 + 185 -> 8 + 29; n = 9, 20000 rows: inner 105 + 267 -> 46 + 141; n = 10, 4096
+// rows: inner 94 + 257 -> 31 + 109 (before column_total_kernel's loads in flight,
+// 5 to 10 less since). Geometric product, N(0, 1) rows: Cl(7,0) 47 + 220 -> 34 + 86,
+// Cl(6,1) 45 + 218 -> 44 + 100, Cl(7,1) 78 + 240 -> 29 + 83, Cl(9,0) 105 + 268 ->
+// 36 + 91, Cl(9,0,1) 93 + 258 -> 23 + 51, Cl(10,0) 95 + 259 -> 12 + 32. Where x is
+// not of one scale the forward and the weight gradient go by their terms: 111 + 151,
+// 100 + 160, 127 + 172, 139 + 228, 91 + 144, 106 + 145, faster than the GEMMs as a
+// training step except at Cl(9,0) (even). The backward is bound by
 // writing and reading back the per-row weight gradients beside x, gy and gx.
 static bool use_rows(int op, int n, uint32_t neg, uint32_t nul) { return product_has_form(op, n, neg, nul); }
 

@@ -193,11 +193,11 @@ __device__ __forceinline__ void term_pair(float (&acc)[16], const float (&x)[16]
 // generator takes away is passed over. The lanes of a wave may share a block: 2^log
 // of them (log <= 4), whose numbers differ in the lane's top bits, take every
 // 2^log-th pair each (from `slice` on), and the first stores the sum; all lanes
-// of the wave are then active, with a block each.
+// of the wave are then active, with a block each, and may leave it unstored.
 template <int MODE, bool FRONT>
 __device__ __forceinline__ void term_block_of(const float* __restrict__ X, const float* __restrict__ Y,
                                               float* __restrict__ out, unsigned h, const TermSpec& t, unsigned slice,
-                                              int log) {
+                                              int log, bool keep) {
     float acc[16];
 #pragma unroll
     for (int l = 0; l < 16; ++l) acc[l] = 0.f;
@@ -228,7 +228,7 @@ __device__ __forceinline__ void term_block_of(const float* __restrict__ X, const
     if (log >= 2) term_add(acc, [](float v) { return swap16_sum(v); });
     if (log >= 3) term_add(acc, [](float v) { return v + xor16<8>(v); });
     if (log >= 4) term_add(acc, [](float v) { return v + xor16<4>(v); });
-    if (slice != 0u) return;
+    if (slice != 0u || !keep) return;
     const unsigned ph = term_place<FRONT>(h, t);
     if (!FRONT) term_flip(acc, term_chi(ph, t), 0u);
     term_store<FRONT>(out, ph, t, acc);
@@ -237,9 +237,9 @@ __device__ __forceinline__ void term_block_of(const float* __restrict__ X, const
 template <int MODE>
 __device__ __forceinline__ void term_block(const float* __restrict__ X, const float* __restrict__ Y,
                                            float* __restrict__ out, unsigned h, const TermSpec& t, unsigned slice = 0,
-                                           int log = 0) {
-    if (t.front) term_block_of<MODE, true>(X, Y, out, h, t, slice, log);  // uniform
-    else term_block_of<MODE, false>(X, Y, out, h, t, slice, log);
+                                           int log = 0, bool keep = true) {
+    if (t.front) term_block_of<MODE, true>(X, Y, out, h, t, slice, log, keep);  // uniform
+    else term_block_of<MODE, false>(X, Y, out, h, t, slice, log, keep);
 }
 
 // ---- coefficients of one scale -------------------------------------------------

@@ -750,16 +750,14 @@ bool rep_table(int n, uint32_t neg, RepTable& T) {
 
 bool split_applicable(int op, int n, uint32_t neg, uint32_t nul);
 bool rep7_applicable(uint32_t neg);
-// lda, ldb of the functions below: 0 if a / b is one row read for every batch
-// row, nonzero: packed rows
+// lda, ldb: 0 if a / b is one row read for every batch row, nonzero: packed rows
 int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
              void* stream);
 int rep7_bwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc, int64_t ldg,
              float* ga, float* gb, int64_t batch, void* stream);
-int split_fwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
-              void* stream);
-int split_bwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc,
-              int64_t ldg, float* ga, float* gb, int64_t batch, void* stream);
+int split_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream);
+int split_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
+              float* gb, int64_t batch, void* stream);
 
 bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul);
 int rep32_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
@@ -816,10 +814,16 @@ static long long rep16_bwd_blocks(int64_t batch) {
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 
-// (real-type n <= 8 takes packed rows only; its broadcast form is rep_bcast_fwd)
+// Real-type n <= 8 takes packed rows only (its broadcast form is rep_bcast_fwd),
+// and so does the split form: a layer of such a signature runs rep32, which forms
+// rows that are not of one scale term by term, as the layers' GEMMs did for every row.
+static bool use_split(int n, uint32_t neg, uint32_t nul, int64_t lda, int64_t ldb) {
+    return lda && ldb && split_applicable(CLF_OP_GEOM, n, neg, nul);
+}
+
 int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb, float* c,
             int64_t batch, void* stream) {
-    if (split_applicable(CLF_OP_GEOM, n, neg, nul)) return split_fwd(n, neg, a, lda, b, ldb, c, batch, stream);
+    if (use_split(n, neg, nul, lda, ldb)) return split_fwd(n, neg, a, b, c, batch, stream);
     if (n >= 9) return rep32_fwd(n, neg, nul, a, lda, b, ldb, c, batch, stream);
     if (n == 7) return rep7_fwd(neg, a, lda, b, ldb, c, batch, stream);
     RepTable T;
@@ -858,8 +862,7 @@ int rep_fwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, cons
 
 int rep_bwd(int n, uint32_t neg, uint32_t nul, const float* a, int64_t lda, const float* b, int64_t ldb,
             const float* gc, int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
-    if (split_applicable(CLF_OP_GEOM, n, neg, nul))
-        return split_bwd(n, neg, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
+    if (use_split(n, neg, nul, lda, ldb)) return split_bwd(n, neg, a, b, gc, ldg, ga, gb, batch, stream);
     if (n >= 9) return rep32_bwd(n, neg, nul, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
     if (n == 7) return rep7_bwd(neg, a, lda, b, ldb, gc, ldg, ga, gb, batch, stream);
     RepTable T;

@@ -28,12 +28,14 @@
 // stages them in its LDS slots, converts (lane = x), multiplies with the
 // 4-block 16x16x1 MFMA chain of rep_common.h (block b = row b), and brings the
 // products back through the stride-20 relayout. Waves walk the batch with a
-// grid stride and prefetch the next rows into registers.
+// grid stride and prefetch the next rows into registers. A layer's launch takes
+// one group per wave and forms rows that are not of one scale term by term
+// (geom_terms.h; 120000 rows 28 -> 34 us forward for the test).
 #include <algorithm>
 #include <map>
 #include <mutex>
 
-#include "rep_common.h"
+#include "geom_terms.h"
 
 namespace clf {
 
@@ -47,6 +49,7 @@ struct Rep7Table {
     unsigned e[16 * 8];
     unsigned zhi[16];  // high z bits of lane x's labels
     unsigned odd_xor;  // multiple of 4 xor-ed into odd rows' blade offsets in LDS
+    TermSpec terms;    // for a layer's rows that are not of one scale
 };
 
 // Four rows: lane l moves float4 chunks l and l + 64 of the group (row c >> 5);
@@ -98,6 +101,49 @@ __device__ __forceinline__ void store7(float* __restrict__ dstg, const float* __
         if (NT) store_stream(q, v[j]);
         else *q = v[j];
     }
+}
+
+// Which of a wave's rows are not of one scale (geom_terms.h), bit r for row r
+__device__ __forceinline__ unsigned uneven7(const Pre7& p) {
+    unsigned bad = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const float q = swap16_sum(row16_sum(sumsq4(p.v[j])));  // of the half-wave, one row
+        const float level = even_level(q, 7);
+        const unsigned long long ranged = __ballot(even_range(q));
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            if (!even_count(even_large(p.v[j], level, 0xffffffffull << (32 * r)), 128) || !((ranged >> (32 * r)) & 1ull))
+                bad |= 1u << (2 * j + r);
+    }
+    return bad;
+}
+
+// store7 for the rows that are not in `bad`
+template <bool NT>
+__device__ __forceinline__ void store7_even(float* __restrict__ dstg, const float* __restrict__ src, long long row0,
+                                            long long batch, int lane, unsigned oddc, unsigned bad) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int c = lane + 64 * j;
+        const float4 v = reinterpret_cast<const float4*>(src)[slot7(c, oddc)];
+        if (row0 + (c >> 5) >= batch || ((bad >> (c >> 5)) & 1u)) continue;
+        float4* q = reinterpret_cast<float4*>(dstg + (row0 + (c >> 5)) * kRep7Dim) + (c & 31);
+        if (NT) store_stream(q, v);
+        else *q = v;
+    }
+}
+
+// the rows of `bad` by their terms: eight blocks a row, two lanes to a block
+template <int MODE>
+__device__ __forceinline__ void terms7(const float* __restrict__ X, long long ldx, const float* __restrict__ Y,
+                                       long long ldy, float* __restrict__ out, long long row0, long long batch,
+                                       int lane, unsigned bad, const TermSpec& t) {
+    const unsigned r = ((unsigned)lane >> 3) & 3u;
+    const bool live = row0 + r < batch;
+    const long long row = live ? row0 + r : batch - 1;
+    term_block<MODE>(X + ((row & row_mask(ldx)) << 7), Y + ((row & row_mask(ldy)) << 7), out + (row << 7), lane & 7u, t,
+                     (unsigned)lane >> 5, 1, live && ((bad >> r) & 1u));
 }
 
 __device__ __forceinline__ float sgn7(float v, unsigned e, int shift) {
@@ -254,10 +300,13 @@ __device__ __forceinline__ void product_q7(float* __restrict__ rel, const float 
 // index is wave-uniform, so the row bookkeeping runs on the scalar unit.
 // ONE: the grid covers the batch (one group per wave), so no next group is
 // prefetched (the same in the backward)
-template <bool PAIR, bool NT, bool ONE>
-__global__ __launch_bounds__(256) void rep7_fwd_kernel(
-    const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
+// SCALES (with ONE; the layers, whose rows the GEMMs summed term by term before):
+// rows that are not of one scale are formed term by term
+template <bool PAIR, bool NT, bool ONE, bool SCALES = false>
+__global__ __launch_bounds__(256) void rep7_fwd_kernel(const float* __restrict__ A, long long lda,
+                                                        const float* __restrict__ B, long long ldb,
                                                         float* __restrict__ C, long long batch, Rep7Table T) {
+    static_assert(ONE || !SCALES, "one group per wave");
     constexpr int D = PAIR ? 2 : 3;
     // per wave: staged a | b, later the relayout (over both), then c in the b
     // slot until the next group's stores
@@ -290,6 +339,8 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(
             pa = fetch7<NT>(A, row0 + stride, batch, lane, lda);
             pb = fetch7<NT>(B, row0 + stride, batch, lane, ldb);
         }
+        unsigned bad = 0;
+        if (SCALES) bad = uneven7(pa) | uneven7(pb);
         wave_lds_sync();
         if constexpr (PAIR) {
             float ta[4], tah[4], tb[4], tbh[4];
@@ -310,6 +361,11 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(
             scatter7_single(sb + rb * kRep7Dim, ent, q);
         }
         wave_lds_sync();
+        if constexpr (SCALES) {
+            store7_even<NT>(C, sb, row0, batch, lane, oddc, bad);
+            if (bad) terms7<TERM_C>(A, lda, B, ldb, C, row0, batch, lane, bad, T.terms);
+            return;
+        }
     }
     if (row0 != rfirst) store7<NT>(C, sb, row0 - stride, batch, lane, oddc);
 }
@@ -319,11 +375,12 @@ __global__ __launch_bounds__(256) void rep7_fwd_kernel(
 // after the other: gc and b are staged first (a is loaded meanwhile), then a
 // over b, and each gradient's relayout and rows in blade order use a scratch
 // slot, so few converted operands are live at once.
-template <bool PAIR, bool NT, bool WA, bool WB, bool ONE>
+template <bool PAIR, bool NT, bool WA, bool WB, bool ONE, bool SCALES = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void rep7_bwd_kernel(
     const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
-    const float* __restrict__ GC, long long ldg,
-    float* __restrict__ GA, float* __restrict__ GB, long long batch, Rep7Table T) {
+    const float* __restrict__ GC, long long ldg, float* __restrict__ GA, float* __restrict__ GB, long long batch,
+    Rep7Table T) {
+    static_assert(ONE || !SCALES, "one group per wave");
     constexpr int D = PAIR ? 2 : 3;
     constexpr int L = 1 << D;
     __shared__ float lds[4][2 * kRep7GroupFloats + kRelayoutFloats];  // per wave: gc | b, then a | scratch
@@ -351,6 +408,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
         stage7(sg, pg, lane, oddc);
         stage7(sx, pb, lane, oddc);
         const Pre7 pa = fetch7<NT>(A, row0, batch, lane, lda);
+        unsigned bad_a = 0, bad_b = 0;  // ga's and gb's rows by terms
+        if (SCALES) {
+            bad_a = bad_b = uneven7(pg);
+            if (WA) bad_a |= uneven7(pb);
+            if (WB) bad_b |= uneven7(pa);
+        }
         // the previous group's gb leaves the scratch slot (stored after this wait)
         if (WB && row0 != rfirst) store7<NT>(GB, sr, row0 - stride, batch, lane, oddc);  // uniform
         wave_lds_sync();
@@ -377,7 +440,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
             pg = fetch7<NT>(GC, row0 + stride, batch, lane, ldg);
             pb = fetch7<NT>(B, row0 + stride, batch, lane, ldb);
         }
-        if (WA) store7<NT>(GA, sr, row0, batch, lane, oddc);  // after this group's second wait
+        // after this group's second wait
+        if (WA && SCALES) store7_even<NT>(GA, sr, row0, batch, lane, oddc, bad_a);
+        else if (WA) store7<NT>(GA, sr, row0, batch, lane, oddc);
         wave_lds_sync();
         if (WB) {
             float q[L];
@@ -397,6 +462,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void r
             }
         }
         wave_lds_sync();
+        if constexpr (SCALES) {
+            if (WB) store7_even<NT>(GB, sr, row0, batch, lane, oddc, bad_b);
+            if (WA && bad_a) terms7<TERM_GA>(B, ldb, GC, ldg, GA, row0, batch, lane, bad_a, T.terms);
+            if (WB && bad_b) terms7<TERM_GB>(A, lda, GC, ldg, GB, row0, batch, lane, bad_b, T.terms);
+            return;
+        }
     }
     if (WB && row0 != rfirst) store7<NT>(GB, sr, row0 - stride, batch, lane, oddc);
 }
@@ -550,7 +621,9 @@ static bool rep7_table_build(uint32_t neg, Rep7Table& T) {
 // Tables are built once per signature and kept (immutable after insertion).
 static bool rep7_table(uint32_t neg, Rep7Table& T) {
     static TableCache<Rep7Table, 128> cache;
-    return cache.get((int)(neg & 0x7fu), T, [&](Rep7Table& t) { return rep7_table_build(neg & 0x7fu, t); });
+    return cache.get((int)(neg & 0x7fu), T, [&](Rep7Table& t) {
+        return rep7_table_build(neg & 0x7fu, t) && term_spec(7, neg & 0x7fu, 0u, t.terms);
+    });
 }
 
 bool rep7_applicable(uint32_t neg) {
@@ -564,12 +637,22 @@ bool rep7_applicable(uint32_t neg) {
 // prefetch, 2048 or 4096 workgroups for C2's 65536 rows measured within 2 %.)
 static unsigned rep7_grid(int64_t batch) {
     const long long g = (batch + 15) / 16;
-    const long long cap = 1LL << 24;
+    const long long cap = 1LL << 22;  // well inside the 2^32 work-items of one launch dimension
     return (unsigned)(g < 1 ? 1 : (g > cap ? cap : g));
 }
 
+// A layer's launch (one operand is one row) takes one group per wave: rows past
+// the bound of a launch are another launch's.
+constexpr int64_t kRep7LayerRows = 16LL << 22;
+
 int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
              void* stream) {
+    const bool layer = !lda || !ldb;
+    if (layer && batch > kRep7LayerRows) {
+        const int64_t off = kRep7LayerRows * kRep7Dim;
+        if (int rc = rep7_fwd(neg, a, lda, b, ldb, c, kRep7LayerRows, stream)) return rc;
+        return rep7_fwd(neg, lda ? a + off : a, lda, ldb ? b + off : b, ldb, c + off, batch - kRep7LayerRows, stream);
+    }
     Rep7Table T;
     if (!rep7_table(neg & 0x7fu, T)) return set_error(CLF_ERR_UNSUPPORTED, "no n = 7 matrix representation found");
     const bool pair = (host_popc(neg & 0x7fu) & 1) != 0;
@@ -577,13 +660,14 @@ int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t 
     const dim3 g(rep7_grid(batch));
     const bool one = (long long)g.x * 16 >= batch;
     const bool nt = stream_nt(3.0 * 512.0 * (double)batch);
-#define CLF_REP7_FWD_ONE(P, NT, ONE)                                                                             \
-    hipLaunchKernelGGL((rep7_fwd_kernel<P, NT, ONE>), g, dim3(256), 0, s, a, (long long)lda, b, (long long)ldb, c, \
-                       (long long)batch, T)
-#define CLF_REP7_FWD(P, NT)                     \
-    do {                                        \
-        if (one) CLF_REP7_FWD_ONE(P, NT, true); \
-        else CLF_REP7_FWD_ONE(P, NT, false);    \
+#define CLF_REP7_FWD_ONE(P, NT, ONE, SCALES)                                                               \
+    hipLaunchKernelGGL((rep7_fwd_kernel<P, NT, ONE, SCALES>), g, dim3(256), 0, s, a, (long long)lda, b,     \
+                       (long long)ldb, c, (long long)batch, T)
+#define CLF_REP7_FWD(P, NT)                                  \
+    do {                                                     \
+        if (layer) CLF_REP7_FWD_ONE(P, NT, true, true);      \
+        else if (one) CLF_REP7_FWD_ONE(P, NT, true, false);  \
+        else CLF_REP7_FWD_ONE(P, NT, false, false);          \
     } while (0)
     if (pair) {
         if (nt) CLF_REP7_FWD(true, true);
@@ -600,6 +684,13 @@ int rep7_fwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t 
 
 int rep7_bwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc, int64_t ldg,
              float* ga, float* gb, int64_t batch, void* stream) {
+    const bool layer = !lda || !ldb;
+    if (layer && batch > kRep7LayerRows) {
+        const int64_t off = kRep7LayerRows * kRep7Dim;
+        if (int rc = rep7_bwd(neg, a, lda, b, ldb, gc, ldg, ga, gb, kRep7LayerRows, stream)) return rc;
+        return rep7_bwd(neg, lda ? a + off : a, lda, ldb ? b + off : b, ldb, ldg ? gc + off : gc, ldg,
+                        ga ? ga + off : ga, gb ? gb + off : gb, batch - kRep7LayerRows, stream);
+    }
     Rep7Table T;
     if (!rep7_table(neg & 0x7fu, T)) return set_error(CLF_ERR_UNSUPPORTED, "no n = 7 matrix representation found");
     const bool pair = (host_popc(neg & 0x7fu) & 1) != 0;
@@ -608,13 +699,14 @@ int rep7_bwd(uint32_t neg, const float* a, int64_t lda, const float* b, int64_t 
     const bool one = (long long)g.x * 16 >= batch;
     const bool nt = stream_nt((3 + (ga != nullptr) + (gb != nullptr)) * 512.0 * (double)batch);
     if (!ga && !gb) return CLF_OK;
-#define CLF_REP7_BWD_ONE(P, NT, WA, WB, ONE)                                                                  \
-    hipLaunchKernelGGL((rep7_bwd_kernel<P, NT, WA, WB, ONE>), g, dim3(256), 0, s, a, (long long)lda, b,        \
+#define CLF_REP7_BWD_ONE(P, NT, WA, WB, ONE, SCALES)                                                        \
+    hipLaunchKernelGGL((rep7_bwd_kernel<P, NT, WA, WB, ONE, SCALES>), g, dim3(256), 0, s, a, (long long)lda, b, \
                        (long long)ldb, gc, (long long)ldg, ga, gb, (long long)batch, T)
-#define CLF_REP7_BWD(P, NT, WA, WB)                     \
-    do {                                                \
-        if (one) CLF_REP7_BWD_ONE(P, NT, WA, WB, true); \
-        else CLF_REP7_BWD_ONE(P, NT, WA, WB, false);    \
+#define CLF_REP7_BWD(P, NT, WA, WB)                                  \
+    do {                                                             \
+        if (layer) CLF_REP7_BWD_ONE(P, NT, WA, WB, true, true);      \
+        else if (one) CLF_REP7_BWD_ONE(P, NT, WA, WB, true, false);  \
+        else CLF_REP7_BWD_ONE(P, NT, WA, WB, false, false);          \
     } while (0)
 #define CLF_REP7_BWD_W(P, NT)                 \
     do {                                      \

@@ -639,20 +639,18 @@ static void launch_fused(const SplitTable& T, const float* X, const float* Y, fl
     hipLaunchKernelGGL(split_fused_kernel<KIND>, grid, dim3(64 * kFusedWaves), 0, s, P, T);
 }
 
-int split_fwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, float* c, int64_t batch,
-              void* stream) {
+int split_fwd(int n, uint32_t neg, const float* a, const float* b, float* c, int64_t batch, void* stream) {
     SplitTable T;
     if (!split_table(neg & 511u, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no split representation");
     hipStream_t s = (hipStream_t)stream;
-    const long long la = lda ? 1LL << n : 0, lb = ldb ? 1LL << n : 0;
     if (n == 9) {
-        const PairSpec ab[1] = {{a, b, 0u, la, lb}};
+        const PairSpec ab[1] = {{a, b, 0u}};
         launch_pairs(T, ab, 1, 512, c, 512, batch, s);
     } else if (split_fused_enabled()) {
-        launch_fused<0>(T, a, b, c, batch, s, la, lb);
+        launch_fused<0>(T, a, b, c, batch, s);
     } else {
-        const PairSpec c0[1] = {{a, b, 0u, la, lb}};
-        const PairSpec c1[2] = {{a, b + 512, 0u, la, lb}, {a + 512, b, kHatY, la, lb}};
+        const PairSpec c0[1] = {{a, b, 0u}};
+        const PairSpec c1[2] = {{a, b + 512, 0u}, {a + 512, b, kHatY}};
         launch_pairs(T, c0, 1, 1024, c, 1024, batch, s);
         launch_pairs(T, c1, 2, 1024, c + 512, 1024, batch, s);
     }
@@ -661,35 +659,35 @@ int split_fwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, 
 }
 
 // gc's rows are ldg floats apart: 2^n, or 0 for one row broadcast over the batch
-int split_bwd(int n, uint32_t neg, const float* a, int64_t lda, const float* b, int64_t ldb, const float* gc,
-              int64_t ldg, float* ga, float* gb, int64_t batch, void* stream) {
+int split_bwd(int n, uint32_t neg, const float* a, const float* b, const float* gc, int64_t ldg, float* ga,
+              float* gb, int64_t batch, void* stream) {
     SplitTable T;
     if (!split_table(neg & 511u, T)) return set_error(CLF_ERR_UNSUPPORTED, "signature has no split representation");
     hipStream_t s = (hipStream_t)stream;
-    const long long lg = (long long)ldg, la = lda ? 1LL << n : 0, lb = ldb ? 1LL << n : 0;
+    const long long lg = (long long)ldg;
     if (n == 9) {
         if (ga) {
-            const PairSpec p[1] = {{gc, b, kTransB, lg, lb}};
+            const PairSpec p[1] = {{gc, b, kTransB, lg, -1}};
             launch_pairs(T, p, 1, 512, ga, 512, batch, s);
         }
         if (gb) {
-            const PairSpec p[1] = {{a, gc, kTransA, la, lg}};
+            const PairSpec p[1] = {{a, gc, kTransA, -1, lg}};
             launch_pairs(T, p, 1, 512, gb, 512, batch, s);
         }
     } else if (split_fused_enabled()) {
-        if (ga) launch_fused<1>(T, gc, b, ga, batch, s, lg, lb);
-        if (gb) launch_fused<2>(T, a, gc, gb, batch, s, la, lg);
+        if (ga) launch_fused<1>(T, gc, b, ga, batch, s, lg, 1024);
+        if (gb) launch_fused<2>(T, a, gc, gb, batch, s, 1024, lg);
     } else {
         const float *L0 = a, *L1 = a + 512, *R0 = b, *R1 = b + 512, *G0 = gc, *G1 = gc + 512;
         if (ga) {
-            const PairSpec l0[2] = {{G0, R0, kTransB, lg, lb}, {G1, R1, kTransB, lg, lb}};
-            const PairSpec l1[1] = {{G1, R0, kTransB | kHatY, lg, lb}};
+            const PairSpec l0[2] = {{G0, R0, kTransB, lg, -1}, {G1, R1, kTransB, lg, -1}};
+            const PairSpec l1[1] = {{G1, R0, kTransB | kHatY, lg, -1}};
             launch_pairs(T, l0, 2, 1024, ga, 1024, batch, s);
             launch_pairs(T, l1, 1, 1024, ga + 512, 1024, batch, s);
         }
         if (gb) {
-            const PairSpec r0[2] = {{L0, G0, kTransA, la, lg}, {L1, G1, kTransA | kHatX | kHatY, la, lg}};
-            const PairSpec r1[1] = {{L0, G1, kTransA, la, lg}};
+            const PairSpec r0[2] = {{L0, G0, kTransA, -1, lg}, {L1, G1, kTransA | kHatX | kHatY, -1, lg}};
+            const PairSpec r1[1] = {{L0, G1, kTransA, -1, lg}};
             launch_pairs(T, r0, 2, 1024, gb, 1024, batch, s);
             launch_pairs(T, r1, 1, 1024, gb + 512, 1024, batch, s);
         }

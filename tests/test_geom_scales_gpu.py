@@ -143,3 +143,33 @@ def test_not_finite(m, value, clf_env):
     for u, v in zip(got, run()):
         assert torch.equal(u.isnan(), v.isnan()) and torch.equal(u.isinf(), v.isinf())
         assert torch.equal(u[u.isinf()], v[v.isinf()])
+
+
+@pytest.mark.parametrize("m", ["+" * 7, "+" * 6 + "-", "-+-+-+-", "+" * 7 + "-", "+" * 9, "+-" * 4 + "+", "+" * 8 + "-",
+                               "+" * 9 + "0", "-+" * 4 + "+0", "+" * 10])
+@pytest.mark.parametrize("side", [0, 1])
+def test_layers(m, side):
+    """A layer's value and gradients (weight one row of the batch's products):
+    the weight gradient sums batch * 2^n terms, the bar grows with their root."""
+    metric, n = signature(m), len(m)
+    count = 37
+    for kinds in (("graded", "near one", "dense"), ("vector", "dense", "near one"), ("share 0.6", "share 0.9", "dense"),
+                  ("dense", "dense", "graded"), ("dense", "dense", "dense")):
+        g = torch.Generator().manual_seed(n)
+        x, w, gy = rows(kinds[0], n, count, g), rows(kinds[1], n, 1, g), rows(kinds[2], n, count, g)
+        print(f"[case] layer scales {m} side={side} {kinds}", flush=True)
+        xd, wd = x.cuda().requires_grad_(), w.cuda().requires_grad_()
+        y = cc.bcast.bcast_product("geom", xd, wd, metric, side=side)
+        got = (y.detach(), *torch.autograd.grad(y, (xd, wd), gy.cuda()))
+        x64, w64 = x.double().requires_grad_(), w.double().requires_grad_()
+        a64, b64 = (x64, w64.expand_as(x64)) if side == 0 else (w64.expand_as(x64), x64)
+        y64 = O.einsum_product("geom", a64, b64, metric)
+        ref = (y64.detach(), *torch.autograd.grad(y64, (x64, w64), gy.double()))
+        X, W, G = x.cuda(), w.cuda().expand(count, -1), gy.cuda()
+        terms = (term_sums(metric, *((X, W) if side == 0 else (W, X)), "c"),
+                 term_sums(metric, W, G, "ga" if side == 0 else "gb"),
+                 term_sums(metric, X, G, "gb" if side == 0 else "ga").sum(0, keepdim=True))
+        for u, v, t, scale in zip(got, ref, terms, (1, 1, count ** 0.5)):
+            err = (u.double() - v.cuda()).abs()
+            assert bool((err[t == 0] == 0).all())
+            assert float((err / t.clamp_min(1e-300)).max()) <= scale * bar(n), kinds
