@@ -396,6 +396,14 @@ static size_t rows_ws_floats(int n, int64_t batch) {
 // writing and reading back the per-row weight gradients beside x, gy and gx.
 static bool use_rows(int op, int n, uint32_t neg, uint32_t nul) { return product_has_form(op, n, neg, nul); }
 
+// Whether this weight can be read by every row's product: aligned, and outside
+// the output, which the GEMMs write after they have taken the weight in whole.
+static bool rows_weight(int n, const float* w, const float* out, int64_t batch) {
+    const uintptr_t w0 = (uintptr_t)w, w1 = (uintptr_t)(w + ((size_t)1 << n));
+    const uintptr_t o0 = (uintptr_t)out, o1 = (uintptr_t)(out + ((size_t)batch << n));
+    return !(w0 & 15u) && (!out || w1 <= o0 || o1 <= w0);
+}
+
 static int rows_fwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* x, const float* w, float* y,
                     int64_t batch, void* stream) {
     return side == 0 ? product_fwd_ld(op, n, neg, nul, x, 1, w, 0, y, batch, stream)
@@ -476,7 +484,7 @@ int bcast_fwd(int op, int side, int n, uint32_t neg, uint32_t nul, const float* 
     if ((((uintptr_t)x) | ((uintptr_t)y) | ((uintptr_t)ws)) & 15u)
         return set_error(CLF_ERR_ARG, "pointers must be 16-byte aligned");
     if (rep_bcast_applicable(op, n, neg, nul)) return rep_bcast_fwd(side, n, neg, x, w, y, batch, stream);
-    if (use_rows(op, n, neg, nul) && !(((uintptr_t)w) & 15u))
+    if (use_rows(op, n, neg, nul) && rows_weight(n, w, y, batch))
         return rows_fwd(op, side, n, neg, nul, x, w, y, batch, stream);
     hipStream_t s = (hipStream_t)stream;
     const int D = 1 << n;
@@ -510,7 +518,7 @@ static int bcast_bwd_launch(int op, int side, int n, uint32_t neg, uint32_t nul,
                             int max_splits, void* stream) {
     if (rep_bcast_applicable(op, n, neg, nul))
         return rep_bcast_bwd(side, n, neg, x, w, gy, ldg, gx, gw, batch, ws, stream);
-    if (batch > 0 && use_rows(op, n, neg, nul) && !(((uintptr_t)w) & 15u))
+    if (batch > 0 && use_rows(op, n, neg, nul) && rows_weight(n, w, gx, batch))
         return rows_bwd(op, side, n, neg, nul, x, w, gy, ldg, gx, gw, batch, ws, stream);
     hipStream_t s = (hipStream_t)stream;
     const int D = 1 << n;
@@ -608,7 +616,7 @@ int bcast_bwd_noalloc(int op, int side, int n, uint32_t neg, uint32_t nul, const
     size_t need;
     if (rep_bcast_applicable(op, n, neg, nul)) {
         need = rep_bcast_ws_floats(batch) * sizeof(float);
-    } else if (use_rows(op, n, neg, nul)) {
+    } else if (use_rows(op, n, neg, nul) && rows_weight(n, w, gx, batch)) {
         need = rows_ws_floats(n, batch) * sizeof(float);
     } else {
         const int cap = noalloc_max_splits(n);

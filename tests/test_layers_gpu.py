@@ -221,3 +221,41 @@ def test_rows_path_edges(op, metric, rows, side):
     r0 = torch.autograd.grad(fn(x2, w2, metric).sum() if side == 0 else fn(w2, x2, metric).sum(), (x2, w2))
     assert rel_err(g0[0], r0[0]) <= TOL
     assert rel_err(g0[1], r0[1].double().sum(0, keepdim=True)) <= TOL
+
+
+@pytest.mark.parametrize("op,metric", [("wedge", (1,) * 8), ("geom", (1,) * 7), ("geom", (1,) * 10), ("lc", (1,) * 9)])
+@pytest.mark.parametrize("at", [0, 3])
+def test_weight_inside_the_output(op, metric, at):
+    """The C entry points take a weight that lies in the output's memory (row
+    `at` of it): the result is the one of a separate weight, forward and input
+    gradient, also without a workspace of the caller's."""
+    from cliffordcuda_amd import _lib
+    lib, code, n, rows = _lib.load(), O.OPS.index(op), len(metric), 77
+    D = 1 << n
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, gy, w = (torch.randn(r, D, device="cuda", generator=g) for r in (rows, rows, 1))
+    x1, w1 = x.clone().requires_grad_(), w.clone().requires_grad_()
+    y = bcast.bcast_product(op, x1, w1, metric)
+    gx, gw = torch.autograd.grad(y, (x1, w1), gy)
+    nbytes = lib.clf_product_bcast_ws_bytes(n, rows)
+    ws = torch.empty(nbytes // 4, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    neg = sum(1 << k for k, m in enumerate(metric) if m < 0)
+
+    def into(call):
+        out, got_w = torch.zeros(rows, D, device="cuda"), torch.empty(1, D, device="cuda")
+        out[at] = w[0]
+        torch.cuda.synchronize()
+        _lib.check(call(out.data_ptr(), out[at].data_ptr(), got_w.data_ptr()), "bcast")
+        return out, got_w
+
+    print(f"[case] weight inside the output op={op} metric={metric} at={at}", flush=True)
+    out, _ = into(lambda o, wp, _: lib.clf_product_bcast_fwd(code, 0, n, neg, 0, x.data_ptr(), wp, o, rows,
+                                                             ws.data_ptr(), nbytes, stream))
+    assert rel_err(out, y) <= TOL
+    out, got_w = into(lambda o, wp, q: lib.clf_product_bcast_bwd(code, 0, n, neg, 0, x.data_ptr(), wp, gy.data_ptr(), o,
+                                                                 q, rows, ws.data_ptr(), nbytes, stream))
+    assert rel_err(out, gx) <= TOL and rel_err(got_w, gw) <= TOL
+    out, got_w = into(lambda o, wp, q: lib.clf_product_bcast_bwd_noalloc(code, 0, n, neg, 0, x.data_ptr(), wp,
+                                                                         gy.data_ptr(), o, q, rows, stream))
+    assert rel_err(out, gx) <= TOL and rel_err(got_w, gw) <= TOL
