@@ -810,7 +810,7 @@ static long long rep_blocks(int n, int64_t batch) {
 // kernel's grid-stride loop covers any batch.
 static long long rep16_bwd_blocks(int64_t batch) {
     const long long g = (batch + 15) / 16;
-    const long long cap = 1LL << 24;
+    const long long cap = 1LL << 22;  // well inside the 2^32 work-items of one launch dimension
     return g < 1 ? 1 : (g > cap ? cap : g);
 }
 

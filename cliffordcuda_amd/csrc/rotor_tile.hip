@@ -501,7 +501,7 @@ template <int N>
 static void launch_tile(bool fwd, const float* cs, const float* x, float* y, int64_t batch, hipStream_t s,
                         long long ldx) {
     const long long per = tile_groups_per_block<N>();
-    const long long most = (1LL << 24) * per;  // rows of one launch
+    const long long most = (1LL << 22) * per;  // rows of one launch, well inside its 2^32 work-items
     const bool nt = stream_nt(2.0 * 4.0 * (double)(1LL << N) * (double)batch);
     for (long long r0 = 0; r0 < batch; r0 += most) {
         const long long rows = batch - r0 < most ? batch - r0 : most;
