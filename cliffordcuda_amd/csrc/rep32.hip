@@ -784,18 +784,19 @@ bool rep32_applicable(int op, int n, uint32_t neg, uint32_t nul) {
 
 // Rows up to which the small-batch per-term kernels are faster: a row's 2^K
 // waves of the 32 x 32 kernels are one dependent chain of 2^K products each,
-// the per-term kernels spread it over more workgroups. Forward + backward, us,
-// per-term against 32 x 32: n = 9, K = 1: 300 rows 6.4 + 9.0 against 6.9 + 10.2,
-// 1500 rows 25 + 45 against 10.2 + 17.7; n = 10, K = 1: 64 rows 5.7 + 7.7
-// against 6.7 + 9.5, 300 rows 10.8 + 19.3 against 7.2 + 9.9; n = 11, K = 1: 16
-// rows 5.4 + 9.1 against 6.0 + 9.9, 64 rows 10.2 + 18.9 against 6.3 + 10.2;
-// n = 11, K = 2: 64 rows 8.9 + 15.7 against 8.1 + 13.1; n = 12: 1 row 5.5 + 8.9
-// against 7.5 + 13.1, 16 rows 10.2 + 18.9 against 8.2 + 13.6. K = 0 has no such
-// rows (n = 10, 1 row: 4.9 + 7.6 against 4.2 + 6.2).
+// the per-term kernels spread it over more workgroups. Forward + backward on the
+// device, us, per-term against 32 x 32, N(0, 1) rows, on both sides of each line:
+// n = 9 (K = 1) 768 rows 21.6 against 22.4, 1024 rows 67 against 23 (Cl(8,0,1) 18.9
+// against 21.5, 68 against 22); n = 10 (K = 1) 128 rows 16.1 against 17.5, 192 rows
+// 22.1 against 17.1; n = 11, K = 1, 32 rows 17.1 against 17.8, 64 rows 28 against 18
+// (Cl(10,0,1) 16.7 against 17.9, 27 against 18); n = 11, K = 2, 32 rows 17.1 against
+// 22.6, 48 rows 23.9 against 22.6; n = 12, 8 rows 18.3 against 23.5, 16 rows 31
+// against 24 (Cl(10,0,2) 17.4 against 23.2, 28 against 23). K = 0 has no such rows
+// (n = 10, 1 row: 12.8 against 11.8).
 int64_t rep32_rows(int n, uint32_t neg, uint32_t nul) {
     BigSplit c;
     if (!big_split(n, neg, nul, c) || c.k == 0) return 0;
-    return n == 9 ? 512 : n == 10 ? 128 : n == 11 ? (c.k == 1 ? 16 : 32) : 4;
+    return n == 9 ? 768 : n == 10 ? 128 : n == 11 ? 32 : 8;
 }
 
 // M(K, D) for the (K, D) of c, one of big_split's

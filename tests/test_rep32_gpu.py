@@ -1,5 +1,5 @@
 """The geometric product of large algebras on 32 x 32 matrices: against the
-fp64 oracle at the edges of a workgroup's rows, and against the per-term
+fp64 oracle at the edges of a workgroup's rows, in every form, and against the per-term
 kernels over every form the rule accepts (signs in any order, ext generators of
 each square, a broadcast upstream gradient, one gradient only)."""
 import pytest
@@ -7,6 +7,7 @@ import torch
 
 import cliffordcuda_amd as cc
 from oracle import clifford_oracle as O
+from tests.test_rep32_model import FORMS
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-5  # normwise, as for every product: 3 sqrt(2^n) sums of fp32 terms stay below 1e-6
@@ -43,8 +44,11 @@ def gpu(metric, a, b, gc):
     return c.detach(), ga, gb
 
 
-@pytest.mark.parametrize("metric", [(1,) * 8 + (-1,), (-1,) * 2 + (1,) * 7, (1,) * 10, (1,) * 8 + (-1,) * 2,
-                                    (1,) * 10 + (-1,), (1,) * 8 + (-1,) * 3, (1,) * 12], ids=ids)
+# FORMS: one signature per (K, D) whose low generators have both squares, so that
+# no few rows go to the per-term kernels; of the others those with K > 0 do
+@pytest.mark.parametrize("metric", list(FORMS.values()) + [
+    (1,) * 8 + (-1,), (-1,) * 2 + (1,) * 7, (1,) * 10, (1,) * 8 + (-1,) * 2, (1,) * 10 + (-1,), (1,) * 8 + (-1,) * 3,
+    (1,) * 12], ids=ids)
 @pytest.mark.parametrize("batch", [1, 3, 5])
 def test_against_oracle(metric, batch):
     a, b, gc = inputs(batch, len(metric), 3 + batch)
@@ -58,7 +62,7 @@ def test_against_oracle(metric, batch):
 
 @pytest.mark.parametrize("metric", SIGNATURES, ids=ids)
 def test_equals_per_term_kernels(metric, clf_env):
-    rows = 515 if len(metric) == 9 else 131 if len(metric) == 10 else 33 + len(metric)  # past the few-rows rule
+    rows = 771 if len(metric) == 9 else 131 if len(metric) == 10 else 33 + len(metric)  # past the few-rows rule
     a, b, gc = inputs(rows, len(metric), 7)
     row = gc[:1].cuda().expand(rows, -1)  # the gradient of a weighted sum: batch stride 0
     got = gpu(metric, a, b, gc.cuda()) + gpu(metric, a, b, row)

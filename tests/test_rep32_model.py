@@ -131,6 +131,18 @@ def test_served_signatures():
     assert split((1,) * 10 + (0, 0))[0] == [10, 11] and split((1,) * 9 + (0,) * 3) is None
 
 
+# one signature per (ext generators K, dummies D), low generators of both squares
+FORMS = {(0, 1): (1, -1) + (1,) * 7, (1, 2): (1, -1, 1, 1, -1, 1, 1, 1, 1), (0, 0): (1, -1) * 5,
+         (1, 1): (1, -1, 1, 1, -1) + (1,) * 5, (1, 0): (-1, 1) * 4 + (1, 1, -1), (2, 1): (1, -1, 1) * 3 + (1, 1),
+         (2, 0): (1, 1, -1) * 4}
+
+
+def test_forms():
+    for (k, d), metric in FORMS.items():
+        ext, dressed = split(metric)
+        assert (len(ext), len(dressed) - len(metric)) == (k, d) and len(set(metric[:4])) == 2
+
+
 def word(r, p):
     return ((r ^ ((r >> 3) & 1)) << 5) ^ (p ^ ((r & 7) << 2))
 
