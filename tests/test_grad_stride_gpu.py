@@ -31,7 +31,8 @@ def _expanded(batch, n, seed):
 # (op, metric, CLF_* switches): each line lands on a different backward route
 PRODUCT_CASES = [
     ("geom", (1, 1, 0), {}),                                      # generic, n < 4
-    ("inner", (1, 1, 1, -1, 0), {}),                              # generic, mixed low metric
+    ("inner", (1, 1, 1, -1, 0), {}),                              # blocked, mixed low metric
+    ("inner", (1, 1, 1, -1, 0), {"CLF_PRODUCT_PATH": "generic"}),
     ("lc", (1,) * 5, {"CLF_PRODUCT_PATH": "generic"}),
     ("geom", (1,) * 5, {"CLF_PRODUCT_PATH": "balanced"}),
     ("geom", (1,) * 5, {}),                                       # blocked
@@ -40,7 +41,8 @@ PRODUCT_CASES = [
     ("regressive", (1,) * 6 + (-1,), {"CLF_PRODUCT_PATH": "blocked"}),
     ("geom", (1,) * 6 + (-1,), {}),                               # n = 7 matrix representation
     ("geom", (1,) * 6 + (-1,), {"CLF_GEOM_PATH": "direct"}),
-    ("geom", (1,) * 7 + (-1,), {}),                               # n = 8 matrix representation
+    ("geom", (1,) * 8, {}),                                       # n = 8 matrix representation
+    ("geom", (1,) * 7 + (-1,), {}),                               # n = 8, one generator from it
     ("inner", (1,) * 8, {}),                                      # balanced inner (two deals)
     ("rc", (1,) * 8, {}),
     ("geom", (1,) * 9, {}),                                       # n = 9 split representation
@@ -48,8 +50,10 @@ PRODUCT_CASES = [
     ("geom", (1,) * 9 + (0,), {"CLF_SPLIT_PATH": "pairs"}),
     ("lc", (1,) * 9 + (0,), {}),
     ("inner", (1,) * 9 + (0,), {}),
-    ("geom", (1,) * 12, {"CLF_PRODUCT_PATH": "blocked"}),         # blocked at n = 12
+    ("geom", (1,) * 12, {"CLF_PRODUCT_PATH": "blocked", "CLF_GEOM_PATH": "direct"}),  # blocked at n = 12
     ("geom", (1,) * 12, {}),                                      # small-batch split kernels
+    ("geom", (1, 1, -1) * 4, {}),                                 # 32 x 32 matrices, n = 12
+    ("geom", (1,) * 10, {}),                                      # and n = 10
     ("regressive", (1,) * 11, {}),
     ("inner", (1,) * 9 + (0,), {"CLF_PRODUCT_PATH": "split"}),
     ("wedge", (1,) * 12, {"CLF_PRODUCT_PATH": "tiled"}),

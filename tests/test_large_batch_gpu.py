@@ -1,8 +1,8 @@
 """64-bit row offsets: batches whose last rows start past float index 2**31
 (8 GiB per operand) on every kernel family of the hot path -- the Cl(8,0)
-matrix representation, the n = 7 representation, the split representation
-(n = 10 with a null generator), the balanced and blocked per-term kernels and
-the graded ops. Rows are independent, so the rows of the large batch (first,
+matrix representation and its one-generator extension, the n = 7 representation,
+the split representation (n = 10 with a null generator), the 32 x 32 one, the
+balanced and blocked per-term kernels and the graded ops. Rows are independent, so the rows of the large batch (first,
 middle and last ones) must equal, bit for bit, the same rows computed as a
 batch of their own, forward and backward."""
 import pytest
@@ -19,6 +19,9 @@ CASES = [
     ((1,) * 8, "left_contraction", None),  # balanced kernels
     ((1,) * 6 + (-1,), "geom_prod", None),  # n = 7 representation
     ((1,) * 9 + (0,), "geom_prod", None),  # split representation, fused kernels
+    ((1,) * 7 + (-1,), "geom_prod", None),  # n = 8, one generator from the representation
+    ((1,) * 10, "geom_prod", None),  # 32 x 32 matrices, a row per wave
+    ((1,) * 10 + (-1,), "geom_prod", None),  # two waves a row
 ]
 
 
@@ -72,11 +75,14 @@ def test_rows_past_2_31_floats(metric, op, path, clf_env):
     torch.cuda.empty_cache()
 
 
-# (layer class, metric): the Cl(8,0) representation layer, the GEMM layer path,
-# the rotor on the Cl(8,0) representation and the register plane-rotation chain
+# (layer class, metric): the Cl(8,0) representation layer, layers on the per-row
+# kernels, the GEMM layer path (low generators of both squares), the rotor on the
+# Cl(8,0) representation and on tiles of generators
 LAYER_CASES = [
     ("GeometricProductLayer", (1,) * 8),
     ("WedgeProductLayer", (1,) * 8),
+    ("GeometricProductLayer", (1,) * 7),
+    ("LeftContractionLayer", (1, -1) * 4),
     ("RotorLayer", (1,) * 7 + (-1,)),
     ("RotorLayer", (1,) * 9),
 ]

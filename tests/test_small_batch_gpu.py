@@ -77,7 +77,9 @@ def test_small_batch_parity_n12(op):
 def test_split_forced_equals_whole_row_kernels(op, clf_env):
     """CLF_PRODUCT_PATH=split at a ragged batch of 300 rows (n = 10), 37 rows
     (n = 11) and 129 rows (n = 9) against the balanced / whole-row kernels (=blocked), which the
-    oracle tests pin on their own."""
+    oracle tests pin on their own. (CLF_GEOM_PATH=direct: the geometric product's
+    matrix representations come before this switch.)"""
+    clf_env.setenv("CLF_GEOM_PATH", "direct")
     for metric, batch in (((1,) * 8 + (-1, 1), 300), ((1,) * 11, 37), ((1,) * 5 + (-1, 1, 1, 1), 129)):
         n = len(metric)
         a, b, gc = [t.cuda() for t in inputs(n, batch, 130 + n)]
@@ -120,6 +122,7 @@ def test_small_batch_forward_n8(op, metric, clf_env):
         c = cc.products.product(op, a.cuda(), b.cuda(), metric)
         c64 = O.einsum_product(op, a.double(), b.double(), metric)
         assert rel_err(c, c64) <= TOL
+    clf_env.setenv("CLF_GEOM_PATH", "direct")  # before the geometric product's matrix representations
     a, b, _ = [t.cuda() for t in inputs(8, 129, 158)]
     print(f"[case] split forced n=8 forward op={op} metric={metric} batch=129", flush=True)
     clf_env.setenv("CLF_PRODUCT_PATH", "split")

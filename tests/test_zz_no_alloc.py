@@ -49,13 +49,16 @@ def run_both(lib, op, side, metric, batch, seed):
 CASES = [
     ("geom", 0, (1,) * 8),                    # matrix-representation layer path (C3's)
     ("geom", 1, (1, -1) * 4),                 # same path, weight on the left
-    ("wedge", 0, (1,) * 7 + (-1,)),           # MFMA GEMM path, n = 8
-    ("lc", 1, (1,) * 6 + (-1, 0)),            # GEMM path with a null generator
-    ("geom", 0, (1,) * 9 + (0,)),             # GEMM path at n = 10: split count capped by the array
+    ("wedge", 0, (1,) * 7 + (-1,)),           # per-row kernels, n = 8
+    ("lc", 1, (1,) * 6 + (-1, 0)),            # per-row kernels with a null generator
+    ("geom", 0, (1,) * 9 + (0,)),             # per-row kernels at n = 10: the largest chunk of weight gradients
+    ("lc", 0, (1, -1) * 4),                   # MFMA GEMM path (low generators of both squares), n = 8
+    ("inner", 1, (0,) + (1,) * 6),            # GEMM path with a null low generator
+    ("inner", 0, (1, -1) * 5),                # GEMM path at n = 10: split count capped by the array
 ]
 
 
-@pytest.mark.parametrize("op,side,metric", CASES, ids=[f"{c[0]}-s{c[1]}-n{len(c[2])}" for c in CASES])
+@pytest.mark.parametrize("op,side,metric", CASES, ids=[f"{c[0]}-s{c[1]}-n{len(c[2])}-{i}" for i, c in enumerate(CASES)])
 def test_noalloc_matches_workspace_entry_point(op, side, metric):
     lib = _lib.load()
     n = len(metric)
