@@ -26,9 +26,11 @@
 //
 // Bound: 3 and 5 KB a row over HBM, 1024 / 2048 matrix-core cycles and about 500 /
 // 960 vector instructions per four rows (the scale test is 100 / 160 of them).
-// Measured (us, forward + backward, 50001 N(0, 1) rows): Cl(7,1) 31 + 59 (27 + 53
-// without the test; the per-term kernels 91 + 170), Cl(7,0,1) 30 + 55 (28 + 49;
-// 78 + 150); rows that all go by their terms 150 + 240 and 118 + 205.
+// Measured (us, forward + backward, 50001 N(0, 1) rows): Cl(7,1) 30 + 57 (28 + 52
+// without the test; the per-term kernels 91 + 170), Cl(7,0,1) 31 + 53 (28 + 48;
+// 78 + 150); rows that all go by their terms 146 + 232 and 119 + 190. The backward
+// keeps each gradient's relayout and rows over its second operand's slot, four
+// workgroups on a CU (with a slot of their own, three: 60 and 57).
 #include <mutex>
 
 #include "geom_terms.h"
@@ -233,13 +235,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     const float* __restrict__ A, long long lda, const float* __restrict__ B, long long ldb,
     const float* __restrict__ GC, long long ldg, float* __restrict__ GA, float* __restrict__ GB, long long batch,
     TwistTable T) {
-    __shared__ float lds[4][2 * 4 * 256 + kRelayoutFloats];  // gc | b, then a | relayout and rows of each gradient
+    // gc | b, over it the relayout and the rows of ga, then a and the same of gb
+    __shared__ float lds[4][4 * 256 + kRelayoutFloats];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const unsigned x = lane & 15u;
     const int rb = lane >> 4;
     float* s0 = &lds[wave][0];
     float* s1 = s0 + 4 * 256;
-    float* sr = s1 + 4 * 256;
     const unsigned oddx = (rb & 1) ? T.rep.odd_xor : 0u, oddc = T.rep.odd_xor >> 2;
     const float rho = (T.d && (x & 8u)) ? -1.f : 1.f, sigma = (T.d && !(x & 8u)) ? -1.f : 1.f;
     unsigned ent[16];
@@ -258,31 +260,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void t
     if (WA && bad_a != 15u) {
         const Parts g = twist_convert<0>(s0 + rb * 256, ent);
         const Parts b = twist_convert<0>(s1 + rb * 256, ent);
+        wave_lds_sync();
         const floatx16 acc = twist_products(g, b, 1.f, T.lambda, 1.f, 1.f, sigma);
-        relayout_store(sr, acc, lane);
+        relayout_store(s1, acc, lane);
         wave_lds_sync();
         float w[16];
-        relayout_load(sr, rb, x, w);
+        relayout_load(s1, rb, x, w);
         wave_lds_sync();
-        twist_unconvert(w, rho, sr + rb * 256, ent);
+        twist_unconvert(w, rho, s1 + rb * 256, ent);
+        wave_lds_sync();
+        twist_store<NT>(GA, s1, row0, batch, lane, oddc, bad_a);
     }
-    wave_lds_sync();
     const unsigned bad_b = WB ? bad_g | twist_uneven(pa, T, lane) : 0u;
-    if (WB) stage16(s1, pa, lane, oddc);
-    if (WA) twist_store<NT>(GA, sr, row0, batch, lane, oddc, bad_a);
-    wave_lds_sync();
     if (WB && bad_b != 15u) {
+        wave_lds_sync();
+        stage16(s1, pa, lane, oddc);
+        wave_lds_sync();
         const Parts a = twist_convert<1>(s1 + rb * 256, ent);
         const Parts g = twist_convert<1>(s0 + rb * 256, ent);
+        wave_lds_sync();
         const floatx16 acc = twist_products(a, g, 1.f, 1.f, T.lambda, 1.f, sigma);
-        relayout_store(sr, acc, lane);
+        relayout_store(s1, acc, lane);
         wave_lds_sync();
         float w[16];
-        relayout_load(sr, rb, x, w);
+        relayout_load(s1, rb, x, w);
         wave_lds_sync();
-        twist_unconvert(w, rho, sr + rb * 256, ent);
+        twist_unconvert(w, rho, s1 + rb * 256, ent);
         wave_lds_sync();
-        twist_store<NT>(GB, sr, row0, batch, lane, oddc, bad_b);
+        twist_store<NT>(GB, s1, row0, batch, lane, oddc, bad_b);
     }
     if (WA && bad_a) twist_terms<TERM_GA>(B, ldb, GC, ldg, GA, row0, batch, lane, bad_a, T.terms);
     if (WB && bad_b) twist_terms<TERM_GB>(A, lda, GC, ldg, GB, row0, batch, lane, bad_b, T.terms);
