@@ -2,11 +2,12 @@
 (1, 2^n) shared by the batch: the computation of the product layers
 (reference ``src/cliffordcuda/layers.py:30-50``).
 
-For n in [7, 10] this runs as fp32 MFMA GEMMs against the signed 2^n x 2^n
-matrix of w (``clf_product_bcast_fwd`` / ``_bwd``): the weight is never
-expanded to (batch, 2^n) and its gradient is reduced on the device. Smaller
-algebras use the per-row product kernels on the expanded weight, as the
-reference does.
+For n in [7, 10] one library call (``clf_product_bcast_fwd`` / ``_bwd``) runs
+the per-row product kernels with the weight as a one-row operand or, where no
+form fits the signature (mixed or null low metrics), fp32 MFMA GEMMs against the
+signed 2^n x 2^n matrix of w: the weight is never expanded to (batch, 2^n) and
+its gradient is reduced on the device. Smaller algebras use the per-row product
+kernels on the expanded weight, as the reference does.
 """
 from __future__ import annotations
 

@@ -3749,8 +3749,8 @@ __global__ __launch_bounds__(256) void prod_bwd_tiled(const float* __restrict__ 
 }
 
 // ---- generic path: one thread per output coefficient, closed-form signs ----
-// Used for n < 4 and for metrics whose low four generators are not all +1 or
-// all -1 (or contain a null generator).
+// Used for n < 4 and, where the low four generators have different squares or
+// null ones, for rows beyond the blocked kernels' LDS (n >= 13).
 __global__ __launch_bounds__(256) void prod_fwd_generic(int op, int n, unsigned neg, unsigned nul,
                                                          const float* __restrict__ A, const float* __restrict__ B,
                                                          float* __restrict__ C, long long batch) {
@@ -3842,8 +3842,6 @@ static void block_sign_params(int n, uint32_t neg, uint32_t nul, BlkParams& P) {
 
 constexpr size_t kBlockedLdsMax = 48 * 1024;
 
-// Launch shape for the whole-row blocked kernels. Returns false if the rows do
-// not fit the LDS budget (tiled path) or the metric needs the generic path.
 // Row skews of the blocked kernels' slots (bslot), 2 bits per staged row r at
 // bits 2 (r & 15): the rows that share a lane set of a ds_read_b128 (4 at n = 7,
 // 2 at n = 8, 4 of the 8 at n <= 6) get distinct skews, chosen on the CPU so
@@ -3856,6 +3854,8 @@ static unsigned blocked_row_skew(int n) {
     return 0u;
 }
 
+// Launch shape for the whole-row blocked kernels; false if the rows do not fit
+// the LDS budget (n >= 13).
 static bool blocked_launch(int n, uint32_t neg, uint32_t nul, int nops, BlkParams& P, dim3& grid, dim3& block,
                            size_t& lds_bytes) {
     const int nh = n - 4;

@@ -289,8 +289,11 @@ int clf_inverse_versor(int n, const float* x, const float* xr, float* y, int* fl
  * y = op(x, w) (side 0, x on the left, as the reference layers compute it,
  * src/cliffordcuda/layers.py:43-47) or y = op(w, x) (side 1), with one weight
  * multivector w (2^n floats) shared by all `batch` rows of x. Replaces the
- * layer path expand -> per-row kernel -> autograd batch sum. Implemented as
- * fp32 MFMA GEMMs against the signed 2^n x 2^n matrix of w. Supported n: 7..10.
+ * layer path expand -> per-row kernel -> autograd batch sum. Runs the per-row
+ * product kernels with w as a one-row operand (the weight gradient as their
+ * rows' column sums) or, where no form fits the signature (mixed or null low
+ * metrics) or w lies in the output's memory, fp32 MFMA GEMMs against the signed
+ * 2^n x 2^n matrix of w. Supported n: 7..10.
  * ws: device workspace of clf_product_bcast_ws_bytes(n, batch) bytes, 16-byte
  * aligned, owned by the caller; calls that share a workspace must not overlap. */
 size_t clf_product_bcast_ws_bytes(int n, int64_t batch);
