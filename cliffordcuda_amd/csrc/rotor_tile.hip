@@ -21,11 +21,14 @@
 // bits, chunk bit i = the i-th lane bit of both layouts. A lane bit that
 // changes from x to y puts y on chunk bits i and its own high bit, so the low
 // chunk bits are the lane number on both sides: free of bank conflicts for
-// ds_write_b128 (8 lanes) and ds_read_b128 (its 16-lane sets) alike.
+// ds_write_b128 (8 lanes) and ds_read_b128 (its 16-lane sets) alike (counted:
+// none forward, 0.04 to 0.36 cycles an LDS instruction in the composite backward).
 //
-// Bound: at batches that fill the card the rows over HBM (8, with gradient 12
-// bytes a coefficient), with the planes' arithmetic and the exchanges' LDS
-// traffic close behind; for a few rows the serial chain of one wave. Five
+// Bound: at batches that fill the card the planes' arithmetic (vector issue 55 to
+// 77 % of the time forward, 41 to 54 % backward) and the rows over HBM (8, with
+// gradient 12 bytes a coefficient); the n = 12 backward also the spills of 106
+// registers (139 MiB written for 64 MiB of rows); for a few rows the serial chain
+// of one wave. Five
 // register bits at n <= 11 keep that chain short (32 floats a lane) at two to
 // three more exchanges than six bits would take. Measured, forward (before: one
 // wave per row with lane shuffles, or rows in LDS with a barrier per plane), us:
